@@ -4,8 +4,9 @@
 //   M2L       : gather-GEMM on MFMA (16x16x4 f32 or f64): 32 target cells of
 //               one octant x 64 operator rows per workgroup, the 189 transfer
 //               vectors of that octant reduced in registers
-//   P2P       : one workgroup per target leaf, the 27 neighbour leaves staged
-//               through LDS, targets x source-splits mapped onto 256 lanes
+//   P2P       : the 27 neighbour leaves of a target leaf staged through LDS;
+//               mixed form: squared distances on FP16 MFMA of exact splits,
+//               roots and sums in FP32; FP64 form: targets x source-splits on 256 lanes
 #include <array>
 #include <cmath>
 #include <algorithm>
@@ -101,12 +102,11 @@ struct BoxArgs {
   double cell;   // leaf cell width
 };
 
-template <class T>
 __global__ void prepare_points_kernel(const double* __restrict__ pts, const double* __restrict__ w,
                                       const int32_t* __restrict__ perm,
                                       const int32_t* __restrict__ point_leaf,
                                       const uint64_t* __restrict__ leaf_codes, int64_t n, BoxArgs b,
-                                      V4<T>* __restrict__ out) {
+                                      V4<double>* __restrict__ out) {
   int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= n) return;
   int32_t j = perm[i];
@@ -119,20 +119,14 @@ __global__ void prepare_points_kernel(const double* __restrict__ pts, const doub
     double center = b.lo[k] + (c[k] + 0.5) * b.cell;
     xi[k] = (pts[3 * j + k] - center) * inv_h;
   }
-  V4<T> v;
-  v.x = static_cast<T>(xi[0]);
-  v.y = static_cast<T>(xi[1]);
-  v.z = static_cast<T>(xi[2]);
-  v.w = w ? static_cast<T>(w[j]) : T(0);
-  out[i] = v;
+  out[i] = {xi[0], xi[1], xi[2], w ? w[j] : 0.0};
 }
 
-template <class T>
 __global__ void set_weights_kernel(const double* __restrict__ w, const int32_t* __restrict__ perm,
-                                   int64_t n, V4<T>* __restrict__ pts) {
+                                   int64_t n, V4<double>* __restrict__ pts) {
   int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  pts[i].w = static_cast<T>(w[perm[i]]);
+  pts[i].w = w[perm[i]];
 }
 
 constexpr int kP2mChunk = 64;
@@ -394,16 +388,15 @@ __device__ __forceinline__ int p2p_shape(int nt, int* tp_out) {
   return best_r;
 }
 
-// kComp: compensated (Kahan) sums per target and FP64 sums over the source
-// splits, for weights that cancel strongly (kriging).
-// The passes of one target leaf with R targets per thread and tp target
-// slots (tp x nsplit threads; the sources staged through sp in chunks).
-template <class T, int KIND, bool kComp, int R>
+// The passes of one target leaf of the FP64 near field with R targets per
+// thread and tp target slots (tp x nsplit threads; the sources staged through
+// sp in chunks).
+template <int KIND, int R>
 __device__ __forceinline__ void p2p_passes(int nt, int ts, int tp, int total, int nnb, const int* nb_start,
-                                           const int* nb_src, const T (*nb_off)[3], V4<T>* sp, int cap,
-                                           T (*red)[kThreads], const V4<T>* __restrict__ tpts,
-                                           const V4<T>* __restrict__ spts, const double* __restrict__ y_far,
-                                           const int32_t* __restrict__ tperm, T pa, T pb,
+                                           const int* nb_src, const double (*nb_off)[3], V4<double>* sp, int cap,
+                                           double (*red)[kThreads], const V4<double>* __restrict__ tpts,
+                                           const V4<double>* __restrict__ spts, const double* __restrict__ y_far,
+                                           const int32_t* __restrict__ tperm, double pa, double pb,
                                            double* __restrict__ out) {
   // Every thread carries R targets (ti + r tp), so each source read from LDS
   // serves R pairs; tp target slots x nsplit source splits fill the 256 lanes.
@@ -411,14 +404,13 @@ __device__ __forceinline__ void p2p_passes(int nt, int ts, int tp, int total, in
   const int ti = threadIdx.x & (tp - 1);
   const int si = threadIdx.x / tp;
   for (int c0 = 0; c0 < nt; c0 += R * tp) {
-    V4<T> tq[R];
-    T acc[R], cmp[R];
+    V4<double> tq[R];
+    double acc[R];
 #pragma unroll
     for (int r = 0; r < R; r++) {
       const int i = c0 + r * tp + ti;
-      tq[r] = i < nt ? tpts[ts + i] : V4<T>{T(0), T(0), T(0), T(0)};
-      acc[r] = T(0);
-      cmp[r] = T(0);
+      tq[r] = i < nt ? tpts[ts + i] : V4<double>{0.0, 0.0, 0.0, 0.0};
+      acc[r] = 0.0;
     }
     for (int cb = 0; cb < total; cb += cap) {
       const int cnt = min(cap, total - cb);
@@ -427,7 +419,7 @@ __device__ __forceinline__ void p2p_passes(int nt, int ts, int tp, int total, in
         int g = cb + e;
         int k = 0;
         while (k + 1 < nnb && nb_start[k + 1] <= g) k++;
-        V4<T> q = spts[nb_src[k] + (g - nb_start[k])];
+        V4<double> q = spts[nb_src[k] + (g - nb_start[k])];
         q.x += nb_off[k][0];
         q.y += nb_off[k][1];
         q.z += nb_off[k][2];
@@ -439,22 +431,15 @@ __device__ __forceinline__ void p2p_passes(int nt, int ts, int tp, int total, in
       // offset, the shape function and one FMA. Four sources per trip keep
       // their LDS reads ahead of the arithmetic; the sum order over sources
       // is the plain sequential one.
-      const T seed = phi_seed<T, KIND>(pb);
-      auto pair = [&](const V4<T>& q, int r) {
-        T dx = tq[r].x - q.x, dy = tq[r].y - q.y, dz = tq[r].z - q.z;
-        T r2 = fma(dz, dz, fma(dy, dy, fma(dx, dx, seed)));
-        if constexpr (kComp) {
-          const T y = q.w * phi_shape<T, KIND>(r2, pb) - cmp[r];
-          const T t = acc[r] + y;
-          cmp[r] = (t - acc[r]) - y;
-          acc[r] = t;
-        } else {
-          acc[r] = fma(q.w, phi_shape<T, KIND>(r2, pb), acc[r]);
-        }
+      const double seed = phi_seed<double, KIND>(pb);
+      auto pair = [&](const V4<double>& q, int r) {
+        const double dx = tq[r].x - q.x, dy = tq[r].y - q.y, dz = tq[r].z - q.z;
+        const double r2 = fma(dz, dz, fma(dy, dy, fma(dx, dx, seed)));
+        acc[r] = fma(q.w, phi_shape<double, KIND>(r2, pb), acc[r]);
       };
       int j = si;
       for (; j + 3 * nsplit < cnt; j += 4 * nsplit) {
-        const V4<T> q0 = sp[j], q1 = sp[j + nsplit], q2 = sp[j + 2 * nsplit], q3 = sp[j + 3 * nsplit];
+        const V4<double> q0 = sp[j], q1 = sp[j + nsplit], q2 = sp[j + 2 * nsplit], q3 = sp[j + 3 * nsplit];
 #pragma unroll
         for (int r = 0; r < R; r++) {
           pair(q0, r);
@@ -464,47 +449,48 @@ __device__ __forceinline__ void p2p_passes(int nt, int ts, int tp, int total, in
         }
       }
       for (; j < cnt; j += nsplit) {
-        const V4<T> q = sp[j];
+        const V4<double> q = sp[j];
 #pragma unroll
         for (int r = 0; r < R; r++) pair(q, r);
       }
     }
     __syncthreads();  // red overlays the staged sources
 #pragma unroll
-    for (int r = 0; r < R; r++) red[r][threadIdx.x] = kComp ? acc[r] - cmp[r] : acc[r];
+    for (int r = 0; r < R; r++) red[r][threadIdx.x] = acc[r];
     __syncthreads();
     if (si == 0) {
 #pragma unroll
       for (int r = 0; r < R; r++) {
         const int i = c0 + r * tp + ti;
         if (i >= nt) continue;
-        using S = std::conditional_t<kComp, double, T>;
-        S sum = S(0);
-        for (int k = 0; k < nsplit; k++) sum += static_cast<S>(red[r][ti + k * tp]);
+        double sum = 0.0;
+        for (int k = 0; k < nsplit; k++) sum += red[r][ti + k * tp];
         const int gi = ts + i;
         double far = y_far ? y_far[gi] : 0.0;
-        out[tperm[gi]] = far + static_cast<double>(sum);
+        out[tperm[gi]] = far + sum;
       }
     }
     __syncthreads();
   }
 }
 
-// One target leaf of one evaluation's near field.
-template <class T, int KIND, bool kComp>
+// One target leaf of one evaluation's FP64 near field.
+template <int KIND>
 __device__ __forceinline__ void p2p_leaf(int leaf, const int32_t* __restrict__ tls, const int32_t* __restrict__ sls,
-                                         const int32_t* __restrict__ p2p, const V4<T>* __restrict__ tpts,
-                                         const V4<T>* __restrict__ spts, const double* __restrict__ y_far,
-                                         const int32_t* __restrict__ tperm, T pa, T pb, double* __restrict__ out) {
-  constexpr int CAP = 32768 / static_cast<int>(sizeof(V4<T>));
-  __shared__ V4<T> sp[CAP];
+                                         const int32_t* __restrict__ p2p, const V4<double>* __restrict__ tpts,
+                                         const V4<double>* __restrict__ spts, const double* __restrict__ y_far,
+                                         const int32_t* __restrict__ tperm, double pa, double pb,
+                                         double* __restrict__ out) {
+  constexpr int CAP = 32768 / static_cast<int>(sizeof(V4<double>));
+  __shared__ V4<double> sp[CAP];
   __shared__ int nb_start[28];
   __shared__ int nb_src[27];
-  __shared__ T nb_off[27][3];
+  __shared__ double nb_off[27][3];
   __shared__ int nb_count;
   // The split partials of a pass, over the staged sources (read after them).
-  static_assert(kP2PMaxR * kThreads * sizeof(T) <= sizeof(V4<T>) * CAP, "partials exceed the staging buffer");
-  T (*red)[kThreads] = reinterpret_cast<T (*)[kThreads]>(sp);
+  static_assert(kP2PMaxR * kThreads * sizeof(double) <= sizeof(V4<double>) * CAP,
+                "partials exceed the staging buffer");
+  double (*red)[kThreads] = reinterpret_cast<double (*)[kThreads]>(sp);
   const int ts = tls[leaf], te = tls[leaf + 1];
   const int nt = te - ts;
   if (threadIdx.x == 0) {
@@ -515,9 +501,9 @@ __device__ __forceinline__ void p2p_leaf(int leaf, const int32_t* __restrict__ t
       int a = sls[sl], b = sls[sl + 1];
       nb_src[k] = a;
       nb_start[k] = total;
-      nb_off[k][0] = T(2 * (s / 9 - 1));
-      nb_off[k][1] = T(2 * ((s / 3) % 3 - 1));
-      nb_off[k][2] = T(2 * (s % 3 - 1));
+      nb_off[k][0] = 2 * (s / 9 - 1);
+      nb_off[k][1] = 2 * ((s / 3) % 3 - 1);
+      nb_off[k][2] = 2 * (s % 3 - 1);
       total += b - a;
       k++;
     }
@@ -529,9 +515,9 @@ __device__ __forceinline__ void p2p_leaf(int leaf, const int32_t* __restrict__ t
   const int total = nb_start[nnb];
   int tp = kThreads;
   const int r = p2p_shape(nt, &tp);
-#define PAM_P2P_PASSES(RR)                                                                                     \
-  p2p_passes<T, KIND, kComp, RR>(nt, ts, tp, total, nnb, nb_start, nb_src, nb_off, sp, CAP, red, tpts, spts, \
-                                 y_far, tperm, pa, pb, out)
+#define PAM_P2P_PASSES(RR)                                                                                    \
+  p2p_passes<KIND, RR>(nt, ts, tp, total, nnb, nb_start, nb_src, nb_off, sp, CAP, red, tpts, spts, y_far, tperm, \
+                       pa, pb, out)
   switch (r) {
     case 4: PAM_P2P_PASSES(4); break;
     case 5: PAM_P2P_PASSES(5); break;
@@ -543,18 +529,344 @@ __device__ __forceinline__ void p2p_leaf(int leaf, const int32_t* __restrict__ t
 }
 
 // The near fields of up to kMaxFmmJobs evaluations (same precision, kernel
-// kind and summation form) in one launch: workgroup g takes target leaf
-// g - first_leaf of the last job whose first_leaf <= g. A single evaluation
-// is the one-job case of the same kernel, so its result does not depend on
-// what shares the launch.
-template <class T, int KIND, bool kComp>
-__global__ void __launch_bounds__(kThreads) p2p_jobs_kernel(P2PJobs<T> jobs) {
-  const int g = blockIdx.x;
+// kind and summation form) in one launch: a workgroup belongs to the last job
+// whose first_block <= its index. A single evaluation is the one-job case of
+// the same kernel, so its result does not depend on what shares the launch.
+template <class T>
+__device__ __forceinline__ const P2PJob<T>& p2p_job_of(const P2PJobs<T>& jobs, int g) {
   int k = 0;
-  while (k + 1 < jobs.n && jobs.j[k + 1].first_leaf <= g) k++;
-  const P2PJob<T>& j = jobs.j[k];
-  p2p_leaf<T, KIND, kComp>(g - j.first_leaf, j.tls, j.sls, j.p2p, j.tpts, j.spts, j.y_far, j.tperm, j.pa, j.pb,
-                           j.out);
+  while (k + 1 < jobs.n && jobs.j[k + 1].first_block <= g) k++;
+  return jobs.j[k];
+}
+
+template <int KIND>
+__global__ void __launch_bounds__(kThreads) p2p_jobs_kernel(P2PJobs<double> jobs) {
+  const int g = blockIdx.x;
+  const P2PJob<double>& j = p2p_job_of(jobs, g);
+  p2p_leaf<KIND>(g - j.first_block, j.tls, j.sls, j.p2p, j.tpts, j.spts, j.y_far, j.tperm, j.pa, j.pb, j.out);
+}
+
+// ---- near field of the mixed form: squared distances on the FP16 matrix unit ----
+//
+// Per pair the VALU needs 36 cycles per 64 pairs for three differences, three
+// FMAs, the hardware square root (8) and the weighted FMA; FP32 and FP64
+// matrix instructions take as long on the same lanes (measured: no overlap
+// with VALU work). The FP16 matrix unit is separate, so |s|^2 - 2 s.t + |t|^2
+// is formed there, from coordinates split so that the cancellation is exact:
+// in units of 2^-9 of the leaf half width, s = S + s1 + s2 with S an integer
+// (|S| <= 1536), s1 a multiple of 2^-11 (|s1| <= 1/2) and s2 the rest in FP16
+// (|s2| <= 2^-12, stored times 2^12). Three v_mfma_f32_16x16x16_f16 give, for
+// 16 sources and 16 targets, each starting from the sum so far,
+//   |S - T|^2                          integers below 2^24: exact;
+//   2 (S - T).(s1 - t1)                multiples of 2^-11 below 2^13: exact
+//                                      beside a small |S - T|^2, else one rounding;
+//   |s1 - t1|^2 + 2 (S - T).(s2 - t2)  one rounding; terms below 2^2.
+// What only the source (target) decides is summed beforehand and enters as
+// one or two FP16 pieces against constants. The neglected 2 (s1 - t1).(s2 -
+// t2) is below 2^-9 units (2^-27 of the half width squared) and zero for
+// coincident points. So r^2 keeps FP32 relative accuracy down to distances
+// where FP32 coordinates end. The VALU is left with root and FMA (12 cycles
+// per 64 pairs; the three matrix instructions show with 7 more).
+// Near field of 1M x 1M uniform points at order 8 (5.9e9 pairs, MI355X, alone):
+// 1.65 ms on the VALU, 1.62 ms with FP64 matrix distances, 0.99 ms this way;
+// 300k surface points (symmetric, uneven leaves): 1.68 to 0.65 ms, of which
+// about half is the finer split of the leaves. Four or six tiles per wave
+// instead of five: 1.09 and 1.00 ms. Two workgroups per leaf at 4,096 leaves:
+// 1.05 ms; at 512 leaves eight per leaf fill the chip.
+constexpr int kMfSrc = kThreads;  // sources staged per chunk: one per thread
+constexpr int kMfMaxTiles = 5;  // 16-target tiles per wave and pass
+constexpr double kMfUnit = 0x1p-9;
+// Workgroups wanted in a launch of one evaluation: a leaf's tiles are shared
+// out to several workgroups when there are fewer leaves.
+constexpr int kMfBlocks = 4096, kMfMaxParts = 8;
+
+using h16x4 = _Float16 __attribute__((ext_vector_type(4)));
+using f32x4v = float __attribute__((ext_vector_type(4)));
+
+// A leaf-local coordinate split as above; the FP64 rest of the integer part
+// is below 1/2, so FP32 holds it to 2^-26 units.
+struct MfCoord {
+  float i, f1, f2;  // integer part, multiple of 2^-11, 2^12 x the rest (FP16 values)
+};
+__device__ __forceinline__ MfCoord mf_split(double x) {
+  const double u = x * (1.0 / kMfUnit);
+  const double r = rint(u);
+  const float rho = static_cast<float>(u - r);
+  const float f1 = rintf(rho * 2048.0f) * 0x1p-11f;
+  return {static_cast<float>(r), f1, static_cast<float>(static_cast<_Float16>((rho - f1) * 4096.0f))};
+}
+// The parts that only one point decides: |P|^2 = 4096 a + b, 2 P.p1 = c1 + c2,
+// |p1|^2 + 2 P.p2 = d1 + 2^-10 d2, all FP16 values.
+struct MfSelf {
+  float a, b, c1, c2, d1, d2;
+};
+__device__ __forceinline__ float mf_half(float v) { return static_cast<float>(static_cast<_Float16>(v)); }
+__device__ __forceinline__ MfSelf mf_self(const MfCoord& x, const MfCoord& y, const MfCoord& z) {
+  const float n = fmaf(z.i, z.i, fmaf(y.i, y.i, x.i * x.i));
+  MfSelf s;
+  s.a = rintf(n * 0x1p-12f);
+  s.b = fmaf(s.a, -4096.0f, n);
+  const float c = 2.0f * fmaf(z.i, z.f1, fmaf(y.i, y.f1, x.i * x.f1));
+  s.c1 = mf_half(c);
+  s.c2 = c - s.c1;
+  const float d = fmaf(z.f1, z.f1, fmaf(y.f1, y.f1, x.f1 * x.f1)) +
+                  0x1p-11f * fmaf(z.i, z.f2, fmaf(y.i, y.f2, x.i * x.f2));
+  s.d1 = mf_half(d);
+  s.d2 = (d - s.d1) * 1024.0f;
+  return s;
+}
+__device__ __forceinline__ h16x4 mf_pack(float a, float b, float c, float d) {
+  return h16x4{static_cast<_Float16>(a), static_cast<_Float16>(b), static_cast<_Float16>(c),
+               static_cast<_Float16>(d)};
+}
+
+// Running sums of a lane's rows of one target tile: two FP32 chains, or, for
+// weights that cancel strongly (kComp), FP64 sums of the chunks' compensated
+// (Kahan) FP32 sums.
+template <bool kComp>
+struct MfSum {
+  float even = 0.0f, odd = 0.0f;
+  __device__ double value() const { return static_cast<double>(even) + static_cast<double>(odd); }
+};
+template <>
+struct MfSum<true> {
+  double sum = 0.0;
+  __device__ double value() const { return sum; }
+};
+
+// A target as a matrix column of the three products: reduction indices 4 grp
+// .. 4 grp + 3 (the sources' rows are written in p2p_mf_jobs_kernel).
+struct MfColumn {
+  h16x4 b[3];
+};
+__device__ __forceinline__ MfColumn mf_column(const V4<double>& p, int grp) {
+  const MfCoord x = mf_split(p.x), y = mf_split(p.y), z = mf_split(p.z);
+  const MfSelf q = mf_self(x, y, z);
+  const float k = 0x1p-12f;
+  const h16x4 zero = mf_pack(0.0f, 0.0f, 0.0f, 0.0f);
+  if (grp == 0)
+    return {{mf_pack(x.i, y.i, z.i, 4096.0f), mf_pack(-2.0f * x.i, -2.0f * y.i, -2.0f * z.i, -2.0f * x.f1),
+             mf_pack(-2.0f * x.f1, -2.0f * y.f1, -2.0f * z.f1, -2.0f * k * x.i)}};
+  if (grp == 1)
+    return {{mf_pack(1.0f, q.a, q.b, 0.0f), mf_pack(-2.0f * y.f1, -2.0f * z.f1, 1.0f, 1.0f),
+             mf_pack(-2.0f * k * y.i, -2.0f * k * z.i, -2.0f * x.f2, -2.0f * y.f2)}};
+  if (grp == 2)
+    return {{zero, mf_pack(q.c1, q.c2, 0.0f, 0.0f), mf_pack(-2.0f * z.f2, 1.0f, 0x1p-10f, q.d1)}};
+  return {{zero, zero, mf_pack(q.d2, 0.0f, 0.0f, 0.0f)}};
+}
+
+// Adds to tot[0..M) the sums of M target tiles (their columns t) over the
+// staged source blocks s0, s0 + ds, ...: MFMA row = source, column = target; a
+// lane holds rows 4 (lane / 16) + i of column lane % 16.
+template <int KIND, bool kComp, int M>
+__device__ __forceinline__ void mf_tiles(const h16x4* sa, const f32x4v* sw, int nblk, int s0, int ds,
+                                         const MfColumn* t, float pb, float seed, MfSum<kComp>* tot) {
+  const int lane = threadIdx.x & 63, grp = lane >> 4;
+  const f32x4v init{seed, seed, seed, seed};
+  float acc[M], cmp[M];  // kComp: sum and compensation; else the even and odd chains
+#pragma unroll
+  for (int m = 0; m < M; m++) {
+    if constexpr (kComp) {
+      acc[m] = cmp[m] = 0.0f;
+    } else {
+      acc[m] = tot[m].even;
+      cmp[m] = tot[m].odd;
+    }
+  }
+  for (int blk = s0; blk < nblk; blk += ds) {
+    const h16x4 a0 = sa[blk * 192 + lane], a1 = sa[blk * 192 + 64 + lane], a2 = sa[blk * 192 + 128 + lane];
+    const f32x4v w = sw[blk * 4 + grp];
+    f32x4v d[M];
+#pragma unroll
+    for (int m = 0; m < M; m++) d[m] = __builtin_amdgcn_mfma_f32_16x16x16f16(a0, t[m].b[0], init, 0, 0, 0);
+#pragma unroll
+    for (int m = 0; m < M; m++) d[m] = __builtin_amdgcn_mfma_f32_16x16x16f16(a1, t[m].b[1], d[m], 0, 0, 0);
+#pragma unroll
+    for (int m = 0; m < M; m++) d[m] = __builtin_amdgcn_mfma_f32_16x16x16f16(a2, t[m].b[2], d[m], 0, 0, 0);
+#pragma unroll
+    for (int m = 0; m < M; m++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const float phi = phi_shape<float, KIND>(fabsf(d[m][i]), pb);
+        if constexpr (kComp) {
+          const float y = w[i] * phi - cmp[m];
+          const float s = acc[m] + y;
+          cmp[m] = (s - acc[m]) - y;
+          acc[m] = s;
+        } else if (i % 2 == 0) {
+          acc[m] = fmaf(w[i], phi, acc[m]);
+        } else {
+          cmp[m] = fmaf(w[i], phi, cmp[m]);
+        }
+      }
+  }
+#pragma unroll
+  for (int m = 0; m < M; m++) {
+    if constexpr (kComp) {
+      tot[m].sum += static_cast<double>(acc[m]) - static_cast<double>(cmp[m]);
+    } else {
+      tot[m].even = acc[m];
+      tot[m].odd = cmp[m];
+    }
+  }
+}
+
+template <int KIND, bool kComp>
+__global__ void __launch_bounds__(kThreads, 4) p2p_mf_jobs_kernel(P2PJobs<float> jobs) {
+  __shared__ h16x4 sa[kMfSrc / 16 * 192];  // [16-source block][product][reduction index / 4][row]
+  __shared__ f32x4v sw[kMfSrc / 4];        // [block][row]: weights
+  __shared__ int nb_start[28];
+  __shared__ int nb_src[27];
+  __shared__ float nb_off[27][3];  // in units
+  __shared__ int nb_count;
+  __shared__ double red[4][kMfMaxTiles * 16];
+  const P2PJob<float>& j = p2p_job_of(jobs, static_cast<int>(blockIdx.x));
+  // Groups of 64 leaves: the workgroups of eight consecutive (sibling) leaves
+  // on one XCD (workgroup i runs on XCD i % 8), whose L2 then holds their
+  // shared neighbours.
+  int leaf, part;
+  {
+    const int lb = static_cast<int>(blockIdx.x) - j.first_block;
+    const int per = 64 * j.parts, grp = lb / per;
+    if ((grp + 1) * 64 <= j.n_leaves) {
+      const int r = lb - grp * per, q = r / 8;
+      leaf = grp * 64 + (r & 7) * 8 + q / j.parts;
+      part = q % j.parts;
+    } else {
+      leaf = lb / j.parts;
+      part = lb % j.parts;
+    }
+  }
+  const int ts = j.tls[leaf], te = j.tls[leaf + 1];
+  const int tiles = (te - ts + 15) / 16;
+  const int tile0 = tiles * part / j.parts, tile1 = tiles * (part + 1) / j.parts;
+  if (tile0 == tile1) return;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  if (wave == 0) {
+    // The neighbour leaves that exist, in slot order, with their offsets and
+    // the prefix sums of their point counts.
+    int a = 0, cnt = 0;
+    const int sl = lane < 27 ? j.p2p[static_cast<int64_t>(leaf) * 27 + lane] : -1;
+    if (sl >= 0) {
+      a = j.sls[sl];
+      cnt = j.sls[sl + 1] - a;
+    }
+    int incl = cnt;
+#pragma unroll
+    for (int d = 1; d < 32; d <<= 1) {
+      const int u = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += u;
+    }
+    const uint64_t have = __ballot(sl >= 0);
+    if (sl >= 0) {
+      const int k = __popcll(have & ((uint64_t{1} << lane) - 1));
+      nb_src[k] = a;
+      nb_start[k] = incl - cnt;
+      constexpr int kLeaf = static_cast<int>(2.0 / kMfUnit);
+      nb_off[k][0] = static_cast<float>(kLeaf * (lane / 9 - 1));
+      nb_off[k][1] = static_cast<float>(kLeaf * ((lane / 3) % 3 - 1));
+      nb_off[k][2] = static_cast<float>(kLeaf * (lane % 3 - 1));
+    }
+    if (lane == 26) {
+      nb_count = __popcll(have);
+      nb_start[__popcll(have)] = incl;
+    }
+  }
+  __syncthreads();
+  const int nnb = nb_count, total = nb_start[nnb];
+  const float pa = j.pa, pb = j.pb;
+  const float seed = phi_seed<float, KIND>(pb);
+  // Entries that no source changes: the constants against the targets' own
+  // parts, and the unused reduction indices.
+  {
+    h16x4* a = sa + (tid >> 4) * 192 + (tid & 15);
+    a[32] = a[48] = a[64 + 48] = mf_pack(0.0f, 0.0f, 0.0f, 0.0f);
+    a[64 + 32] = mf_pack(1.0f, 1.0f, 0.0f, 0.0f);
+    a[128 + 48] = mf_pack(0x1p-10f, 0.0f, 0.0f, 0.0f);
+  }
+  const int npass = (tile1 - tile0 + 4 * kMfMaxTiles - 1) / (4 * kMfMaxTiles);
+  for (int ps = 0; ps < npass; ps++) {
+    const int p0 = tile0 + (tile1 - tile0) * ps / npass, p1 = tile0 + (tile1 - tile0) * (ps + 1) / npass;
+    const int n = p1 - p0;
+    // The pass's tiles over G groups of waves, the sources over 4 / G splits:
+    // as few groups as kMfMaxTiles tiles per wave allow.
+    const int G = n <= kMfMaxTiles ? 1 : (n <= 2 * kMfMaxTiles ? 2 : 4), S = 4 / G;
+    // The groups move over the waves with the workgroup's index, so that the
+    // ones with a tile more do not all sit on the same SIMD.
+    const int rot = (wave + static_cast<int>(blockIdx.x)) & 3;
+    const int grp = rot & (G - 1), split = rot / G;
+    const int mine = n / G + (grp < n % G ? 1 : 0);
+    const int tgt = ts + 16 * (p0 + grp * (n / G) + min(grp, n % G));
+    MfSum<kComp> tot[kMfMaxTiles];
+    MfColumn cols[kMfMaxTiles];
+#pragma unroll
+    for (int m = 0; m < kMfMaxTiles; m++) {
+      const int i = tgt + 16 * m + (lane & 15);
+      cols[m] = mf_column(m < mine && i < te ? j.tpts[i] : V4<double>{0.0, 0.0, 0.0, 0.0}, lane >> 4);
+    }
+    // One source per thread and chunk; the next chunk's is in flight while
+    // this one is multiplied.
+    int k = 0;  // this thread's neighbour; its sources only move forward
+    V4<double> q{0.0, 0.0, 0.0, 0.0};  // filled up with sources of no weight
+    auto fetch = [&](int g) {
+      q = {0.0, 0.0, 0.0, 0.0};
+      if (g >= total) return;
+      while (k + 1 < nnb && nb_start[k + 1] <= g) k++;
+      q = j.spts[nb_src[k] + (g - nb_start[k])];
+    };
+    fetch(tid);
+    for (int cb = 0; cb < total; cb += kMfSrc) {
+      const int nblk = (min(kMfSrc, total - cb) + 15) / 16;
+      MfCoord x = mf_split(q.x), y = mf_split(q.y), z = mf_split(q.z);
+      x.i += nb_off[k][0];  // exact: an integer number of units
+      y.i += nb_off[k][1];
+      z.i += nb_off[k][2];
+      const MfSelf s = mf_self(x, y, z);
+      const float c = 0x1p-12f;
+      __syncthreads();
+      h16x4* a = sa + (tid >> 4) * 192 + (tid & 15);
+      a[0] = mf_pack(-2.0f * x.i, -2.0f * y.i, -2.0f * z.i, s.a);
+      a[16] = mf_pack(s.b, 4096.0f, 1.0f, 0.0f);
+      a[64] = mf_pack(x.f1, y.f1, z.f1, x.i);
+      a[64 + 16] = mf_pack(y.i, z.i, s.c1, s.c2);
+      a[128] = mf_pack(x.f1, y.f1, z.f1, x.f2);
+      a[128 + 16] = mf_pack(y.f2, z.f2, c * x.i, c * y.i);
+      a[128 + 32] = mf_pack(c * z.i, s.d1, s.d2, 1.0f);
+      reinterpret_cast<float*>(sw)[tid] = static_cast<float>(q.w) * pa;  // the kernel's factor a folded in
+      fetch(cb + kMfSrc + tid);
+      __syncthreads();
+      switch (mine) {
+        case 1: mf_tiles<KIND, kComp, 1>(sa, sw, nblk, split, S, cols, pb, seed, tot); break;
+        case 2: mf_tiles<KIND, kComp, 2>(sa, sw, nblk, split, S, cols, pb, seed, tot); break;
+        case 3: mf_tiles<KIND, kComp, 3>(sa, sw, nblk, split, S, cols, pb, seed, tot); break;
+        case 4: mf_tiles<KIND, kComp, 4>(sa, sw, nblk, split, S, cols, pb, seed, tot); break;
+        case 5: mf_tiles<KIND, kComp, 5>(sa, sw, nblk, split, S, cols, pb, seed, tot); break;
+        default: break;
+      }
+    }
+    // Rows of the four lane groups, then the splits in order.
+    double sums[kMfMaxTiles];
+#pragma unroll
+    for (int m = 0; m < kMfMaxTiles; m++) {
+      sums[m] = tot[m].value();
+      sums[m] += __shfl_xor(sums[m], 16, 64);
+      sums[m] += __shfl_xor(sums[m], 32, 64);
+      if (split > 0 && lane < 16) red[rot][m * 16 + lane] = sums[m];
+    }
+    __syncthreads();
+    if (split == 0 && lane < 16) {
+#pragma unroll
+      for (int m = 0; m < kMfMaxTiles; m++) {
+        const int i = tgt + 16 * m + lane;
+        if (m >= mine || i >= te) continue;
+        double sum = sums[m];
+        for (int s = 1; s < S; s++) sum += red[s * G + grp][m * 16 + lane];
+        const double far = j.y_far ? j.y_far[i] : 0.0;
+        j.out[j.tperm[i]] = far + sum;
+      }
+    }
+    __syncthreads();  // red is written again in the next pass
+  }
 }
 
 // ---- gradients at the targets (gradient-transpose kernel,
@@ -598,6 +910,11 @@ __device__ __forceinline__ void lagrange_d_lds(T xi, const T* __restrict__ tk, T
 struct Aniso3 {
   double a[9];  // row-major A
 };
+
+template <class T>
+__device__ __forceinline__ V4<T> point_as(const V4<double>& q) {
+  return {static_cast<T>(q.x), static_cast<T>(q.y), static_cast<T>(q.z), static_cast<T>(q.w)};
+}
 
 constexpr int kL2PGThreads = 128;
 
@@ -666,8 +983,8 @@ l2p_grad_kernel(const int32_t* __restrict__ leaf_start, const V4<double>* __rest
 template <class T, int KIND>
 __global__ void __launch_bounds__(kThreads)
 p2p_grad_kernel(const int32_t* __restrict__ tls, const int32_t* __restrict__ sls,
-                const int32_t* __restrict__ p2p, const V4<T>* __restrict__ tpts,
-                const V4<T>* __restrict__ spts, const int32_t* __restrict__ tperm, T ag, T pb, Aniso3 A,
+                const int32_t* __restrict__ p2p, const V4<double>* __restrict__ tpts,
+                const V4<double>* __restrict__ spts, const int32_t* __restrict__ tperm, T ag, T pb, Aniso3 A,
                 double* __restrict__ out) {
   constexpr int CAP = 32768 / static_cast<int>(sizeof(V4<T>));
   constexpr int R = 2;
@@ -713,7 +1030,7 @@ p2p_grad_kernel(const int32_t* __restrict__ tls, const int32_t* __restrict__ sls
 #pragma unroll
     for (int r = 0; r < R; r++) {
       const int i = c0 + r * tp + ti;
-      tq[r] = i < nt ? tpts[ts + i] : V4<T>{T(0), T(0), T(0), T(0)};
+      tq[r] = i < nt ? point_as<T>(tpts[ts + i]) : V4<T>{T(0), T(0), T(0), T(0)};
       ax[r] = ay[r] = az[r] = T(0);
     }
     for (int cb = 0; cb < total; cb += CAP) {
@@ -723,7 +1040,7 @@ p2p_grad_kernel(const int32_t* __restrict__ tls, const int32_t* __restrict__ sls
         int g = cb + e;
         int k = 0;
         while (k + 1 < nnb && nb_start[k + 1] <= g) k++;
-        V4<T> q = spts[nb_src[k] + (g - nb_start[k])];
+        V4<T> q = point_as<T>(spts[nb_src[k] + (g - nb_start[k])]);
         q.x += nb_off[k][0];
         q.y += nb_off[k][1];
         q.z += nb_off[k][2];
@@ -879,8 +1196,8 @@ l2p_hess_col_kernel(const int32_t* __restrict__ leaf_start, const V4<double>* __
 template <class T, int KIND>
 __global__ void __launch_bounds__(kThreads)
 p2p_hess_col_kernel(const int32_t* __restrict__ tls, const int32_t* __restrict__ sls,
-                    const int32_t* __restrict__ p2p, const V4<T>* __restrict__ tpts,
-                    const V4<T>* __restrict__ spts, const int32_t* __restrict__ tperm, T hc, T pb, Aniso3 A,
+                    const int32_t* __restrict__ p2p, const V4<double>* __restrict__ tpts,
+                    const V4<double>* __restrict__ spts, const int32_t* __restrict__ tperm, T hc, T pb, Aniso3 A,
                     int kcol, double* __restrict__ out) {
   constexpr int CAP = 32768 / static_cast<int>(sizeof(V4<T>));
   constexpr int R = 2;
@@ -927,7 +1244,7 @@ p2p_hess_col_kernel(const int32_t* __restrict__ tls, const int32_t* __restrict__
 #pragma unroll
     for (int r = 0; r < R; r++) {
       const int i = c0 + r * tp + ti;
-      tq[r] = i < nt ? tpts[ts + i] : V4<T>{T(0), T(0), T(0), T(0)};
+      tq[r] = i < nt ? point_as<T>(tpts[ts + i]) : V4<T>{T(0), T(0), T(0), T(0)};
       ax[r] = ay[r] = az[r] = T(0);
     }
     for (int cb = 0; cb < total; cb += CAP) {
@@ -937,7 +1254,7 @@ p2p_hess_col_kernel(const int32_t* __restrict__ tls, const int32_t* __restrict__
         int g = cb + e;
         int k = 0;
         while (k + 1 < nnb && nb_start[k + 1] <= g) k++;
-        V4<T> q = spts[nb_src[k] + (g - nb_start[k])];
+        V4<T> q = point_as<T>(spts[nb_src[k] + (g - nb_start[k])]);
         q.x += nb_off[k][0];
         q.y += nb_off[k][1];
         q.z += nb_off[k][2];
@@ -1909,22 +2226,20 @@ void dispatch_order(int p, F&& f) {
 
 }  // namespace
 
-template <class T>
-void launch_prepare_points(const Tree& t, const double* d_pts, const double* d_w, V4<T>* out,
+void launch_prepare_points(const Tree& t, const double* d_pts, const double* d_w, V4<double>* out,
                            hipStream_t s) {
   int64_t n = t.n_points;
   if (n == 0) return;
   BoxArgs b{{t.box.lo[0], t.box.lo[1], t.box.lo[2]}, t.box.width / std::ldexp(1.0, t.level)};
-  prepare_points_kernel<T><<<ceil_div(n, 256), 256, 0, s>>>(d_pts, d_w, t.perm.get(), t.point_leaf.get(),
+  prepare_points_kernel<<<ceil_div(n, 256), 256, 0, s>>>(d_pts, d_w, t.perm.get(), t.point_leaf.get(),
                                                             t.levels[t.level].codes.get(), n, b, out);
   PAM_LAUNCH_CHECK();
 }
 
-template <class T>
-void launch_set_point_weights(const Tree& t, const double* d_w, V4<T>* pts, hipStream_t s) {
+void launch_set_point_weights(const Tree& t, const double* d_w, V4<double>* pts, hipStream_t s) {
   int64_t n = t.n_points;
   if (n == 0) return;
-  set_weights_kernel<T><<<ceil_div(n, 256), 256, 0, s>>>(d_w, t.perm.get(), n, pts);
+  set_weights_kernel<<<ceil_div(n, 256), 256, 0, s>>>(d_w, t.perm.get(), n, pts);
   PAM_LAUNCH_CHECK();
 }
 
@@ -1975,11 +2290,12 @@ L2PJob<T> make_l2p_job(const Tree& t, const T* l_leaf, const V4<T>* pts, T* y_fa
 }
 
 template <class T>
-P2PJob<T> make_p2p_job(const RbfDesc& rbf, const Tree& trg, const Tree& src, const Lists& lists, const V4<T>* tpts,
-                       const V4<T>* spts, const double* y_far, double* out) {
+P2PJob<T> make_p2p_job(const RbfDesc& rbf, const Tree& trg, const Tree& src, const Lists& lists,
+                       const V4<double>* tpts, const V4<double>* spts, const double* y_far, double* out) {
   P2PJob<T> j{};
   const double h = trg.box.width / std::ldexp(1.0, trg.level) / 2.0;
-  const PhiConsts pc = phi_consts(rbf, h);
+  // The mixed form's kernel works in units of kMfUnit of the leaf half width.
+  const PhiConsts pc = phi_consts(rbf, sizeof(T) == 4 ? h * kMfUnit : h);
   j.tls = trg.leaf_start.get();
   j.sls = src.leaf_start.get();
   j.p2p = lists.p2p.get();
@@ -1988,9 +2304,10 @@ P2PJob<T> make_p2p_job(const RbfDesc& rbf, const Tree& trg, const Tree& src, con
   j.y_far = y_far;
   j.tperm = trg.perm.get();
   j.pa = static_cast<T>(pc.a);
-  j.pb = static_cast<T>(pc.b);
+  j.pb = static_cast<T>(phi_shape_const<T>(rbf.kind, pc.b));
   j.out = out;
   j.n_leaves = static_cast<int>(trg.n_leaves());
+  j.parts = sizeof(T) == 4 && j.n_leaves > 0 ? std::clamp((kMfBlocks + j.n_leaves - 1) / j.n_leaves, 1, kMfMaxParts) : 1;
   return j;
 }
 
@@ -2020,20 +2337,17 @@ void launch_p2p_jobs(int kind, bool compensated, const P2PJob<T>* jobs, int n, h
   int64_t total = 0;
   for (int k = 0; k < n; k++) {
     t.j[t.n] = jobs[k];
-    t.j[t.n].first_leaf = static_cast<int>(total);
-    total += jobs[k].n_leaves;
+    t.j[t.n].first_block = static_cast<int>(total);
+    total += static_cast<int64_t>(jobs[k].n_leaves) * jobs[k].parts;
     if (jobs[k].n_leaves > 0) t.n++;
   }
   if (total == 0) return;
   if (total > INT32_MAX) throw_runtime("too many leaves in one launch");
+  const unsigned grid = static_cast<unsigned>(total);
   dispatch_kind(kind, [&](auto K) {
-    if constexpr (sizeof(T) == 4) {
-      if (compensated) {
-        p2p_jobs_kernel<T, decltype(K)::value, true><<<static_cast<unsigned>(total), kThreads, 0, s>>>(t);
-        return;
-      }
-    }
-    p2p_jobs_kernel<T, decltype(K)::value, false><<<static_cast<unsigned>(total), kThreads, 0, s>>>(t);
+    if constexpr (sizeof(T) == 8) p2p_jobs_kernel<decltype(K)::value><<<grid, kThreads, 0, s>>>(t);
+    else if (compensated) p2p_mf_jobs_kernel<decltype(K)::value, true><<<grid, kThreads, 0, s>>>(t);
+    else p2p_mf_jobs_kernel<decltype(K)::value, false><<<grid, kThreads, 0, s>>>(t);
   });
   PAM_LAUNCH_CHECK();
 }
@@ -2048,7 +2362,7 @@ void launch_l2p(int p, const Tree& t, const T* l_leaf, const V4<T>* pts, T* y_fa
 
 template <class T>
 void launch_p2p(const RbfDesc& rbf, const Tree& trg, const Tree& src, const Lists& lists,
-                const V4<T>* tpts, const V4<T>* spts, const double* y_far, double* out, hipStream_t s,
+                const V4<double>* tpts, const V4<double>* spts, const double* y_far, double* out, hipStream_t s,
                 bool compensated) {
   if (trg.n_leaves() == 0) return;
   const P2PJob<T> j = make_p2p_job<T>(rbf, trg, src, lists, tpts, spts, y_far, out);
@@ -2123,7 +2437,7 @@ void launch_l2p_hess_col(int p, const Tree& t, const double* l_leaf, const V4<do
 
 template <class T>
 void launch_p2p_hess_col(const RbfDesc& rbf, const Tree& trg, const Tree& src, const Lists& lists,
-                         const V4<T>* tpts, const V4<T>* spts, int kcol, double* out3, hipStream_t s) {
+                         const V4<double>* tpts, const V4<double>* spts, int kcol, double* out3, hipStream_t s) {
   int64_t nl = trg.n_leaves();
   if (nl == 0) return;
   if (kcol < 0 || kcol > 2) throw_invalid("Hessian column out of range");
@@ -2141,7 +2455,7 @@ void launch_p2p_hess_col(const RbfDesc& rbf, const Tree& trg, const Tree& src, c
 
 template <class T>
 void launch_p2p_grad(const RbfDesc& rbf, const Tree& trg, const Tree& src, const Lists& lists,
-                     const V4<T>* tpts, const V4<T>* spts, double* out3, hipStream_t s) {
+                     const V4<double>* tpts, const V4<double>* spts, double* out3, hipStream_t s) {
   int64_t nl = trg.n_leaves();
   if (nl == 0) return;
   const double h = trg.box.width / std::ldexp(1.0, trg.level) / 2.0;
@@ -2207,22 +2521,19 @@ void launch_m2l_batch(const M2LOperator& op, const std::vector<M2LLevelSpec<TM, 
 }
 
 #define PAM_INSTANTIATE(T)                                                                          \
-  template void launch_prepare_points<T>(const Tree&, const double*, const double*, V4<T>*,        \
-                                         hipStream_t);                                               \
-  template void launch_set_point_weights<T>(const Tree&, const double*, V4<T>*, hipStream_t);       \
   template void launch_p2m<T>(int, const Tree&, const V4<T>*, T*, hipStream_t);                     \
   template void launch_m2m<T>(int, const Tree&, int, const T*, T*, hipStream_t);                    \
   template void launch_l2l<T>(int, const Tree&, int, const T*, T*, hipStream_t);                    \
   template void launch_l2p<T>(int, const Tree&, const T*, const V4<T>*, T*, hipStream_t, bool);           \
   template L2PJob<T> make_l2p_job<T>(const Tree&, const T*, const V4<T>*, T*, bool, int);                   \
-  template P2PJob<T> make_p2p_job<T>(const RbfDesc&, const Tree&, const Tree&, const Lists&, const V4<T>*,  \
-                                     const V4<T>*, const double*, double*);                                 \
-  template void launch_p2p<T>(const RbfDesc&, const Tree&, const Tree&, const Lists&, const V4<T>*, \
-                              const V4<T>*, const double*, double*, hipStream_t, bool);                 \
-  template void launch_p2p_grad<T>(const RbfDesc&, const Tree&, const Tree&, const Lists&, const V4<T>*, \
-                                   const V4<T>*, double*, hipStream_t);                                  \
-  template void launch_p2p_hess_col<T>(const RbfDesc&, const Tree&, const Tree&, const Lists&, const V4<T>*, \
-                                       const V4<T>*, int, double*, hipStream_t);                           \
+  template P2PJob<T> make_p2p_job<T>(const RbfDesc&, const Tree&, const Tree&, const Lists&, const V4<double>*, \
+                                     const V4<double>*, const double*, double*);                                 \
+  template void launch_p2p<T>(const RbfDesc&, const Tree&, const Tree&, const Lists&, const V4<double>*, \
+                              const V4<double>*, const double*, double*, hipStream_t, bool);                 \
+  template void launch_p2p_grad<T>(const RbfDesc&, const Tree&, const Tree&, const Lists&, const V4<double>*, \
+                                   const V4<double>*, double*, hipStream_t);                                  \
+  template void launch_p2p_hess_col<T>(const RbfDesc&, const Tree&, const Tree&, const Lists&, const V4<double>*, \
+                                       const V4<double>*, int, double*, hipStream_t);                           \
   template void build_m2l_dense<T>(int, const RbfDesc&, double, M2LOperator&, DevBuf<T>&,          \
                                    hipStream_t);                                                    \
   template void launch_m2l_batch<T, double>(const M2LOperator&,                                        \

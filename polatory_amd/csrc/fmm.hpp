@@ -2,8 +2,8 @@
 // order P per axis, P^3 nodes per cell). T = float (mixed form) or double.
 //
 // Storage:
-//   points in tree order as V4<T> = (xi, eta, zeta, w): coordinates local to the
-//   point's leaf, scaled so the leaf is [-1,1]^3;
+//   points in tree order as V4<double> = (xi, eta, zeta, w): coordinates local
+//   to the point's leaf, scaled so the leaf is [-1,1]^3;
 //   expansions [n_cells][kpad(P)] (zero padded), node index (a*P + b)*P + c,
 //   a along x; nodes x_a = cos((2a+1) pi / (2P)).
 #pragma once
@@ -39,11 +39,9 @@ struct M2LOperator {
   size_t per_v = 0;  // elements per transfer vector
 };
 
-template <class T>
-void launch_prepare_points(const Tree& t, const double* d_pts, const double* d_w, V4<T>* out,
+void launch_prepare_points(const Tree& t, const double* d_pts, const double* d_w, V4<double>* out,
                            hipStream_t s);
-template <class T>
-void launch_set_point_weights(const Tree& t, const double* d_w, V4<T>* pts, hipStream_t s);
+void launch_set_point_weights(const Tree& t, const double* d_w, V4<double>* pts, hipStream_t s);
 
 template <class T>
 void launch_p2m(int p, const Tree& t, const V4<T>* pts, T* m_leaf, hipStream_t s);
@@ -56,19 +54,20 @@ void launch_l2l(int p, const Tree& t, int l, const T* l_parent, T* l_child, hipS
 // Near-field (P2P) and far-field (L2P) work of one evaluation as kernel
 // arguments, so that several evaluations, of any model, can share one launch
 // of each (serving). A lone evaluation runs the same kernels with one job.
+// T: arithmetic of the kernel values and sums; the points are FP64 either way.
 constexpr int kMaxFmmJobs = 8;
 template <class T>
 struct P2PJob {
   const int32_t* tls;    // target leaf starts
   const int32_t* sls;    // source leaf starts
   const int32_t* p2p;    // [target leaves][27] source leaves
-  const V4<T>* tpts;     // targets in tree order, leaf-local
-  const V4<T>* spts;     // sources in tree order, leaf-local, with weights
+  const V4<double>* tpts;  // targets in tree order, leaf-local
+  const V4<double>* spts;  // sources in tree order, leaf-local, with weights
   const double* y_far;   // far field in tree order, or null
   const int32_t* tperm;  // tree order -> input order of the targets
   double* out;           // output, input order
-  T pa, pb;              // kernel constants in the leaf unit
-  int n_leaves, first_leaf;
+  T pa, pb;              // kernel constants in the leaf unit (phi_shape_const)
+  int n_leaves, parts, first_block;  // parts: workgroups per leaf
 };
 template <class T>
 struct P2PJobs {
@@ -90,8 +89,8 @@ struct L2PJobs {
   L2PJob<T> j[kMaxFmmJobs];
 };
 template <class T>
-P2PJob<T> make_p2p_job(const RbfDesc& rbf, const Tree& trg, const Tree& src, const Lists& lists, const V4<T>* tpts,
-                       const V4<T>* spts, const double* y_far, double* out);
+P2PJob<T> make_p2p_job(const RbfDesc& rbf, const Tree& trg, const Tree& src, const Lists& lists,
+                       const V4<double>* tpts, const V4<double>* spts, const double* y_far, double* out);
 template <class T>
 L2PJob<T> make_l2p_job(const Tree& t, const T* l_leaf, const V4<T>* pts, T* y_far, bool add_to_output, int kpad);
 // The near field and far field of one evaluation, recorded instead of
@@ -118,14 +117,14 @@ void launch_l2p(int p, const Tree& t, const T* l_leaf, const V4<T>* pts, T* y_fa
 // out[perm[i]] = y_far[i] + near field, FP64 output in input order.
 template <class T>
 void launch_p2p(const RbfDesc& rbf, const Tree& trg, const Tree& src, const Lists& lists,
-                const V4<T>* tpts, const V4<T>* spts, const double* y_far, double* out, hipStream_t s,
+                const V4<double>* tpts, const V4<double>* spts, const double* y_far, double* out, hipStream_t s,
                 bool compensated = false);  // compensated: Kahan sums (FP32 only)
 // Gradients at the targets (fmm/gradient_transpose_kernel.hpp:47-62): the
 // near field writes A^T sum_j w_j grad phi into out3 (n x 3, input order);
 // the far field then adds A^T grad of the leaf local expansions.
 template <class T>
 void launch_p2p_grad(const RbfDesc& rbf, const Tree& trg, const Tree& src, const Lists& lists,
-                     const V4<T>* tpts, const V4<T>* spts, double* out3, hipStream_t s);
+                     const V4<double>* tpts, const V4<double>* spts, double* out3, hipStream_t s);
 void launch_l2p_grad(int p, const Tree& t, const double* l_leaf, const V4<double>* pts, const double* aniso,
                      double* out3, hipStream_t s);
 // Column kcol of the Hessian kernel at the targets (fmm/hessian_kernel.hpp:46-64
@@ -133,7 +132,7 @@ void launch_l2p_grad(int p, const Tree& t, const double* l_leaf, const V4<double
 // near field writes, the far field adds.
 template <class T>
 void launch_p2p_hess_col(const RbfDesc& rbf, const Tree& trg, const Tree& src, const Lists& lists,
-                         const V4<T>* tpts, const V4<T>* spts, int kcol, double* out3, hipStream_t s);
+                         const V4<double>* tpts, const V4<double>* spts, int kcol, double* out3, hipStream_t s);
 void launch_l2p_hess_col(int p, const Tree& t, const double* l_leaf, const V4<double>* pts, const double* aniso,
                          int kcol, double* out3, hipStream_t s);
 

@@ -231,8 +231,8 @@ void FmmEvaluator::set_config(const FmmConfig& c) {
 
 void FmmEvaluator::invalidate_expansions() {
   st_.multipoles_valid = false;
-  st_.s64_valid = st_.s32_valid = false;
-  st_.t64_valid = st_.t32_valid = false;
+  st_.s64_valid = false;
+  st_.t64_valid = false;
 }
 
 void FmmEvaluator::set_source_points(const double* xyz, int64_t n, bool on_device) {
@@ -271,7 +271,7 @@ void FmmEvaluator::set_target_points(const double* xyz, int64_t n, bool on_devic
   if (n > 0) launch_bbox(trg_pts_.get(), n, bbox_out_.get() + 6, bbox_scratch_, stream_);
   trg_tree_dirty_ = true;
   box_valid_ = false;
-  st_.t64_valid = st_.t32_valid = false;
+  st_.t64_valid = false;
   if (!on_device) PAM_HIP(hipStreamSynchronize(stream_));
 }
 
@@ -285,8 +285,7 @@ void FmmEvaluator::set_weights(const double* w, int64_t n, bool on_device) {
   }
   have_weights_ = true;
   // Point coordinates stay; only the weights and the multipoles change.
-  if (st_.s32_valid) launch_set_point_weights<float>(src_tree_, w_.get(), st_.spts32.get(), stream_);
-  if (st_.s64_valid) launch_set_point_weights<double>(src_tree_, w_.get(), st_.spts64.get(), stream_);
+  if (st_.s64_valid) launch_set_point_weights(src_tree_, w_.get(), st_.spts64.get(), stream_);
   st_.multipoles_valid = false;
   if (!on_device) PAM_HIP(hipStreamSynchronize(stream_));
 }
@@ -338,7 +337,7 @@ void FmmEvaluator::ensure_box() {
     if (!same) {
       box_ = b;
       trg_tree_dirty_ = true;
-      st_.t32_valid = st_.t64_valid = false;
+      st_.t64_valid = false;
     }
     box_valid_ = true;
     return;
@@ -389,7 +388,7 @@ void FmmEvaluator::ensure_trees() {
       build_identity_cols(trg_tree_, trg_cols_, stream_);
       trg_tree_dirty_ = false;
       rebuilt = true;
-      st_.t32_valid = st_.t64_valid = false;
+      st_.t64_valid = false;
     }
     if (rebuilt || lists_.level != L) {
       build_lists(trg_tree_, stree, lists_, ws_, stream_, effective_svd_tol(cfg_, rbf_) > 0.0);
@@ -418,14 +417,14 @@ void FmmEvaluator::ensure_trees() {
     build_tree(src_tree_, src_pts_.get(), n_src_, box_, level, ws_, stream_);
     src_tree_dirty_ = false;
     rebuilt = true;
-    st_.s32_valid = st_.s64_valid = false;
+    st_.s64_valid = false;
     st_.multipoles_valid = false;
   };
   auto build_trg = [&](int level) {
     build_tree(trg_tree_, trg_pts_.get(), n_trg_, box_, level, tws, ts);
     trg_tree_dirty_ = false;
     rebuilt = true;
-    st_.t32_valid = st_.t64_valid = false;
+    st_.t64_valid = false;
   };
   int L;
   if (cfg_.leaf_level >= 0) {
@@ -461,13 +460,13 @@ void FmmEvaluator::ensure_trees() {
       if (do_src) {
         src_counts_ = level_counts(hs);
         src_tree_dirty_ = false;
-        st_.s32_valid = st_.s64_valid = false;
+        st_.s64_valid = false;
         st_.multipoles_valid = false;
       }
       if (do_trg) {
         trg_counts_ = level_counts(ht);
         trg_tree_dirty_ = false;
-        st_.t32_valid = st_.t64_valid = false;
+        st_.t64_valid = false;
       }
     };
     const bool sort_src = src_tree_dirty_ || static_cast<int>(src_counts_.size()) != Lmax + 1;
@@ -497,12 +496,12 @@ void FmmEvaluator::ensure_trees() {
     if (!symmetric_ && (sort_trg || resort_trg || trg_tree_.level != L)) {
       finish_tree(trg_tree_, L, trg_counts_, tws, ts);
       rebuilt = true;
-      st_.t32_valid = st_.t64_valid = false;
+      st_.t64_valid = false;
     }
     if (sort_src || resort_src || src_tree_.level != L) {
       finish_tree(src_tree_, L, src_counts_, ws_, stream_);
       rebuilt = true;
-      st_.s32_valid = st_.s64_valid = false;
+      st_.s64_valid = false;
       st_.multipoles_valid = false;
     }
     join();
@@ -564,7 +563,7 @@ void FmmEvaluator::attach_source(const FmmEvaluator* owner) {
   trg_tree_dirty_ = true;
   lists_.level = -1;  // rebuilt on the next evaluation (buffers kept)
   lists_gen_++;
-  st_.t32_valid = st_.t64_valid = false;
+  st_.t64_valid = false;
   // Targets are transformed with the rbf's anisotropy: they must be set again.
   n_trg_ = 0;
 }
@@ -583,15 +582,13 @@ void FmmEvaluator::record(int idx, hipStream_t s) {
 
 template <class TP>
 void FmmEvaluator::prepare_source_expansions() {
-  prepare_source_points<TP>();
+  prepare_source_points();
   prepare_source_multipoles<TP>();
 }
 
-template <class TP>
 void FmmEvaluator::prepare_source_points() {
   FmmState& st = st_;
   const int P = cfg_.order;
-  const int kp = kpad_of(P);
   const int L = src_tree_.level;
   if (st.m.size() < static_cast<size_t>(L) + 1) st.m.resize(L + 1);
   if (st.m_level != L || st.multipole_order != P) {
@@ -601,16 +598,9 @@ void FmmEvaluator::prepare_source_points() {
   }
   if (!st.s64_valid) {
     st.spts64.resize(n_src_);
-    launch_prepare_points<double>(src_tree_, src_pts_.get(), w_.get(), st.spts64.get(), stream_);
+    launch_prepare_points(src_tree_, src_pts_.get(), w_.get(), st.spts64.get(), stream_);
     st.s64_valid = true;
     st.multipoles_valid = false;
-  }
-  if constexpr (sizeof(TP) == 4) {
-    if (!st.s32_valid) {
-      st.spts32.resize(n_src_);
-      launch_prepare_points<float>(src_tree_, src_pts_.get(), w_.get(), st.spts32.get(), stream_);
-      st.s32_valid = true;
-    }
   }
 }
 
@@ -652,32 +642,19 @@ void FmmEvaluator::run_fmm(double* d_out) {
   const int L = stree.level;
   record(1);
   if (!so_) {
-    prepare_source_points<TP>();
+    prepare_source_points();
   } else if (!sst.multipoles_valid || sst.multipole_order != P || !sst.s64_valid ||
-             (sizeof(TP) == 4 && (!sst.s32_valid || !sst.m32_valid))) {
+             (sizeof(TP) == 4 && !sst.m32_valid)) {
     throw_runtime("the shared source side is not prepared (call prepare_source on the owner)");
   }
   if (st.l.size() < static_cast<size_t>(L) + 1) st.l.resize(L + 1);
   if (!symmetric_ && !st.t64_valid) {
     st.tpts64.resize(n_trg_);
-    launch_prepare_points<double>(trg_tree_, trg_pts_.get(), nullptr, st.tpts64.get(), stream_);
+    launch_prepare_points(trg_tree_, trg_pts_.get(), nullptr, st.tpts64.get(), stream_);
     st.t64_valid = true;
   }
-  const V4<double>* tpts64 = symmetric_ ? sst.spts64.get() : st.tpts64.get();
-  const V4<TP>* sp2p;
-  const V4<TP>* tp2p;
-  if constexpr (sizeof(TP) == 4) {
-    if (!symmetric_ && !st.t32_valid) {
-      st.tpts32.resize(n_trg_);
-      launch_prepare_points<float>(trg_tree_, trg_pts_.get(), nullptr, st.tpts32.get(), stream_);
-      st.t32_valid = true;
-    }
-    sp2p = sst.spts32.get();
-    tp2p = symmetric_ ? sst.spts32.get() : st.tpts32.get();
-  } else {
-    sp2p = sst.spts64.get();
-    tp2p = tpts64;
-  }
+  const V4<double>* tpts = symmetric_ ? sst.spts64.get() : st.tpts64.get();
+  const V4<double>* spts = sst.spts64.get();
   if (!so_) prepare_source_multipoles<TP>();
   record(2);
   // Fork: the near field (VALU work) writes the output on the second stream
@@ -690,16 +667,16 @@ void FmmEvaluator::run_fmm(double* d_out) {
       defer_->fp32 = sizeof(TP) == 4;
       defer_->compensated = cfg_.precision == kMixedComp;
       defer_->kind = rbf_.kind;
-      if constexpr (sizeof(TP) == 4) defer_->p2p32 = make_p2p_job<float>(rbf_, tt, stree, lists_, tp2p, sp2p, nullptr, d_out);
-      else defer_->p2p64 = make_p2p_job<double>(rbf_, tt, stree, lists_, tp2p, sp2p, nullptr, d_out);
+      if constexpr (sizeof(TP) == 4) defer_->p2p32 = make_p2p_job<float>(rbf_, tt, stree, lists_, tpts, spts, nullptr, d_out);
+      else defer_->p2p64 = make_p2p_job<double>(rbf_, tt, stree, lists_, tpts, spts, nullptr, d_out);
       return;
     }
     PAM_HIP(hipEventRecord(fork_ev_, stream_));
     PAM_HIP(hipStreamWaitEvent(ps, fork_ev_, 0));
     record(7, ps);
-    if (hess_col_ >= 0) launch_p2p_hess_col<TP>(rbf_, tt, stree, lists_, tp2p, sp2p, hess_col_, d_out, ps);
-    else if (grad_) launch_p2p_grad<TP>(rbf_, tt, stree, lists_, tp2p, sp2p, d_out, ps);
-    else launch_p2p<TP>(rbf_, tt, stree, lists_, tp2p, sp2p, nullptr, d_out, ps, cfg_.precision == kMixedComp);
+    if (hess_col_ >= 0) launch_p2p_hess_col<TP>(rbf_, tt, stree, lists_, tpts, spts, hess_col_, d_out, ps);
+    else if (grad_) launch_p2p_grad<TP>(rbf_, tt, stree, lists_, tpts, spts, d_out, ps);
+    else launch_p2p<TP>(rbf_, tt, stree, lists_, tpts, spts, nullptr, d_out, ps, cfg_.precision == kMixedComp);
     record(8, ps);
     PAM_HIP(hipEventRecord(join_ev_, ps));
   };
@@ -806,7 +783,7 @@ void FmmEvaluator::run_fmm(double* d_out) {
   record(4);
   if (!overlap) near_field(stream_);
   if (defer_) {
-    defer_->l2p = make_l2p_job<double>(tt, st.l[L].get(), tpts64, d_out, true, kp);
+    defer_->l2p = make_l2p_job<double>(tt, st.l[L].get(), tpts, d_out, true, kp);
     defer_->order = P;
     defer_->valid = true;
     for (int i = 5; i <= 8; i++) record(i);
@@ -815,9 +792,9 @@ void FmmEvaluator::run_fmm(double* d_out) {
   // Join the near field, then add the far field to it.
   PAM_HIP(hipStreamWaitEvent(stream_, join_ev_, 0));
   record(5);
-  if (hess_col_ >= 0) launch_l2p_hess_col(P, tt, st.l[L].get(), tpts64, rbf_.aniso, hess_col_, d_out, stream_);
-  else if (grad_) launch_l2p_grad(P, tt, st.l[L].get(), tpts64, rbf_.aniso, d_out, stream_);
-  else launch_l2p<double>(P, tt, st.l[L].get(), tpts64, d_out, stream_, true);
+  if (hess_col_ >= 0) launch_l2p_hess_col(P, tt, st.l[L].get(), tpts, rbf_.aniso, hess_col_, d_out, stream_);
+  else if (grad_) launch_l2p_grad(P, tt, st.l[L].get(), tpts, rbf_.aniso, d_out, stream_);
+  else launch_l2p<double>(P, tt, st.l[L].get(), tpts, d_out, stream_, true);
   record(6);
 }
 

@@ -46,11 +46,10 @@ struct FmmStats {
 };
 
 // Expansions and the light O(N P^3) stages (P2M, M2M, L2L, L2P) are FP64 in
-// both forms; the mixed form runs P2P on FP32 copies of the points and M2L on
-// FP32 MFMA (operands rounded to FP32, FP64 accumulation).
+// both forms; the mixed form evaluates the near field's kernel values and sums
+// in FP32 (from FP64 points) and M2L on FP32 MFMA (operands rounded to FP32, FP64 accumulation).
 struct FmmState {
   DevBuf<V4<double>> spts64, tpts64;
-  DevBuf<V4<float>> spts32, tpts32;
   std::vector<DevBuf<double>> m, l;    // per level, P^3 node values
   std::vector<DevBuf<float>> m32;      // per level, FP32 copy of m (mixed-form M2L operand)
   std::vector<DevBuf<double>> mt, lt;  // per level, compressed coefficients
@@ -63,7 +62,7 @@ struct FmmState {
   M2LPairSchedule m2l_psched;
   uint64_t m2l_sched_gen = 0;
   int m2l_sched_rpad = 0;
-  bool s64_valid = false, t64_valid = false, s32_valid = false, t32_valid = false;
+  bool s64_valid = false, t64_valid = false;
   bool multipoles_valid = false, m32_valid = false;
   int multipole_order = 0;
   int m_level = -1;  // leaf level the multipoles were computed for
@@ -154,7 +153,6 @@ class FmmEvaluator {
   const FmmEvaluator& S() const { return so_ ? *so_ : *this; }
   template <class TP>
   void prepare_source_expansions();
-  template <class TP>
   void prepare_source_points();
   template <class TP>
   void prepare_source_multipoles();

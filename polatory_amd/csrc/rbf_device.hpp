@@ -70,6 +70,13 @@ __device__ __forceinline__ double sqrt_nr(double x) {
   return x > 0.0 ? s : 0.0;
 }
 
+// The constant b that phi_shape<T> expects: the FP32 exponential is 2^(b r),
+// with log2 e folded in before the rounding to FP32.
+template <class T>
+inline double phi_shape_const(int kind, double b) {
+  return sizeof(T) == 4 && kind == kExp ? b * 1.4426950408889634074 : b;
+}
+
 // phi without its factor a, for loops that fold a into the weights:
 // r2c = r^2 + b for bh3 / th3 (the caller seeds its sum of squares with b),
 // r2c = r^2 for exp.
@@ -88,10 +95,9 @@ __device__ __forceinline__ T phi_shape(T r2c, T b) {
     if constexpr (KIND == kBh3) {
       return __builtin_amdgcn_sqrtf(r2c);
     } else if constexpr (KIND == kTh3) {
-      float rho = __builtin_amdgcn_sqrtf(r2c);
-      return rho * rho * rho;
+      return r2c * __builtin_amdgcn_sqrtf(r2c);
     } else {
-      return __expf(b * __builtin_amdgcn_sqrtf(r2c));
+      return __builtin_amdgcn_exp2f(b * __builtin_amdgcn_sqrtf(r2c));
     }
   }
 }

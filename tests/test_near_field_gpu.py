@@ -1,0 +1,74 @@
+"""The near field alone: points inside the eight central leaves of a level-2
+tree are all neighbours of each other, so no far field contributes. Sizes sit
+on the edges of the mixed kernel's tiles (16 targets, 5 tiles per wave, 256
+sources per chunk). Calls go through the C ABI."""
+import numpy as np
+import pytest
+
+import polatory_amd as pa
+
+pytestmark = pytest.mark.gpu
+
+KINDS = {"bh3": ("BH3", pa.Biharmonic3D, [1.5, 0.0]), "bh3c": ("BH3", pa.Biharmonic3D, [1.0, 0.03]),
+         "th3": ("TH3", pa.Triharmonic3D, [0.7, 0.0]), "exp": ("EXP", pa.CovExponential, [1.2, 0.4])}
+H = 1.01 / 4 / 2  # leaf half width
+
+
+@pytest.mark.parametrize("precision", ["mixed", "mixed_comp"])
+@pytest.mark.parametrize("kind", list(KINDS))
+@pytest.mark.parametrize("n_src,n_trg", [(1, 1), (15, 17), (257, 16), (2048, 640), (2049, 81 * 8), (700, 2600),
+                                         (5000, 3000)])
+def test_mixed_near_field_matches_direct_sum(orc, kind, precision, n_src, n_trg):
+    print("near field", kind, precision, n_src, n_trg, flush=True)
+    name, cls, params = KINDS[kind]
+    rng = np.random.default_rng(n_src + n_trg)
+    src = rng.uniform(0.25, 0.75, (n_src, 3))
+    trg = rng.uniform(0.25, 0.75, (n_trg, 3))
+    k = min(n_src, n_trg) // 2
+    trg[:k] = src[:k]  # coincident pairs
+    if n_trg > 1000:
+        trg[k:k + 100] = src[:1] + rng.uniform(-1e-5, 1e-5, (100, 3))  # nearly coincident ones
+    w = rng.normal(size=n_src)
+    ev = pa.make_fmm_evaluator(cls(params), ((0, 0, 0), (1, 1, 1)))
+    ev.set_config(pa.FmmConfig(precision, 4, 2, "fmm"))
+    ev.set_source_points(src)
+    ev.set_weights(w)
+    ev.set_target_points(trg)
+    y = ev.evaluate()
+    ref = orc.direct_rbf_sum(orc.make_rbf(getattr(orc, name), params), src, w, trg)
+    # Per pair: r^2 in FP32 from exact splits (three roundings of the matrix
+    # unit of up to 2^-21 together, observed 4.8e-7 of the largest term), root,
+    # product and sums 2^-24 each along chains of n / 8; the exponential turns
+    # a relative error of r into 3 r / range times as much. Absolute floor:
+    # r^2 is off by up to 2^-37 H^2 for coincident points, r by 2^-18 H.
+    d = np.linalg.norm(trg[:, None, :] - src[None, :, :], axis=2)
+    if kind in ("bh3", "bh3c"):
+        phi, slope, grow = params[0] * np.sqrt(d * d + params[1] ** 2), params[0], 1.0
+    elif kind == "th3":
+        phi, slope, grow = params[0] * d ** 3, 0.0, 3.0
+    else:
+        phi, slope, grow = params[0] * np.exp(-3 * d / params[1]), 3 * params[0] / params[1], 1.0 + 3 * d / params[1]
+    rel = 2.0 ** -21 * grow + 2.0 ** -24 * (2 + n_src / 8 ** 0.5 / 8)
+    bound = (np.abs(w) * (phi * rel + slope * H * 2.0 ** -18 * (d < 1e-3))).sum(axis=1) + 1e-12
+    worst = np.max(np.abs(y - ref) / bound)
+    print(f"  worst error / bound {worst:.3f}, rel {np.abs(y - ref).max() / np.abs(ref).max():.2e}", flush=True)
+    assert worst <= 1.0
+
+
+def test_mixed_near_field_does_not_depend_on_shared_launches():
+    """One leaf of many targets next to leaves of few: every pass and split of
+    the wave groups gives the bits of the same evaluation repeated."""
+    rng = np.random.default_rng(3)
+    src = rng.uniform(0.25, 0.75, (4000, 3))
+    trg = np.concatenate([rng.uniform(0.26, 0.49, (2000, 3)), rng.uniform(0.51, 0.75, (37, 3))])
+    w = rng.normal(size=4000)
+    outs = []
+    for overlap in (True, False):
+        ev = pa.make_fmm_evaluator(pa.Biharmonic3D(), ((0, 0, 0), (1, 1, 1)))
+        ev.set_config(pa.FmmConfig("mixed", 4, 2, "fmm"))
+        ev.set_overlap(overlap)
+        ev.set_source_points(src)
+        ev.set_weights(w)
+        ev.set_target_points(trg)
+        outs.append(ev.evaluate())
+    np.testing.assert_array_equal(outs[0], outs[1])
