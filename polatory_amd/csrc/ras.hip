@@ -15,6 +15,7 @@
 #include <numeric>
 #include <queue>
 
+#include "coarse_dense.hpp"
 #include "device_api.hpp"
 #include "rbf_device.hpp"
 
@@ -845,41 +846,6 @@ void launch_cholesky_batch(int nb, int n_dom, const int64_t* ptr, int l, const i
   PAM_LAUNCH_CHECK();
 }
 
-// A single large matrix, per panel step: the diagonal block by one
-// workgroup (its inverse written out), the rows below it by one thread per
-// row, the trailing tiles by one workgroup per tile.
-__global__ void __launch_bounds__(kT)
-cholesky_panel_kernel(double* __restrict__ a, int n, int k0, int32_t* __restrict__ flag, double* __restrict__ inv_out) {
-  __shared__ CholSmem<double, kNb> sm;
-  chol_diag(sm, a, n, k0, flag);
-  const double (*inv)[kNb + 1] = reinterpret_cast<const double (*)[kNb + 1]>(&sm.dt[0][0]);
-  for (int e = threadIdx.x; e < kNb * kNb; e += kT) inv_out[e] = inv[e / kNb][e % kNb];
-}
-
-// The rows below the panel's diagonal block, spread over workgroups.
-__global__ void __launch_bounds__(kT)
-cholesky_rows_kernel(double* __restrict__ a, int n, int k0, const double* __restrict__ inv_in) {
-  __shared__ double inv[kNb][kNb + 1];
-  for (int e = threadIdx.x; e < kNb * kNb; e += kT) inv[e / kNb][e % kNb] = inv_in[e];
-  __syncthreads();
-  const int kb = min(kNb, n - k0);
-  chol_rows<double, kNb>(a, n, k0, inv, k0 + kb + static_cast<int>(blockIdx.x * kT + threadIdx.x),
-                         static_cast<int>(gridDim.x * kT));
-}
-
-__global__ void __launch_bounds__(kT)
-cholesky_trailing_kernel(double* __restrict__ a, int n, int k0) {
-  __shared__ CholSmem<double, kNb> sm;
-  // blockIdx.x -> (I, J) with I >= J
-  const int t = blockIdx.x;
-  int I = static_cast<int>((sqrt(8.0 * t + 1.0) - 1.0) / 2.0);
-  while ((I + 1) * (I + 2) / 2 <= t) I++;
-  while (I * (I + 1) / 2 > t) I--;
-  const int J = t - I * (I + 1) / 2;
-  chol_tile(sm, a, n, k0, I, J, true);
-}
-
-
 // Sum of the partials of the first 64 threads, added in lane order by one
 // thread: the result does not depend on the workgroup size.
 __device__ __forceinline__ double lane_ordered_sum(double v, double* sh) {
@@ -1066,29 +1032,19 @@ ras_solve_kernel(RbfSet r, int l, const double* __restrict__ pts, const double* 
   });
 }
 
-// The coarse grid's solve as a dense operator: workgroup u0 solves for the
-// unit vector e_u0 and writes column u0 of op ((m + l) x m, row-major).
-__global__ void __launch_bounds__(kT)
-coarse_operator_kernel(RbfSet r, int l, const double* __restrict__ pts, const double* __restrict__ gpts, int64_t mu_v,
-                       const int32_t* __restrict__ idx, int m,
-                       const double* __restrict__ lag, const double* __restrict__ mat,
-                       const double* __restrict__ pinv, double* __restrict__ op) {
-  extern __shared__ double sm[];
-  __shared__ double sh[kT];
-  const int u0 = blockIdx.x;
-  double* vals = sm;
-  double* y = sm + m;
-  for (int u = threadIdx.x; u < m; u += kT) vals[u] = u == u0 ? 1.0 : 0.0;
-  __syncthreads();
-  solve_domain<kT>(r, l, pts, gpts, mu_v, idx, m, lag, mat, vals, y, sh, 1, pinv,
-               [&](int u, double v) { op[static_cast<int64_t>(u) * m + u0] = v; });
+// A_top of the coarse grid: the rows of its first l points against all of its
+// m rows (l x m).
+__global__ void coarse_atop_kernel(RbfSet r, int l, const double* __restrict__ pts, const double* __restrict__ gpts,
+                                   int64_t mu_v, const int32_t* __restrict__ idx, int m, double* __restrict__ atop) {
+  const int e = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
+  if (e < l * m) atop[e] = flat_entry(r, pts, gpts, mu_v, idx[e / m], idx[e % m]);
 }
 
 // Coarse solve by the dense operator: out[idx[u]] = (op d)[u] for u < m and
 // out[mu + a] = (op d)[m + a], d = res[idx[.]]. One wavefront per row, the
 // row's products summed in a fixed order.
 constexpr int kCoarseRowsPerBlock = kT / 64;
-constexpr int kCoarseOpMax = 8192;  // largest coarse grid given a dense operator (512 MiB)
+constexpr int kCoarseOpMax = 6144;  // largest coarse grid given a dense operator
 
 __global__ void __launch_bounds__(kT)
 coarse_apply_kernel(const int32_t* __restrict__ idx, int m, int l, const double* __restrict__ op,
@@ -2048,16 +2004,24 @@ RasPreconditioner::RasPreconditioner(const Model& model, const std::vector<doubl
     hipStream_t cs = fork_stream();
     setup_batch(coarse_, h_domains_[0], true, cs, false, flag_.get());
     // The coarse solve is one domain: solved by a single workgroup it would
-    // serialize on one CU, so it is turned into a dense operator once (one
-    // workgroup per unit vector) and applied as a matrix-vector product.
+    // serialize on one CU, so it is turned into a dense operator once and
+    // applied as a matrix-vector product.
     const int m = static_cast<int>(coarse_.h_ptr[1] - coarse_.h_ptr[0]);
-    const size_t shmem = sizeof(double) * 2 * static_cast<size_t>(m);
-    if (coarse_.n_dom == 1 && m > 0 && m <= kCoarseOpMax && shmem <= 96 * 1024) {
+    if (has_coarse_operator(coarse_)) {
+      SetupTmp& tmp = *setup_tmp_.back();
+      const int n = m - l_;
       coarse_.op.resize(static_cast<size_t>(m + l_) * m);
-      RbfSet rs = make_rbf_set(model_);
-      coarse_operator_kernel<<<m, kT, shmem, cs>>>(rs, l_, d_pts_.get(), d_gpts_.get(), mu_, coarse_.idx.get(), m,
-                                                   lag_.get(), coarse_.mat.get(), pinv_.get(), coarse_.op.get());
-      PAM_LAUNCH_CHECK();
+      tmp.t.resize(static_cast<size_t>(std::max(n, 1)) * std::max(n, 1));
+      tmp.atop.resize(static_cast<size_t>(std::max(l_ * m, 1)));
+      if (l_ > 0) {
+        RbfSet rs = make_rbf_set(model_);
+        coarse_atop_kernel<<<ceil_div(l_ * m, kT), kT, 0, cs>>>(rs, l_, d_pts_.get(), d_gpts_.get(), mu_,
+                                                                coarse_.idx.get(), m, tmp.atop.get());
+        PAM_LAUNCH_CHECK();
+      }
+      launch_coarse_inverse(coarse_.mat.get(), n, tmp.x.get(), tmp.t.get(), cs);
+      launch_coarse_operator(tmp.x.get(), m, l_, coarse_.idx.get(), lag_.get(), tmp.atop.get(), pinv_.get(),
+                             coarse_.op.get(), cs);
       coarse_.has_op = true;
     }
   }
@@ -2139,9 +2103,14 @@ void RasPreconditioner::join_streams() {
   }
 }
 
+// The coarse grid gets a dense operator up to 6,144 rows (302 MiB).
+bool RasPreconditioner::has_coarse_operator(const DomainBatch& b) {
+  const int64_t m = b.n_dom == 1 ? b.h_ptr[1] - b.h_ptr[0] : 0;
+  return m > 0 && m <= kCoarseOpMax;
+}
+
 void RasPreconditioner::setup_batch(DomainBatch& b, const std::vector<Domain>& doms, bool coarse, hipStream_t ls,
                                     bool fp32, int32_t* flag) {
-  (void)coarse;
   b.n_dom = static_cast<int>(doms.size());
   b.h_ptr.assign(b.n_dom + 1, 0);
   std::vector<int64_t> mptr(b.n_dom + 1, 0);
@@ -2224,21 +2193,13 @@ void RasPreconditioner::setup_batch(DomainBatch& b, const std::vector<Domain>& d
     return;
   }
   const int n0 = static_cast<int>(b.h_ptr.back() - l_);
-  if (b.n_dom == 1 && n0 > 4 * kTile) {
+  const bool op = coarse && has_coarse_operator(b);
+  if (b.n_dom == 1 && (op || n0 > 4 * kTile)) {
     // One large matrix (the coarse grid): many workgroups per panel step
     // instead of one workgroup for the whole factorisation.
-    tmp->inv.resize(static_cast<size_t>(kNb) * kNb);
-    for (int k0 = 0; k0 < n0; k0 += kNb) {
-      cholesky_panel_kernel<<<1, kT, 0, ls>>>(b.mat.get(), n0, k0, flag, tmp->inv.get());
-      PAM_LAUNCH_CHECK();
-      const int rem = n0 - std::min(kNb, n0 - k0) - k0;
-      if (rem <= 0) break;
-      cholesky_rows_kernel<<<ceil_div(rem, kT), kT, 0, ls>>>(b.mat.get(), n0, k0, tmp->inv.get());
-      PAM_LAUNCH_CHECK();
-      const int nt = (rem + kTile - 1) / kTile;
-      cholesky_trailing_kernel<<<nt * (nt + 1) / 2, kT, 0, ls>>>(b.mat.get(), n0, k0);
-      PAM_LAUNCH_CHECK();
-    }
+    tmp->inv.resize(static_cast<size_t>(kCoarseBlk) * kCoarseBlk);
+    if (op) tmp->x.resize(static_cast<size_t>(std::max(n0, 1)) * std::max(n0, 1));
+    launch_coarse_factor(b.mat.get(), n0, flag, op ? tmp->x.get() : nullptr, tmp->inv.get(), ls);
   } else {
     launch_cholesky_batch<double>(coarse ? kNb : factor_panel(b, false, ls, tmp->mptr), b.n_dom, b.ptr.get(), l_,
                                   b.mat_ptr.get(), b.mat.get(), flag, ls);

@@ -138,7 +138,9 @@ class RasPreconditioner : public LinearOperator {
     std::vector<uint8_t> inner;
     std::vector<int64_t> mptr;
     DevBuf<double> u, atl, rows, inv;
+    DevBuf<double> x, t, atop;  // coarse grid: inverse of the factor, scratch, A_top
   };
+  static bool has_coarse_operator(const DomainBatch& b);
   std::vector<std::unique_ptr<SetupTmp>> setup_tmp_;
   void solve(int level, const double* d_res, double* d_w);
   void launch_solve(const DomainBatch& b, int level, int threads, const double* d_res, double* d_w);
