@@ -27,6 +27,8 @@ void radix_sort_pairs(uint64_t* keys, int32_t* vals, int64_t n, int bits, DevBuf
 void launch_iota(int32_t* vals, int64_t n, hipStream_t s);
 // out[i] = in[idx[i]] (gather) for doubles
 void launch_gather_f64(const double* in, const int32_t* idx, int64_t n, double* out, hipStream_t s);
+
+// ---- direct_sums.hip --------------------------------------------------------
 // FP64 direct sum: out[i] (+)= sum_j w[j] * phi(t_i - s_j) over transformed points.
 void direct_sum_f64(const RbfDesc& rbf, const double* src, const double* w, int64_t n_src,
                     const double* trg, int64_t n_trg, double* out, bool accumulate,
@@ -41,14 +43,22 @@ void direct_sum_f64_into(const RbfDesc& rbf, const double* src, const double* w,
                          const double* trg, int64_t n_trg, double* out, bool accumulate, double* partial,
                          hipStream_t s);
 // FP64 direct gradient sum (gradient-transpose kernel): out3[3 i + k] =
-// (A^T sum_j w[j] grad phi(t_i - s_j))_k over transformed points (rbf_eval.hip).
+// (A^T sum_j w[j] grad phi(t_i - s_j))_k over transformed points.
 void direct_gradient_f64(const RbfDesc& rbf, const double* src, const double* w, int64_t n_src,
                          const double* trg, int64_t n_trg, double* out3, DevBuf<double>& scratch,
                          hipStream_t s);
 // FP64 direct sum of column kcol of the Hessian kernel: out3[3 i + c] =
-// (A^T sum_j w[j] H(t_i - s_j) A e_kcol)_c over transformed points (rbf_eval.hip).
+// (A^T sum_j w[j] H(t_i - s_j) A e_kcol)_c over transformed points.
 void direct_hessian_column_f64(const RbfDesc& rbf, const double* src, const double* w, int64_t n_src,
                                const double* trg, int64_t n_trg, int kcol, double* out3, DevBuf<double>& scratch,
+                               hipStream_t s);
+// FP64 direct sums over sources with 3-vector weights w3 (x y z per source,
+// untransformed): out[i] = -sum_j (A w3_j) . grad phi(t_i - s_j), and
+// out3[3 i + k] = -(A^T sum_j H(t_i - s_j) A w3_j)_k, over transformed points.
+void direct_dipole_f64(const RbfDesc& rbf, const double* src, const double* w3, int64_t n_src, const double* trg,
+                       int64_t n_trg, double* out, DevBuf<double>& scratch, hipStream_t s);
+void direct_dipole_hessian_f64(const RbfDesc& rbf, const double* src, const double* w3, int64_t n_src,
+                               const double* trg, int64_t n_trg, double* out3, DevBuf<double>& scratch,
                                hipStream_t s);
 // Batched FP64 direct sums over host query sets, for small evaluations of
 // several resident models at once: one upload, one direct-sum launch, one
@@ -81,6 +91,8 @@ class DirectBatch {
   HostStage<double> up_, down_;
   DevBuf<double> d_in_, d_part_, d_out_;
 };
+
+// ---- util.hip: polynomials ----
 // out3[3 i + k] += d/dx_k sum_m c_m m(p_i) (gradient of the polynomial part).
 void launch_poly_grad(int degree, const double* pts, int64_t n, const double* d_coeffs, double* out3,
                       hipStream_t s);

@@ -6,6 +6,7 @@
 //
 // The kernels, the source split and the summation order are those of
 // pam_direct_evaluate, so for the same inputs the result is the same bits.
+#include <algorithm>
 #include <array>
 #include <mutex>
 
@@ -16,11 +17,14 @@
 namespace {
 
 constexpr int64_t kScratchDoubles = PAM_NOALLOC_SCRATCH_BYTES / 8;
+// Partial sums beyond those that the documented limit counts: up to 2,048
+// chunks of 64 targets where the sources are split more finely than it says.
+constexpr int64_t kSlackDoubles = 2048 * 64 + 32768;
 
 // The shared work area. Host code never uses this name as an address: it
 // stands for the host-side shadow, not device memory. The device address is
 // looked up per device with hipGetSymbolAddress and kept in g_ptr.
-__device__ __align__(256) double scratch[kScratchDoubles];
+__device__ __align__(256) double scratch[kScratchDoubles + kSlackDoubles];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_mu;
@@ -42,6 +46,15 @@ double* scratch_ptr() {
   return g_ptr[dev];
 }
 
+// Partial sums that a call is charged for: one per target and chunk of at
+// least 1,024 sources, with about 2,048 blocks of 256 targets and a chunk.
+int64_t counted_partial(int64_t n_trg, int64_t n_src) {
+  if (n_trg == 0) return 0;
+  const int64_t gx = (n_trg + 255) / 256, want = (2048 + gx - 1) / gx;
+  const int64_t chunk = std::max<int64_t>(n_src / want, 1024);
+  return (n_src > 0 ? (n_src + chunk - 1) / chunk : 1) * n_trg;
+}
+
 }  // namespace
 
 extern "C" {
@@ -55,12 +68,15 @@ int pam_direct_evaluate_device_noalloc(const pam_rbf* rbf, const double* d_src, 
     if (n_src > 0 && (!d_src || !d_w)) pam::throw_invalid("null source or weight pointer");
     if (n_trg > 0 && (!d_trg || !d_out)) pam::throw_invalid("null target or output pointer");
     // Work area: transformed targets, transformed sources, partial sums.
-    const int64_t need = 3 * n_trg + 3 * n_src + static_cast<int64_t>(pam::direct_partial_size(n_trg, n_src));
+    const int64_t need = 3 * n_trg + 3 * n_src + counted_partial(n_trg, n_src);
     if (need > kScratchDoubles)
       pam::throw_invalid("pam_direct_evaluate_device_noalloc: 3 n_trg + 3 n_src + partial sums = " +
                          std::to_string(need) + " doubles exceed the fixed work area of " +
                          std::to_string(kScratchDoubles) + " doubles (PAM_NOALLOC_SCRATCH_BYTES)");
     if (n_trg == 0) return;
+    if (3 * n_trg + 3 * n_src + static_cast<int64_t>(pam::direct_partial_size(n_trg, n_src)) >
+        kScratchDoubles + kSlackDoubles)
+      pam::throw_runtime("direct sum: partial sums exceed the work area");
     double* base = scratch_ptr();
     hipStream_t s = static_cast<hipStream_t>(stream);
     double* t_pts = base;

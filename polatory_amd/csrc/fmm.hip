@@ -577,8 +577,9 @@ constexpr int kMfSrc = kThreads;  // sources staged per chunk: one per thread
 constexpr int kMfMaxTiles = 5;  // 16-target tiles per wave and pass
 constexpr double kMfUnit = 0x1p-9;
 // Workgroups wanted in a launch of one evaluation: a leaf's tiles are shared
-// out to several workgroups when there are fewer leaves.
-constexpr int kMfBlocks = 4096, kMfMaxParts = 8;
+// out to several workgroups when there are fewer leaves, kMfPartTiles at least
+// to each (every one of them stages the leaf's sources for itself).
+constexpr int kMfBlocks = 4096, kMfMaxParts = 8, kMfPartTiles = 4;
 
 using h16x4 = _Float16 __attribute__((ext_vector_type(4)));
 using f32x4v = float __attribute__((ext_vector_type(4)));
@@ -739,7 +740,9 @@ __global__ void __launch_bounds__(kThreads, 4) p2p_mf_jobs_kernel(P2PJobs<float>
   }
   const int ts = j.tls[leaf], te = j.tls[leaf + 1];
   const int tiles = (te - ts + 15) / 16;
-  const int tile0 = tiles * part / j.parts, tile1 = tiles * (part + 1) / j.parts;
+  const int parts = min(j.parts, max(1, tiles / kMfPartTiles));
+  if (part >= parts) return;
+  const int tile0 = tiles * part / parts, tile1 = tiles * (part + 1) / parts;
   if (tile0 == tile1) return;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   if (wave == 0) {

@@ -1,4 +1,5 @@
-// Gradient-kernel sources as three gradient-transpose passes.
+// Sources with 3-vector weights: one direct sum, or three gradient-transpose
+// (Hessian-column) passes of the FMM.
 #include "fmm_dipole.hpp"
 
 #include "device_api.hpp"
@@ -52,18 +53,20 @@ void DipoleSourceEvaluator::evaluate(double* out, int64_t n, bool on_device) {
     tmp_.resize(static_cast<size_t>(nt));
     d_out = tmp_.get();
   }
-  wk_.resize(static_cast<size_t>(n_src_));
-  g3_.resize(static_cast<size_t>(nt) * 3);
-  for (int k = 0; k < 3; k++) {
-    if (n_src_ > 0) {
-      extract_component_kernel<<<ceil_div(n_src_, 256), 256, 0, s>>>(w3_.get(), n_src_, k, wk_.get());
-      PAM_LAUNCH_CHECK();
-    }
-    ev_.set_weights(wk_.get(), n_src_, true);
-    ev_.evaluate_gradient(g3_.get(), nt, true);
-    if (nt > 0) {
-      minus_component_kernel<<<ceil_div(nt, 256), 256, 0, s>>>(g3_.get(), nt, k, d_out);
-      PAM_LAUNCH_CHECK();
+  if (!ev_.evaluate_vector_direct(w3_.get(), false, d_out, nt)) {
+    wk_.resize(static_cast<size_t>(n_src_));
+    g3_.resize(static_cast<size_t>(nt) * 3);
+    for (int k = 0; k < 3; k++) {
+      if (n_src_ > 0) {
+        extract_component_kernel<<<ceil_div(n_src_, 256), 256, 0, s>>>(w3_.get(), n_src_, k, wk_.get());
+        PAM_LAUNCH_CHECK();
+      }
+      ev_.set_weights(wk_.get(), n_src_, true);
+      ev_.evaluate_gradient(g3_.get(), nt, true);
+      if (nt > 0) {
+        minus_component_kernel<<<ceil_div(nt, 256), 256, 0, s>>>(g3_.get(), nt, k, d_out);
+        PAM_LAUNCH_CHECK();
+      }
     }
   }
   if (!on_device) {
@@ -96,18 +99,20 @@ void DipoleHessianEvaluator::evaluate(double* out, int64_t n, bool on_device) {
     tmp_.resize(static_cast<size_t>(nt) * 3);
     d_out = tmp_.get();
   }
-  wk_.resize(static_cast<size_t>(n_src_));
-  g3_.resize(static_cast<size_t>(nt) * 3);
-  for (int k = 0; k < 3; k++) {
-    if (n_src_ > 0) {
-      extract_component_kernel<<<ceil_div(n_src_, 256), 256, 0, s>>>(w3_.get(), n_src_, k, wk_.get());
-      PAM_LAUNCH_CHECK();
-    }
-    ev_.set_weights(wk_.get(), n_src_, true);
-    ev_.evaluate_hessian_column(k, g3_.get(), nt, true);
-    if (nt > 0) {
-      minus_all_kernel<<<ceil_div(3 * nt, 256), 256, 0, s>>>(g3_.get(), 3 * nt, k, d_out);
-      PAM_LAUNCH_CHECK();
+  if (!ev_.evaluate_vector_direct(w3_.get(), true, d_out, nt)) {
+    wk_.resize(static_cast<size_t>(n_src_));
+    g3_.resize(static_cast<size_t>(nt) * 3);
+    for (int k = 0; k < 3; k++) {
+      if (n_src_ > 0) {
+        extract_component_kernel<<<ceil_div(n_src_, 256), 256, 0, s>>>(w3_.get(), n_src_, k, wk_.get());
+        PAM_LAUNCH_CHECK();
+      }
+      ev_.set_weights(wk_.get(), n_src_, true);
+      ev_.evaluate_hessian_column(k, g3_.get(), nt, true);
+      if (nt > 0) {
+        minus_all_kernel<<<ceil_div(3 * nt, 256), 256, 0, s>>>(g3_.get(), 3 * nt, k, d_out);
+        PAM_LAUNCH_CHECK();
+      }
     }
   }
   if (!on_device) {

@@ -997,16 +997,40 @@ void FmmEvaluator::evaluate_impl(double* out, int64_t n, bool on_device) {
   } else {
     for (int i = 1; i <= 8; i++) record(i);
   }
-  stats_.precision = cfg_.precision;
-  stats_.order = cfg_.order;
-  stats_.leaf_level = stats_.direct ? -1 : src.src_tree_.level;
-  stats_.n_src_leaves = stats_.direct ? 0 : src.src_tree_.n_leaves();
-  stats_.n_trg_leaves = stats_.direct ? 0 : target_tree().n_leaves();
-  stats_pending_ = true;
+  finish_stats();
   if (!on_device) {
     tmp.download(out, static_cast<size_t>(nt) * per, stream_);
     PAM_HIP(hipStreamSynchronize(stream_));
   }
+}
+
+void FmmEvaluator::finish_stats() {
+  stats_.precision = cfg_.precision;
+  stats_.order = cfg_.order;
+  stats_.leaf_level = stats_.direct ? -1 : S().src_tree_.level;
+  stats_.n_src_leaves = stats_.direct ? 0 : S().src_tree_.n_leaves();
+  stats_.n_trg_leaves = stats_.direct ? 0 : target_tree().n_leaves();
+  stats_pending_ = true;
+}
+
+bool FmmEvaluator::evaluate_vector_direct(const double* d_w3, bool hessian, double* d_out, int64_t n) {
+  if (so_ || symmetric_) return false;
+  const int64_t nt = n_trg();
+  if (n != nt) throw_invalid("output size must equal the number of target points");
+  if (nt == 0 || n_src_ == 0 || !config_valid_) return false;
+  timing_valid_ = true;
+  record(0);
+  if (!use_direct()) return false;
+  stats_ = FmmStats{};
+  for (int i = 1; i <= 5; i++) record(i);
+  if (hessian)
+    direct_dipole_hessian_f64(rbf_, src_pts_.get(), d_w3, n_src_, trg_pts_.get(), nt, d_out, direct_scratch_, stream_);
+  else
+    direct_dipole_f64(rbf_, src_pts_.get(), d_w3, n_src_, trg_pts_.get(), nt, d_out, direct_scratch_, stream_);
+  for (int i = 6; i <= 8; i++) record(i);
+  stats_.direct = 1;
+  finish_stats();
+  return true;
 }
 
 const FmmStats& FmmEvaluator::stats() {

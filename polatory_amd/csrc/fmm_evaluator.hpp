@@ -108,6 +108,12 @@ class FmmEvaluator {
   // block of make_fmm_hessian_evaluator): out has 3 n_trg entries,
   // A^T sum_j w_j H(A (t_i - s_j)) A e_k per target. Source-target only.
   void evaluate_hessian_column(int k, double* out, int64_t n, bool on_device);
+  // Sums over sources with 3-vector weights (d_w3: x y z per source) in one
+  // pass, when this evaluator would take the direct sum: values
+  // (fmm/gradient_kernel.hpp) or, with hessian, 3-vectors
+  // (fmm/hessian_kernel.hpp) at the targets. Returns false, with nothing done,
+  // when it would not.
+  bool evaluate_vector_direct(const double* d_w3, bool hessian, double* d_out, int64_t n);
   // Makes this a gradient-transpose evaluator (make_fmm_evaluator.cpp:119-148):
   // evaluate() returns the gradients and the accuracy search measures them.
   void set_gradient_kernel(bool on);
@@ -159,6 +165,7 @@ class FmmEvaluator {
   template <class TP>
   void run_fmm(double* d_out);
   void evaluate_impl(double* out, int64_t n, bool on_device);
+  void finish_stats();
   void invalidate_expansions();
   void record(int idx, hipStream_t s = nullptr);
 

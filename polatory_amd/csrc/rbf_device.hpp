@@ -77,6 +77,26 @@ inline double phi_shape_const(int kind, double b) {
   return sizeof(T) == 4 && kind == kExp ? b * 1.4426950408889634074 : b;
 }
 
+// The same for x > 0 (no test for zero).
+__device__ __forceinline__ double sqrt_pos(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double s = x * y, h = 0.5 * y;
+  const double r = fma(-s, h, 0.5);
+  s = fma(s, r, s);
+  h = fma(h, r, h);
+  return fma(fma(-s, s, x), h, s);
+}
+
+// sum_k c_k m_k(x, y, z) over the monomials of degree 0..2
+// (polynomial/monomial_basis.hpp:198-209 order: 1, x, y, z, x^2, xy, xz, y^2, yz, z^2).
+__device__ __forceinline__ double poly_value(int degree, const double* __restrict__ c, double x, double y,
+                                             double z) {
+  double acc = c[0];
+  if (degree >= 1) acc += c[1] * x + c[2] * y + c[3] * z;
+  if (degree >= 2) acc += c[4] * x * x + c[5] * x * y + c[6] * x * z + c[7] * y * y + c[8] * y * z + c[9] * z * z;
+  return acc;
+}
+
 // phi without its factor a, for loops that fold a into the weights:
 // r2c = r^2 + b for bh3 / th3 (the caller seeds its sum of squares with b),
 // r2c = r^2 for exp.
