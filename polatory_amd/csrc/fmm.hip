@@ -580,6 +580,11 @@ constexpr double kMfUnit = 0x1p-9;
 // out to several workgroups when there are fewer leaves, kMfPartTiles at least
 // to each (every one of them stages the leaf's sources for itself).
 constexpr int kMfBlocks = 4096, kMfMaxParts = 8, kMfPartTiles = 4;
+// Where that leaves fewer than kMfFill workgroups (four rounds of the chip's
+// 1,024), the source chunks are dealt out as well, kMfPartChunks at least to
+// each part, and the parts' sums added by a second launch. 220,731 sources in
+// 512 leaves: 43,881 targets 0.349 to 0.148 ms, 8,000 targets 0.170 to 0.083 ms.
+constexpr int kMfFill = 4096, kMfMaxSparts = 3, kMfPartChunks = 4;
 
 using h16x4 = _Float16 __attribute__((ext_vector_type(4)));
 using f32x4v = float __attribute__((ext_vector_type(4)));
@@ -712,6 +717,48 @@ __device__ __forceinline__ void mf_tiles(const h16x4* sa, const f32x4v* sw, int 
   }
 }
 
+// The leaf, target part and source part of a job's workgroup. Groups of 64
+// leaves: the workgroups of eight consecutive (sibling) leaves on one XCD
+// (workgroup i runs on XCD i % 8), whose L2 then holds their shared neighbours.
+template <class T>
+__device__ __forceinline__ void p2p_unit(const P2PJob<T>& j, int lb, int* leaf, int* part, int* spart) {
+  const int units = j.parts * j.sparts, per = 64 * units, grp = lb / per;
+  int u;
+  if ((grp + 1) * 64 <= j.n_leaves) {
+    const int r = lb - grp * per, q = r / 8;
+    *leaf = grp * 64 + (r & 7) * 8 + q / units;
+    u = q % units;
+  } else {
+    *leaf = lb / units;
+    u = lb % units;
+  }
+  *part = u / j.sparts;
+  *spart = u % j.sparts;
+}
+
+// Output of target i (tree order): the sum plus the far field in input order,
+// or this source part's partial sum.
+template <class T>
+__device__ __forceinline__ void p2p_store(const P2PJob<T>& j, int spart, int i, double sum) {
+  if (j.sparts > 1) j.partial[static_cast<int64_t>(spart) * j.n_trg + i] = sum;
+  else j.out[j.tperm[i]] = (j.y_far ? j.y_far[i] : 0.0) + sum;
+}
+
+// The source parts of every target, in order.
+template <class T>
+__global__ void p2p_fold_kernel(P2PJobs<T> jobs) {
+  for (int k = 0; k < jobs.n; k++) {
+    const P2PJob<T>& j = jobs.j[k];
+    if (j.sparts < 2) continue;
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < j.n_trg;
+         i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+      double sum = 0.0;
+      for (int s = 0; s < j.sparts; s++) sum += j.partial[static_cast<int64_t>(s) * j.n_trg + i];
+      j.out[j.tperm[i]] = (j.y_far ? j.y_far[i] : 0.0) + sum;
+    }
+  }
+}
+
 template <int KIND, bool kComp>
 __global__ void __launch_bounds__(kThreads, 4) p2p_mf_jobs_kernel(P2PJobs<float> jobs) {
   __shared__ h16x4 sa[kMfSrc / 16 * 192];  // [16-source block][product][reduction index / 4][row]
@@ -722,22 +769,8 @@ __global__ void __launch_bounds__(kThreads, 4) p2p_mf_jobs_kernel(P2PJobs<float>
   __shared__ int nb_count;
   __shared__ double red[4][kMfMaxTiles * 16];
   const P2PJob<float>& j = p2p_job_of(jobs, static_cast<int>(blockIdx.x));
-  // Groups of 64 leaves: the workgroups of eight consecutive (sibling) leaves
-  // on one XCD (workgroup i runs on XCD i % 8), whose L2 then holds their
-  // shared neighbours.
-  int leaf, part;
-  {
-    const int lb = static_cast<int>(blockIdx.x) - j.first_block;
-    const int per = 64 * j.parts, grp = lb / per;
-    if ((grp + 1) * 64 <= j.n_leaves) {
-      const int r = lb - grp * per, q = r / 8;
-      leaf = grp * 64 + (r & 7) * 8 + q / j.parts;
-      part = q % j.parts;
-    } else {
-      leaf = lb / j.parts;
-      part = lb % j.parts;
-    }
-  }
+  int leaf, part, spart;
+  p2p_unit(j, static_cast<int>(blockIdx.x) - j.first_block, &leaf, &part, &spart);
   const int ts = j.tls[leaf], te = j.tls[leaf + 1];
   const int tiles = (te - ts + 15) / 16;
   const int parts = min(j.parts, max(1, tiles / kMfPartTiles));
@@ -777,6 +810,8 @@ __global__ void __launch_bounds__(kThreads, 4) p2p_mf_jobs_kernel(P2PJobs<float>
   }
   __syncthreads();
   const int nnb = nb_count, total = nb_start[nnb];
+  // This source part's chunks: every sparts-th one.
+  const int first = spart * kMfSrc, step = j.sparts * kMfSrc;
   const float pa = j.pa, pb = j.pb;
   const float seed = phi_seed<float, KIND>(pb);
   // Entries that no source changes: the constants against the targets' own
@@ -817,8 +852,8 @@ __global__ void __launch_bounds__(kThreads, 4) p2p_mf_jobs_kernel(P2PJobs<float>
       while (k + 1 < nnb && nb_start[k + 1] <= g) k++;
       q = j.spts[nb_src[k] + (g - nb_start[k])];
     };
-    fetch(tid);
-    for (int cb = 0; cb < total; cb += kMfSrc) {
+    fetch(first + tid);
+    for (int cb = first; cb < total; cb += step) {
       const int nblk = (min(kMfSrc, total - cb) + 15) / 16;
       MfCoord x = mf_split(q.x), y = mf_split(q.y), z = mf_split(q.z);
       x.i += nb_off[k][0];  // exact: an integer number of units
@@ -836,7 +871,7 @@ __global__ void __launch_bounds__(kThreads, 4) p2p_mf_jobs_kernel(P2PJobs<float>
       a[128 + 16] = mf_pack(y.f2, z.f2, c * x.i, c * y.i);
       a[128 + 32] = mf_pack(c * z.i, s.d1, s.d2, 1.0f);
       reinterpret_cast<float*>(sw)[tid] = static_cast<float>(q.w) * pa;  // the kernel's factor a folded in
-      fetch(cb + kMfSrc + tid);
+      fetch(cb + step + tid);
       __syncthreads();
       switch (mine) {
         case 1: mf_tiles<KIND, kComp, 1>(sa, sw, nblk, split, S, cols, pb, seed, tot); break;
@@ -864,8 +899,7 @@ __global__ void __launch_bounds__(kThreads, 4) p2p_mf_jobs_kernel(P2PJobs<float>
         if (m >= mine || i >= te) continue;
         double sum = sums[m];
         for (int s = 1; s < S; s++) sum += red[s * G + grp][m * 16 + lane];
-        const double far = j.y_far ? j.y_far[i] : 0.0;
-        j.out[j.tperm[i]] = far + sum;
+        p2p_store(j, spart, i, sum);
       }
     }
     __syncthreads();  // red is written again in the next pass
@@ -2294,7 +2328,8 @@ L2PJob<T> make_l2p_job(const Tree& t, const T* l_leaf, const V4<T>* pts, T* y_fa
 
 template <class T>
 P2PJob<T> make_p2p_job(const RbfDesc& rbf, const Tree& trg, const Tree& src, const Lists& lists,
-                       const V4<double>* tpts, const V4<double>* spts, const double* y_far, double* out) {
+                       const V4<double>* tpts, const V4<double>* spts, const double* y_far, double* out,
+                       DevBuf<double>& partial) {
   P2PJob<T> j{};
   const double h = trg.box.width / std::ldexp(1.0, trg.level) / 2.0;
   // The mixed form's kernel works in units of kMfUnit of the leaf half width.
@@ -2310,7 +2345,20 @@ P2PJob<T> make_p2p_job(const RbfDesc& rbf, const Tree& trg, const Tree& src, con
   j.pb = static_cast<T>(phi_shape_const<T>(rbf.kind, pc.b));
   j.out = out;
   j.n_leaves = static_cast<int>(trg.n_leaves());
-  j.parts = sizeof(T) == 4 && j.n_leaves > 0 ? std::clamp((kMfBlocks + j.n_leaves - 1) / j.n_leaves, 1, kMfMaxParts) : 1;
+  j.n_trg = trg.n_points;
+  j.parts = j.sparts = 1;
+  if (sizeof(T) == 4 && j.n_leaves > 0) {
+    j.parts = std::clamp((kMfBlocks + j.n_leaves - 1) / j.n_leaves, 1, kMfMaxParts);
+    // averages over the leaves
+    const double tiles = static_cast<double>(j.n_trg) / j.n_leaves / 16;
+    const double blocks = j.n_leaves * std::clamp(tiles / kMfPartTiles, 1.0, static_cast<double>(j.parts));
+    const double chunks = 27.0 * static_cast<double>(src.n_points) / static_cast<double>(std::max<int64_t>(src.n_leaves(), 1)) / kMfSrc;
+    j.sparts = std::clamp(static_cast<int>(std::min(kMfFill / blocks, chunks / kMfPartChunks)), 1, kMfMaxSparts);
+    if (j.sparts > 1) {
+      partial.resize(static_cast<size_t>(j.sparts) * j.n_trg);
+      j.partial = partial.get();
+    }
+  }
   return j;
 }
 
@@ -2337,11 +2385,12 @@ template <class T>
 void launch_p2p_jobs(int kind, bool compensated, const P2PJob<T>* jobs, int n, hipStream_t s) {
   if (n < 1 || n > kMaxFmmJobs) throw_runtime("P2P job count out of range");
   P2PJobs<T> t{};
-  int64_t total = 0;
+  int64_t total = 0, fold = 0;  // fold: targets of the largest job with source parts
   for (int k = 0; k < n; k++) {
     t.j[t.n] = jobs[k];
     t.j[t.n].first_block = static_cast<int>(total);
-    total += static_cast<int64_t>(jobs[k].n_leaves) * jobs[k].parts;
+    total += static_cast<int64_t>(jobs[k].n_leaves) * jobs[k].parts * jobs[k].sparts;
+    if (jobs[k].sparts > 1) fold = std::max<int64_t>(fold, jobs[k].n_trg);
     if (jobs[k].n_leaves > 0) t.n++;
   }
   if (total == 0) return;
@@ -2353,6 +2402,10 @@ void launch_p2p_jobs(int kind, bool compensated, const P2PJob<T>* jobs, int n, h
     else p2p_mf_jobs_kernel<decltype(K)::value, false><<<grid, kThreads, 0, s>>>(t);
   });
   PAM_LAUNCH_CHECK();
+  if (fold > 0) {
+    p2p_fold_kernel<T><<<ceil_div(fold, kThreads), kThreads, 0, s>>>(t);
+    PAM_LAUNCH_CHECK();
+  }
 }
 
 template <class T>
@@ -2365,10 +2418,10 @@ void launch_l2p(int p, const Tree& t, const T* l_leaf, const V4<T>* pts, T* y_fa
 
 template <class T>
 void launch_p2p(const RbfDesc& rbf, const Tree& trg, const Tree& src, const Lists& lists,
-                const V4<double>* tpts, const V4<double>* spts, const double* y_far, double* out, hipStream_t s,
-                bool compensated) {
+                const V4<double>* tpts, const V4<double>* spts, const double* y_far, double* out,
+                DevBuf<double>& partial, hipStream_t s, bool compensated) {
   if (trg.n_leaves() == 0) return;
-  const P2PJob<T> j = make_p2p_job<T>(rbf, trg, src, lists, tpts, spts, y_far, out);
+  const P2PJob<T> j = make_p2p_job<T>(rbf, trg, src, lists, tpts, spts, y_far, out, partial);
   launch_p2p_jobs<T>(rbf.kind, compensated, &j, 1, s);
 }
 
@@ -2530,9 +2583,9 @@ void launch_m2l_batch(const M2LOperator& op, const std::vector<M2LLevelSpec<TM, 
   template void launch_l2p<T>(int, const Tree&, const T*, const V4<T>*, T*, hipStream_t, bool);           \
   template L2PJob<T> make_l2p_job<T>(const Tree&, const T*, const V4<T>*, T*, bool, int);                   \
   template P2PJob<T> make_p2p_job<T>(const RbfDesc&, const Tree&, const Tree&, const Lists&, const V4<double>*, \
-                                     const V4<double>*, const double*, double*);                                 \
+                                     const V4<double>*, const double*, double*, DevBuf<double>&);                \
   template void launch_p2p<T>(const RbfDesc&, const Tree&, const Tree&, const Lists&, const V4<double>*, \
-                              const V4<double>*, const double*, double*, hipStream_t, bool);                 \
+                              const V4<double>*, const double*, double*, DevBuf<double>&, hipStream_t, bool);   \
   template void launch_p2p_grad<T>(const RbfDesc&, const Tree&, const Tree&, const Lists&, const V4<double>*, \
                                    const V4<double>*, double*, hipStream_t);                                  \
   template void launch_p2p_hess_col<T>(const RbfDesc&, const Tree&, const Tree&, const Lists&, const V4<double>*, \

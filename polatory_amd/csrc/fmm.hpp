@@ -67,7 +67,9 @@ struct P2PJob {
   const int32_t* tperm;  // tree order -> input order of the targets
   double* out;           // output, input order
   T pa, pb;              // kernel constants in the leaf unit (phi_shape_const)
-  int n_leaves, parts, first_block;  // parts: workgroups per leaf
+  double* partial;       // [sparts][n_trg] sums of the source parts, tree order (sparts > 1)
+  int64_t n_trg;
+  int n_leaves, parts, sparts, first_block;  // parts x sparts workgroups per leaf: target tiles x sources
 };
 template <class T>
 struct P2PJobs {
@@ -90,7 +92,8 @@ struct L2PJobs {
 };
 template <class T>
 P2PJob<T> make_p2p_job(const RbfDesc& rbf, const Tree& trg, const Tree& src, const Lists& lists,
-                       const V4<double>* tpts, const V4<double>* spts, const double* y_far, double* out);
+                       const V4<double>* tpts, const V4<double>* spts, const double* y_far, double* out,
+                       DevBuf<double>& partial);
 template <class T>
 L2PJob<T> make_l2p_job(const Tree& t, const T* l_leaf, const V4<T>* pts, T* y_far, bool add_to_output, int kpad);
 // The near field and far field of one evaluation, recorded instead of
@@ -117,8 +120,8 @@ void launch_l2p(int p, const Tree& t, const T* l_leaf, const V4<T>* pts, T* y_fa
 // out[perm[i]] = y_far[i] + near field, FP64 output in input order.
 template <class T>
 void launch_p2p(const RbfDesc& rbf, const Tree& trg, const Tree& src, const Lists& lists,
-                const V4<double>* tpts, const V4<double>* spts, const double* y_far, double* out, hipStream_t s,
-                bool compensated = false);  // compensated: Kahan sums (FP32 only)
+                const V4<double>* tpts, const V4<double>* spts, const double* y_far, double* out,
+                DevBuf<double>& partial, hipStream_t s, bool compensated = false);  // compensated: Kahan sums (FP32 only)
 // Gradients at the targets (fmm/gradient_transpose_kernel.hpp:47-62): the
 // near field writes A^T sum_j w_j grad phi into out3 (n x 3, input order);
 // the far field then adds A^T grad of the leaf local expansions.

@@ -667,8 +667,8 @@ void FmmEvaluator::run_fmm(double* d_out) {
       defer_->fp32 = sizeof(TP) == 4;
       defer_->compensated = cfg_.precision == kMixedComp;
       defer_->kind = rbf_.kind;
-      if constexpr (sizeof(TP) == 4) defer_->p2p32 = make_p2p_job<float>(rbf_, tt, stree, lists_, tpts, spts, nullptr, d_out);
-      else defer_->p2p64 = make_p2p_job<double>(rbf_, tt, stree, lists_, tpts, spts, nullptr, d_out);
+      if constexpr (sizeof(TP) == 4) defer_->p2p32 = make_p2p_job<float>(rbf_, tt, stree, lists_, tpts, spts, nullptr, d_out, st.p2p_partial);
+      else defer_->p2p64 = make_p2p_job<double>(rbf_, tt, stree, lists_, tpts, spts, nullptr, d_out, st.p2p_partial);
       return;
     }
     PAM_HIP(hipEventRecord(fork_ev_, stream_));
@@ -676,7 +676,7 @@ void FmmEvaluator::run_fmm(double* d_out) {
     record(7, ps);
     if (hess_col_ >= 0) launch_p2p_hess_col<TP>(rbf_, tt, stree, lists_, tpts, spts, hess_col_, d_out, ps);
     else if (grad_) launch_p2p_grad<TP>(rbf_, tt, stree, lists_, tpts, spts, d_out, ps);
-    else launch_p2p<TP>(rbf_, tt, stree, lists_, tpts, spts, nullptr, d_out, ps, cfg_.precision == kMixedComp);
+    else launch_p2p<TP>(rbf_, tt, stree, lists_, tpts, spts, nullptr, d_out, st.p2p_partial, ps, cfg_.precision == kMixedComp);
     record(8, ps);
     PAM_HIP(hipEventRecord(join_ev_, ps));
   };

@@ -54,7 +54,7 @@ struct FmmState {
   std::vector<DevBuf<float>> m32;      // per level, FP32 copy of m (mixed-form M2L operand)
   std::vector<DevBuf<double>> mt, lt;  // per level, compressed coefficients
   std::vector<DevBuf<float>> mt32;     // per level, FP32 copy of mt (mixed-form transfer operand)
-  DevBuf<double> y_far;
+  DevBuf<double> p2p_partial;          // near-field sums of the source parts
   DevBuf<double> m2l_partial;          // split-reduction partial sums of the dense M2L
   M2LSchedule m2l_sched;
   DevBuf<float> m2l_pairs32;           // per-pair transfers of the pair-major M2L (mixed form)

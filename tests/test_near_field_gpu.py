@@ -1,7 +1,8 @@
 """The near field alone: points inside the eight central leaves of a level-2
 tree are all neighbours of each other, so no far field contributes. Sizes sit
 on the edges of the mixed kernel's tiles (16 targets, 5 tiles per wave, 256
-sources per chunk). Calls go through the C ABI."""
+sources per chunk), the last one where the sources are shared out over several
+workgroups. Calls go through the C ABI."""
 import numpy as np
 import pytest
 
@@ -17,7 +18,7 @@ H = 1.01 / 4 / 2  # leaf half width
 @pytest.mark.parametrize("precision", ["mixed", "mixed_comp"])
 @pytest.mark.parametrize("kind", list(KINDS))
 @pytest.mark.parametrize("n_src,n_trg", [(1, 1), (15, 17), (257, 16), (2048, 640), (2049, 81 * 8), (700, 2600),
-                                         (5000, 3000)])
+                                         (5000, 3000), (20000, 120)])
 def test_mixed_near_field_matches_direct_sum(orc, kind, precision, n_src, n_trg):
     print("near field", kind, precision, n_src, n_trg, flush=True)
     name, cls, params = KINDS[kind]
