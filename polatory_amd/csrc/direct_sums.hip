@@ -37,7 +37,7 @@ constexpr int out_per(int mode) { return mode == kDirValue || mode == kDirDipole
 constexpr bool vector_weights(int mode) { return mode == kDirDipole || mode == kDirHessian; }
 
 // Constants of a direct sum: a multiplies the weights (kernel or gradient
-// factor), b as in phi_shape / grad_shape; p0, p1 for the plain expressions.
+// factor), b as in phi_shape / grad_terms; p0, p1 for the plain expressions.
 struct DirectConsts {
   double a, b, p0, p1;
 };
@@ -74,14 +74,6 @@ DirectSplit direct_split(int64_t n_trg, int64_t n_src) {
   return d;
 }
 
-// 1 / sqrt(x): the hardware's reciprocal root (about 2^-23) and one correction
-// of third order, within an ulp.
-__device__ __forceinline__ double rsqrt_nr(double x) {
-  const double y = __builtin_amdgcn_rsq(x);
-  const double e = fma(-(x * y), y, 1.0);
-  return fma(y, e * fma(0.375, e, 0.5), y);
-}
-
 // One pair's term into acc. w: the weight or the vector weight times
 // DirectConsts::a; r2 is seeded (direct_seed).
 template <int KIND, int MODE>
@@ -93,7 +85,7 @@ __device__ __forceinline__ void direct_pair(double dx, double dy, double dz, dou
     else if constexpr (KIND == kTh3) acc[0] = fma(w[0], rho * r2, acc[0]);
     else acc[0] = fma(w[0], exp(b * rho), acc[0]);
   } else {
-    double f, t = 0.0;  // grad_shape, hess_t
+    double f, t = 0.0;  // as in grad_terms
     if constexpr (KIND == kTh3 && MODE != kDirHessian) {
       f = sqrt_pos(r2);
     } else {

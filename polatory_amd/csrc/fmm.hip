@@ -365,169 +365,6 @@ __global__ void __launch_bounds__(kThreads) l2p_jobs_kernel(L2PJobs<T> jobs) {
   l2p_leaf<T, P>(g - j.first_leaf, j.leaf_start, j.pts, j.l, j.kpad, j.y_far, j.perm);
 }
 
-// Targets per thread of the near-field kernel (each source read from LDS
-// serves R pairs): chosen per leaf in [4, kP2PMaxR].
-constexpr int kP2PMinR = 4, kP2PMaxR = 8;
-
-// The R and tp (target slots, a power of two) for a leaf of nt targets: the
-// pair with the fewest idle target slots R tp - nt (ties: the smaller R). A
-// fixed R = 4 rounds 257 targets up to 512 slots, and every idle slot costs
-// a full pass over the leaf's sources; on 1M uniform points (about 244 per
-// leaf) that was a quarter of the pairs computed.
-__device__ __forceinline__ int p2p_shape(int nt, int* tp_out) {
-  int best_r = kP2PMinR, best_tp = kThreads, best_cap = 1 << 30;
-  for (int r = kP2PMinR; r <= kP2PMaxR; r++) {
-    const int per = (nt + r - 1) / r;
-    int tp = 1;
-    while (tp < per && tp < kThreads) tp <<= 1;
-    const int passes = (per + tp - 1) / tp;
-    const int cap = r * tp * passes;
-    if (cap < best_cap) best_cap = cap, best_r = r, best_tp = tp;
-  }
-  *tp_out = best_tp;
-  return best_r;
-}
-
-// The passes of one target leaf of the FP64 near field with R targets per
-// thread and tp target slots (tp x nsplit threads; the sources staged through
-// sp in chunks).
-template <int KIND, int R>
-__device__ __forceinline__ void p2p_passes(int nt, int ts, int tp, int total, int nnb, const int* nb_start,
-                                           const int* nb_src, const double (*nb_off)[3], V4<double>* sp, int cap,
-                                           double (*red)[kThreads], const V4<double>* __restrict__ tpts,
-                                           const V4<double>* __restrict__ spts, const double* __restrict__ y_far,
-                                           const int32_t* __restrict__ tperm, double pa, double pb,
-                                           double* __restrict__ out) {
-  // Every thread carries R targets (ti + r tp), so each source read from LDS
-  // serves R pairs; tp target slots x nsplit source splits fill the 256 lanes.
-  const int nsplit = kThreads / tp;
-  const int ti = threadIdx.x & (tp - 1);
-  const int si = threadIdx.x / tp;
-  for (int c0 = 0; c0 < nt; c0 += R * tp) {
-    V4<double> tq[R];
-    double acc[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-      const int i = c0 + r * tp + ti;
-      tq[r] = i < nt ? tpts[ts + i] : V4<double>{0.0, 0.0, 0.0, 0.0};
-      acc[r] = 0.0;
-    }
-    for (int cb = 0; cb < total; cb += cap) {
-      const int cnt = min(cap, total - cb);
-      __syncthreads();
-      for (int e = threadIdx.x; e < cnt; e += kThreads) {
-        int g = cb + e;
-        int k = 0;
-        while (k + 1 < nnb && nb_start[k + 1] <= g) k++;
-        V4<double> q = spts[nb_src[k] + (g - nb_start[k])];
-        q.x += nb_off[k][0];
-        q.y += nb_off[k][1];
-        q.z += nb_off[k][2];
-        q.w *= pa;  // the kernel's factor a folded into the weight
-        sp[e] = q;
-      }
-      __syncthreads();
-      // Per pair: three differences, three FMAs seeded with the kernel's
-      // offset, the shape function and one FMA. Four sources per trip keep
-      // their LDS reads ahead of the arithmetic; the sum order over sources
-      // is the plain sequential one.
-      const double seed = phi_seed<double, KIND>(pb);
-      auto pair = [&](const V4<double>& q, int r) {
-        const double dx = tq[r].x - q.x, dy = tq[r].y - q.y, dz = tq[r].z - q.z;
-        const double r2 = fma(dz, dz, fma(dy, dy, fma(dx, dx, seed)));
-        acc[r] = fma(q.w, phi_shape<double, KIND>(r2, pb), acc[r]);
-      };
-      int j = si;
-      for (; j + 3 * nsplit < cnt; j += 4 * nsplit) {
-        const V4<double> q0 = sp[j], q1 = sp[j + nsplit], q2 = sp[j + 2 * nsplit], q3 = sp[j + 3 * nsplit];
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-          pair(q0, r);
-          pair(q1, r);
-          pair(q2, r);
-          pair(q3, r);
-        }
-      }
-      for (; j < cnt; j += nsplit) {
-        const V4<double> q = sp[j];
-#pragma unroll
-        for (int r = 0; r < R; r++) pair(q, r);
-      }
-    }
-    __syncthreads();  // red overlays the staged sources
-#pragma unroll
-    for (int r = 0; r < R; r++) red[r][threadIdx.x] = acc[r];
-    __syncthreads();
-    if (si == 0) {
-#pragma unroll
-      for (int r = 0; r < R; r++) {
-        const int i = c0 + r * tp + ti;
-        if (i >= nt) continue;
-        double sum = 0.0;
-        for (int k = 0; k < nsplit; k++) sum += red[r][ti + k * tp];
-        const int gi = ts + i;
-        double far = y_far ? y_far[gi] : 0.0;
-        out[tperm[gi]] = far + sum;
-      }
-    }
-    __syncthreads();
-  }
-}
-
-// One target leaf of one evaluation's FP64 near field.
-template <int KIND>
-__device__ __forceinline__ void p2p_leaf(int leaf, const int32_t* __restrict__ tls, const int32_t* __restrict__ sls,
-                                         const int32_t* __restrict__ p2p, const V4<double>* __restrict__ tpts,
-                                         const V4<double>* __restrict__ spts, const double* __restrict__ y_far,
-                                         const int32_t* __restrict__ tperm, double pa, double pb,
-                                         double* __restrict__ out) {
-  constexpr int CAP = 32768 / static_cast<int>(sizeof(V4<double>));
-  __shared__ V4<double> sp[CAP];
-  __shared__ int nb_start[28];
-  __shared__ int nb_src[27];
-  __shared__ double nb_off[27][3];
-  __shared__ int nb_count;
-  // The split partials of a pass, over the staged sources (read after them).
-  static_assert(kP2PMaxR * kThreads * sizeof(double) <= sizeof(V4<double>) * CAP,
-                "partials exceed the staging buffer");
-  double (*red)[kThreads] = reinterpret_cast<double (*)[kThreads]>(sp);
-  const int ts = tls[leaf], te = tls[leaf + 1];
-  const int nt = te - ts;
-  if (threadIdx.x == 0) {
-    int k = 0, total = 0;
-    for (int s = 0; s < 27; s++) {
-      int sl = p2p[static_cast<int64_t>(leaf) * 27 + s];
-      if (sl < 0) continue;
-      int a = sls[sl], b = sls[sl + 1];
-      nb_src[k] = a;
-      nb_start[k] = total;
-      nb_off[k][0] = 2 * (s / 9 - 1);
-      nb_off[k][1] = 2 * ((s / 3) % 3 - 1);
-      nb_off[k][2] = 2 * (s % 3 - 1);
-      total += b - a;
-      k++;
-    }
-    nb_start[k] = total;
-    nb_count = k;
-  }
-  __syncthreads();
-  const int nnb = nb_count;
-  const int total = nb_start[nnb];
-  int tp = kThreads;
-  const int r = p2p_shape(nt, &tp);
-#define PAM_P2P_PASSES(RR)                                                                                    \
-  p2p_passes<KIND, RR>(nt, ts, tp, total, nnb, nb_start, nb_src, nb_off, sp, CAP, red, tpts, spts, y_far, tperm, \
-                       pa, pb, out)
-  switch (r) {
-    case 4: PAM_P2P_PASSES(4); break;
-    case 5: PAM_P2P_PASSES(5); break;
-    case 6: PAM_P2P_PASSES(6); break;
-    case 7: PAM_P2P_PASSES(7); break;
-    default: PAM_P2P_PASSES(8); break;
-  }
-#undef PAM_P2P_PASSES
-}
-
 // The near fields of up to kMaxFmmJobs evaluations (same precision, kernel
 // kind and summation form) in one launch: a workgroup belongs to the last job
 // whose first_block <= its index. A single evaluation is the one-job case of
@@ -539,11 +376,289 @@ __device__ __forceinline__ const P2PJob<T>& p2p_job_of(const P2PJobs<T>& jobs, i
   return jobs.j[k];
 }
 
+// How a leaf is shared out. Parts of its targets when there are fewer than
+// kP2PBlocks leaves; where that leaves fewer than kP2PFill workgroups (four
+// rounds of the chip's 1,024), the source chunks are dealt out as well, at
+// least kP2PPartChunks to each part, and the parts' sums added by a second
+// launch. Mixed form, 220,731 sources in 512 leaves: 43,881 targets 0.349 to
+// 0.148 ms, 8,000 targets 0.170 to 0.083 ms.
+constexpr int kP2PBlocks = 4096, kP2PMaxParts = 8, kP2PFill = 4096, kP2PPartChunks = 4;
+
+// The leaf, target part and source part of a job's workgroup. Groups of 64
+// leaves: the workgroups of eight consecutive (sibling) leaves on one XCD
+// (workgroup i runs on XCD i % 8), whose L2 then holds their shared neighbours.
+template <class T>
+__device__ __forceinline__ void p2p_unit(const P2PJob<T>& j, int lb, int* leaf, int* part, int* spart) {
+  const int units = j.parts * j.sparts, per = 64 * units, grp = lb / per;
+  int u;
+  if ((grp + 1) * 64 <= j.n_leaves) {
+    const int r = lb - grp * per, q = r / 8;
+    *leaf = grp * 64 + (r & 7) * 8 + q / units;
+    u = q % units;
+  } else {
+    *leaf = lb / units;
+    u = lb % units;
+  }
+  *part = u / j.sparts;
+  *spart = u % j.sparts;
+}
+
+// The neighbour leaves of a target leaf that exist, in slot order, with their
+// offsets and the prefix sums of their point counts; built by the first wave.
+template <class T>
+struct P2PNeighbours {
+  int start[28];
+  int src[27];
+  T off[27][3];
+  int count;
+
+  // width: of a leaf, in the offsets' unit
+  __device__ void build(const P2PJob<T>& j, int leaf, T width, int lane) {
+    int a = 0, cnt = 0;
+    const int sl = lane < 27 ? j.p2p[static_cast<int64_t>(leaf) * 27 + lane] : -1;
+    if (sl >= 0) {
+      a = j.sls[sl];
+      cnt = j.sls[sl + 1] - a;
+    }
+    int incl = cnt;
+#pragma unroll
+    for (int d = 1; d < 32; d <<= 1) {
+      const int u = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += u;
+    }
+    const uint64_t have = __ballot(sl >= 0);
+    if (sl >= 0) {
+      const int k = __popcll(have & ((uint64_t{1} << lane) - 1));
+      src[k] = a;
+      start[k] = incl - cnt;
+      off[k][0] = width * static_cast<T>(lane / 9 - 1);
+      off[k][1] = width * static_cast<T>((lane / 3) % 3 - 1);
+      off[k][2] = width * static_cast<T>(lane % 3 - 1);
+    }
+    if (lane == 26) {
+      count = __popcll(have);
+      start[__popcll(have)] = incl;
+    }
+  }
+};
+
+// Output of target i (tree order): the sum plus the far field in input order,
+// or this source part's partial sum.
+template <class T>
+__device__ __forceinline__ void p2p_store(const P2PJob<T>& j, int spart, int i, double sum) {
+  if (j.sparts > 1) j.partial[static_cast<int64_t>(spart) * j.n_trg + i] = sum;
+  else j.out[j.tperm[i]] = (j.y_far ? j.y_far[i] : 0.0) + sum;
+}
+
+// The source parts of every target, in order.
+template <class T>
+__global__ void p2p_fold_kernel(P2PJobs<T> jobs) {
+  for (int k = 0; k < jobs.n; k++) {
+    const P2PJob<T>& j = jobs.j[k];
+    if (j.sparts < 2) continue;
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < j.n_trg;
+         i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+      double sum = 0.0;
+      for (int s = 0; s < j.sparts; s++) sum += j.partial[static_cast<int64_t>(s) * j.n_trg + i];
+      j.out[j.tperm[i]] = (j.y_far ? j.y_far[i] : 0.0) + sum;
+    }
+  }
+}
+
+struct Aniso3 {
+  double a[9];  // row-major A
+};
+
+// out[tperm[i]] = A^T g for a target's gradient or Hessian column g.
+__device__ __forceinline__ void p2p_store3(const Aniso3& A, double* __restrict__ o, const double (&g)[3]) {
+#pragma unroll
+  for (int k = 0; k < 3; k++) o[k] = (A.a[k] * g[0] + A.a[3 + k] * g[1]) + A.a[6 + k] * g[2];
+}
+
+template <class T>
+__global__ void p2p_fold3_kernel(P2PJob<T> j, Aniso3 A) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= j.n_trg) return;
+  double g[3] = {0.0, 0.0, 0.0};
+  for (int s = 0; s < j.sparts; s++)
+    for (int k = 0; k < 3; k++) g[k] += j.partial[(static_cast<int64_t>(s) * j.n_trg + i) * 3 + k];
+  p2p_store3(A, j.out + 3 * static_cast<int64_t>(j.tperm[i]), g);
+}
+
+template <class T>
+__device__ __forceinline__ V4<T> point_as(const V4<double>& q) {
+  return {static_cast<T>(q.x), static_cast<T>(q.y), static_cast<T>(q.z), static_cast<T>(q.w)};
+}
+
+// ---- near field on the VALU: FP64 values, gradients and Hessian columns ----
+//
+// A workgroup takes up to 16 kNearTiles targets of a leaf against the sources
+// of its 27 neighbours, or a share of them (P2PJob::parts, sparts). 256
+// sources at a time are staged in LDS with the kernel's factor in the weight,
+// the next ones in flight in registers. A thread carries R targets in
+// registers, `slots` (4, 8 or 16) lanes side by side hold different targets
+// and the 256 / slots groups of them different sources, so each source that is
+// read from LDS serves R pairs and at most `slots` target slots are idle.
+// Bound by VALU issue: per pair of an FP64 value three differences, three
+// FMAs, a root of 40 cycles and the weighted FMA, 68 cycles per 64 pairs.
+// That is 97 % of the cycles (the clock falls to 2.0 GHz over one sum and
+// further when sums follow each other). MI355X, near field alone, repeated:
+// 300k x 300k uniform points in FP64, 3.66e9 pairs, 3.77 to 3.14 ms with one
+// workgroup and a test for zero in the root before (2.0 ms when the chip
+// starts cool); 50k surface points 2.45 to 0.38 ms (0.66 with one source part);
+// 30k sources against 60k targets in clusters, exponential, 3.97 to 0.48 ms;
+// gradients in FP32, 200k x 200k, 1.12 to 0.69 ms. Eight source parts at most
+// instead of four: within 2 %.
+enum NearMode : int { kNearValue = 0, kNearGradient = 1, kNearHessian = 2 };
+constexpr int kNearMaxSparts = 4;
+template <class T, int MODE>
+constexpr int kNearTiles = MODE == kNearValue || sizeof(T) == 4 ? 8 : 5;
+
+template <class T, int KIND, int MODE, int R>
+__device__ __forceinline__ void near_pass(const P2PJob<T>& j, const P2PNeighbours<T>& nb, V4<T>* sp, int t0, int n,
+                                          int slots, int spart, const T (&col)[3], double (*red)[16 * kNearTiles<T, MODE>][4]) {
+  constexpr int kOut = MODE == kNearValue ? 1 : 3;
+  const int tid = threadIdx.x;
+  const int ti = tid & (slots - 1), si = tid / slots, splits = kThreads / slots;
+  V4<T> tq[R];
+  T acc[R][kOut];
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    const int i = r * slots + ti;
+    tq[r] = point_as<T>(i < n ? j.tpts[t0 + i] : V4<double>{0.0, 0.0, 0.0, 0.0});
+    for (int o = 0; o < kOut; o++) acc[r][o] = T(0);
+  }
+  const int nnb = nb.count, total = nb.start[nnb];
+  const int first = spart * kThreads, step = j.sparts * kThreads;
+  int k = 0;  // this thread's neighbour; its sources only move forward
+  V4<double> q{0.0, 0.0, 0.0, 0.0};
+  auto fetch = [&](int g) {
+    if (g >= total) return;
+    while (k + 1 < nnb && nb.start[k + 1] <= g) k++;
+    q = j.spts[nb.src[k] + (g - nb.start[k])];
+  };
+  fetch(first + tid);
+  const T pb = j.pb;
+  const T seed = MODE == kNearValue ? phi_seed<T, KIND>(pb) : grad_seed<T, KIND>(pb);
+  for (int cb = first; cb < total; cb += step) {
+    V4<T> s = point_as<T>(q);
+    s.x += nb.off[k][0];
+    s.y += nb.off[k][1];
+    s.z += nb.off[k][2];
+    s.w *= j.pa;
+    __syncthreads();
+    sp[tid] = s;
+    fetch(cb + step + tid);
+    __syncthreads();
+    const int cnt = min(kThreads, total - cb);
+#pragma unroll 2
+    for (int e = si; e < cnt; e += splits) {
+      const V4<T> p = sp[e];
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        const T dx = tq[r].x - p.x, dy = tq[r].y - p.y, dz = tq[r].z - p.z;
+        const T r2 = fma(dz, dz, fma(dy, dy, fma(dx, dx, seed)));
+        if constexpr (MODE == kNearValue) {
+          acc[r][0] = fma(p.w, phi_shape<T, KIND>(r2, pb), acc[r][0]);
+        } else {
+          T f, t;
+          grad_terms<T, KIND, MODE == kNearHessian>(r2, pb, &f, &t);
+          f *= p.w;
+          if constexpr (MODE == kNearGradient) {
+            acc[r][0] = fma(f, dx, acc[r][0]);
+            acc[r][1] = fma(f, dy, acc[r][1]);
+            acc[r][2] = fma(f, dz, acc[r][2]);
+          } else {
+            const T tu = t * fma(dz, col[2], fma(dy, col[1], dx * col[0]));
+            acc[r][0] = fma(f, fma(tu, dx, col[0]), acc[r][0]);
+            acc[r][1] = fma(f, fma(tu, dy, col[1]), acc[r][1]);
+            acc[r][2] = fma(f, fma(tu, dz, col[2]), acc[r][2]);
+          }
+        }
+      }
+    }
+  }
+  // The groups of a wave, then the waves, in FP64.
+#pragma unroll
+  for (int r = 0; r < R; r++)
+#pragma unroll
+    for (int o = 0; o < kOut; o++) {
+      double s = static_cast<double>(acc[r][o]);
+      for (int d = slots; d < 64; d <<= 1) s += __shfl_xor(s, d, 64);
+      if ((tid & 63) < slots) red[o][r * slots + ti][tid >> 6] = s;
+    }
+}
+
+// A workgroup's share of a job. A and the Hessian's column (column kcol of A)
+// are read for the modes that have three outputs.
+template <class T, int KIND, int MODE>
+__device__ __forceinline__ void near_leaf(const P2PJob<T>& j, int unit, const Aniso3& A, int kcol) {
+  constexpr int kOut = MODE == kNearValue ? 1 : 3, kTiles = kNearTiles<T, MODE>;
+  __shared__ V4<T> sp[kThreads];
+  __shared__ P2PNeighbours<T> nb;
+  __shared__ double red[kOut][16 * kTiles][4];
+  int leaf, part, spart;
+  p2p_unit(j, unit, &leaf, &part, &spart);
+  const int ts = j.tls[leaf], te = j.tls[leaf + 1];
+  const int parts = min(j.parts, (te - ts + 16 * kTiles - 1) / (16 * kTiles));
+  if (part >= parts) return;
+  const int p0 = ts + static_cast<int>(static_cast<int64_t>(te - ts) * part / parts);
+  const int p1 = ts + static_cast<int>(static_cast<int64_t>(te - ts) * (part + 1) / parts);
+  if (threadIdx.x < 64) nb.build(j, leaf, T(2), threadIdx.x);
+  T col[3] = {T(0), T(0), T(0)};
+  if constexpr (MODE == kNearHessian)
+    for (int k = 0; k < 3; k++) col[k] = static_cast<T>(A.a[3 * k + kcol]);
+  __syncthreads();
+  const int npass = (p1 - p0 + 16 * kTiles - 1) / (16 * kTiles);
+  for (int ps = 0; ps < npass; ps++) {
+    const int t0 = p0 + (p1 - p0) * ps / npass, n = p0 + (p1 - p0) * (ps + 1) / npass - t0;
+    int slots = 16;
+    while (slots > 4 && 2 * n <= kTiles * slots) slots /= 2;
+#define PAM_NEAR_PASS(RR)                                                                    \
+  case RR:                                                                                   \
+    if constexpr (RR <= kTiles) near_pass<T, KIND, MODE, RR>(j, nb, sp, t0, n, slots, spart, col, red); \
+    break
+    switch ((n + slots - 1) / slots) {
+      PAM_NEAR_PASS(1);
+      PAM_NEAR_PASS(2);
+      PAM_NEAR_PASS(3);
+      PAM_NEAR_PASS(4);
+      PAM_NEAR_PASS(5);
+      PAM_NEAR_PASS(6);
+      PAM_NEAR_PASS(7);
+      PAM_NEAR_PASS(8);
+      default: break;
+    }
+#undef PAM_NEAR_PASS
+    __syncthreads();
+    for (int e = threadIdx.x; e < n; e += kThreads) {
+      double g[kOut];
+      for (int o = 0; o < kOut; o++) g[o] = ((red[o][e][0] + red[o][e][1]) + red[o][e][2]) + red[o][e][3];
+      if constexpr (MODE == kNearValue) {
+        p2p_store(j, spart, t0 + e, g[0]);
+      } else if (j.sparts > 1) {
+        for (int o = 0; o < 3; o++) j.partial[(static_cast<int64_t>(spart) * j.n_trg + t0 + e) * 3 + o] = g[o];
+      } else {
+        p2p_store3(A, j.out + 3 * static_cast<int64_t>(j.tperm[t0 + e]), g);
+      }
+    }
+    __syncthreads();  // red is written again in the next pass
+  }
+}
+
 template <int KIND>
-__global__ void __launch_bounds__(kThreads) p2p_jobs_kernel(P2PJobs<double> jobs) {
-  const int g = blockIdx.x;
-  const P2PJob<double>& j = p2p_job_of(jobs, g);
-  p2p_leaf<KIND>(g - j.first_block, j.tls, j.sls, j.p2p, j.tpts, j.spts, j.y_far, j.tperm, j.pa, j.pb, j.out);
+__global__ void __launch_bounds__(kThreads, 3) p2p_jobs_kernel(P2PJobs<double> jobs) {
+  const P2PJob<double>& j = p2p_job_of(jobs, static_cast<int>(blockIdx.x));
+  near_leaf<double, KIND, kNearValue>(j, static_cast<int>(blockIdx.x) - j.first_block, Aniso3{}, 0);
+}
+
+// Gradients (gradient-transpose kernel, fmm/gradient_transpose_kernel.hpp:47-62:
+// out_i = A^T sum_j w_j grad phi(A (t_i - s_j))) and one column of the Hessian
+// (fmm/hessian_kernel.hpp:46-64, applied to one weight component:
+// out_i = A^T sum_j w_j H(A (t_i - s_j)) a_k, a_k the k-th column of A).
+template <class T, int KIND, int MODE>
+__global__ void __launch_bounds__(kThreads, 3) p2p_vector_kernel(P2PJob<T> j, Aniso3 A, int kcol) {
+  near_leaf<T, KIND, MODE>(j, static_cast<int>(blockIdx.x), A, kcol);
 }
 
 // ---- near field of the mixed form: squared distances on the FP16 matrix unit ----
@@ -576,15 +691,9 @@ __global__ void __launch_bounds__(kThreads) p2p_jobs_kernel(P2PJobs<double> jobs
 constexpr int kMfSrc = kThreads;  // sources staged per chunk: one per thread
 constexpr int kMfMaxTiles = 5;  // 16-target tiles per wave and pass
 constexpr double kMfUnit = 0x1p-9;
-// Workgroups wanted in a launch of one evaluation: a leaf's tiles are shared
-// out to several workgroups when there are fewer leaves, kMfPartTiles at least
-// to each (every one of them stages the leaf's sources for itself).
-constexpr int kMfBlocks = 4096, kMfMaxParts = 8, kMfPartTiles = 4;
-// Where that leaves fewer than kMfFill workgroups (four rounds of the chip's
-// 1,024), the source chunks are dealt out as well, kMfPartChunks at least to
-// each part, and the parts' sums added by a second launch. 220,731 sources in
-// 512 leaves: 43,881 targets 0.349 to 0.148 ms, 8,000 targets 0.170 to 0.083 ms.
-constexpr int kMfFill = 4096, kMfMaxSparts = 3, kMfPartChunks = 4;
+// Target tiles per part at least (every part stages the leaf's sources for
+// itself), and source parts at most.
+constexpr int kMfPartTiles = 4, kMfMaxSparts = 3;
 
 using h16x4 = _Float16 __attribute__((ext_vector_type(4)));
 using f32x4v = float __attribute__((ext_vector_type(4)));
@@ -717,56 +826,11 @@ __device__ __forceinline__ void mf_tiles(const h16x4* sa, const f32x4v* sw, int 
   }
 }
 
-// The leaf, target part and source part of a job's workgroup. Groups of 64
-// leaves: the workgroups of eight consecutive (sibling) leaves on one XCD
-// (workgroup i runs on XCD i % 8), whose L2 then holds their shared neighbours.
-template <class T>
-__device__ __forceinline__ void p2p_unit(const P2PJob<T>& j, int lb, int* leaf, int* part, int* spart) {
-  const int units = j.parts * j.sparts, per = 64 * units, grp = lb / per;
-  int u;
-  if ((grp + 1) * 64 <= j.n_leaves) {
-    const int r = lb - grp * per, q = r / 8;
-    *leaf = grp * 64 + (r & 7) * 8 + q / units;
-    u = q % units;
-  } else {
-    *leaf = lb / units;
-    u = lb % units;
-  }
-  *part = u / j.sparts;
-  *spart = u % j.sparts;
-}
-
-// Output of target i (tree order): the sum plus the far field in input order,
-// or this source part's partial sum.
-template <class T>
-__device__ __forceinline__ void p2p_store(const P2PJob<T>& j, int spart, int i, double sum) {
-  if (j.sparts > 1) j.partial[static_cast<int64_t>(spart) * j.n_trg + i] = sum;
-  else j.out[j.tperm[i]] = (j.y_far ? j.y_far[i] : 0.0) + sum;
-}
-
-// The source parts of every target, in order.
-template <class T>
-__global__ void p2p_fold_kernel(P2PJobs<T> jobs) {
-  for (int k = 0; k < jobs.n; k++) {
-    const P2PJob<T>& j = jobs.j[k];
-    if (j.sparts < 2) continue;
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < j.n_trg;
-         i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-      double sum = 0.0;
-      for (int s = 0; s < j.sparts; s++) sum += j.partial[static_cast<int64_t>(s) * j.n_trg + i];
-      j.out[j.tperm[i]] = (j.y_far ? j.y_far[i] : 0.0) + sum;
-    }
-  }
-}
-
 template <int KIND, bool kComp>
 __global__ void __launch_bounds__(kThreads, 4) p2p_mf_jobs_kernel(P2PJobs<float> jobs) {
   __shared__ h16x4 sa[kMfSrc / 16 * 192];  // [16-source block][product][reduction index / 4][row]
   __shared__ f32x4v sw[kMfSrc / 4];        // [block][row]: weights
-  __shared__ int nb_start[28];
-  __shared__ int nb_src[27];
-  __shared__ float nb_off[27][3];  // in units
-  __shared__ int nb_count;
+  __shared__ P2PNeighbours<float> nb;  // offsets in units
   __shared__ double red[4][kMfMaxTiles * 16];
   const P2PJob<float>& j = p2p_job_of(jobs, static_cast<int>(blockIdx.x));
   int leaf, part, spart;
@@ -778,38 +842,9 @@ __global__ void __launch_bounds__(kThreads, 4) p2p_mf_jobs_kernel(P2PJobs<float>
   const int tile0 = tiles * part / parts, tile1 = tiles * (part + 1) / parts;
   if (tile0 == tile1) return;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  if (wave == 0) {
-    // The neighbour leaves that exist, in slot order, with their offsets and
-    // the prefix sums of their point counts.
-    int a = 0, cnt = 0;
-    const int sl = lane < 27 ? j.p2p[static_cast<int64_t>(leaf) * 27 + lane] : -1;
-    if (sl >= 0) {
-      a = j.sls[sl];
-      cnt = j.sls[sl + 1] - a;
-    }
-    int incl = cnt;
-#pragma unroll
-    for (int d = 1; d < 32; d <<= 1) {
-      const int u = __shfl_up(incl, d, 64);
-      if (lane >= d) incl += u;
-    }
-    const uint64_t have = __ballot(sl >= 0);
-    if (sl >= 0) {
-      const int k = __popcll(have & ((uint64_t{1} << lane) - 1));
-      nb_src[k] = a;
-      nb_start[k] = incl - cnt;
-      constexpr int kLeaf = static_cast<int>(2.0 / kMfUnit);
-      nb_off[k][0] = static_cast<float>(kLeaf * (lane / 9 - 1));
-      nb_off[k][1] = static_cast<float>(kLeaf * ((lane / 3) % 3 - 1));
-      nb_off[k][2] = static_cast<float>(kLeaf * (lane % 3 - 1));
-    }
-    if (lane == 26) {
-      nb_count = __popcll(have);
-      nb_start[__popcll(have)] = incl;
-    }
-  }
+  if (wave == 0) nb.build(j, leaf, static_cast<float>(2.0 / kMfUnit), lane);
   __syncthreads();
-  const int nnb = nb_count, total = nb_start[nnb];
+  const int nnb = nb.count, total = nb.start[nnb];
   // This source part's chunks: every sparts-th one.
   const int first = spart * kMfSrc, step = j.sparts * kMfSrc;
   const float pa = j.pa, pb = j.pb;
@@ -849,16 +884,16 @@ __global__ void __launch_bounds__(kThreads, 4) p2p_mf_jobs_kernel(P2PJobs<float>
     auto fetch = [&](int g) {
       q = {0.0, 0.0, 0.0, 0.0};
       if (g >= total) return;
-      while (k + 1 < nnb && nb_start[k + 1] <= g) k++;
-      q = j.spts[nb_src[k] + (g - nb_start[k])];
+      while (k + 1 < nnb && nb.start[k + 1] <= g) k++;
+      q = j.spts[nb.src[k] + (g - nb.start[k])];
     };
     fetch(first + tid);
     for (int cb = first; cb < total; cb += step) {
       const int nblk = (min(kMfSrc, total - cb) + 15) / 16;
       MfCoord x = mf_split(q.x), y = mf_split(q.y), z = mf_split(q.z);
-      x.i += nb_off[k][0];  // exact: an integer number of units
-      y.i += nb_off[k][1];
-      z.i += nb_off[k][2];
+      x.i += nb.off[k][0];  // exact: an integer number of units
+      y.i += nb.off[k][1];
+      z.i += nb.off[k][2];
       const MfSelf s = mf_self(x, y, z);
       const float c = 0x1p-12f;
       __syncthreads();
@@ -906,7 +941,7 @@ __global__ void __launch_bounds__(kThreads, 4) p2p_mf_jobs_kernel(P2PJobs<float>
   }
 }
 
-// ---- gradients at the targets (gradient-transpose kernel,
+// ---- far field of the gradients at the targets (gradient-transpose kernel,
 // fmm/gradient_transpose_kernel.hpp:47-62): out_i = A^T sum_j w_j grad phi(A (t_i - s_j)) ----
 
 // Lagrange basis and its derivative at the Chebyshev nodes:
@@ -942,15 +977,6 @@ __device__ __forceinline__ void lagrange_d_lds(T xi, const T* __restrict__ tk, T
     s[a][col] = c0 + c1 * sum;
     d[a][col] = c1 * sd;
   }
-}
-
-struct Aniso3 {
-  double a[9];  // row-major A
-};
-
-template <class T>
-__device__ __forceinline__ V4<T> point_as(const V4<double>& q) {
-  return {static_cast<T>(q.x), static_cast<T>(q.y), static_cast<T>(q.z), static_cast<T>(q.w)};
 }
 
 constexpr int kL2PGThreads = 128;
@@ -1015,118 +1041,7 @@ l2p_grad_kernel(const int32_t* __restrict__ leaf_start, const V4<double>* __rest
   }
 }
 
-// Near-field gradient: the layout of p2p_kernel with three sums per target;
-// writes A^T (sum over the 27 neighbour leaves) to the output in input order.
-template <class T, int KIND>
-__global__ void __launch_bounds__(kThreads)
-p2p_grad_kernel(const int32_t* __restrict__ tls, const int32_t* __restrict__ sls,
-                const int32_t* __restrict__ p2p, const V4<double>* __restrict__ tpts,
-                const V4<double>* __restrict__ spts, const int32_t* __restrict__ tperm, T ag, T pb, Aniso3 A,
-                double* __restrict__ out) {
-  constexpr int CAP = 32768 / static_cast<int>(sizeof(V4<T>));
-  constexpr int R = 2;
-  __shared__ V4<T> sp[CAP];
-  __shared__ int nb_start[28];
-  __shared__ int nb_src[27];
-  __shared__ T nb_off[27][3];
-  __shared__ int nb_count;
-  __shared__ T red[R][3][kThreads];
-  const int leaf = blockIdx.x;
-  const int ts = tls[leaf], te = tls[leaf + 1];
-  const int nt = te - ts;
-  if (threadIdx.x == 0) {
-    int k = 0, total = 0;
-    for (int s = 0; s < 27; s++) {
-      int sl = p2p[static_cast<int64_t>(leaf) * 27 + s];
-      if (sl < 0) continue;
-      int a = sls[sl], b = sls[sl + 1];
-      nb_src[k] = a;
-      nb_start[k] = total;
-      nb_off[k][0] = T(2 * (s / 9 - 1));
-      nb_off[k][1] = T(2 * ((s / 3) % 3 - 1));
-      nb_off[k][2] = T(2 * (s % 3 - 1));
-      total += b - a;
-      k++;
-    }
-    nb_start[k] = total;
-    nb_count = k;
-  }
-  __syncthreads();
-  const int nnb = nb_count;
-  const int total = nb_start[nnb];
-  const int per = (nt + R - 1) / R;
-  int tp = 1;
-  while (tp < per && tp < kThreads) tp <<= 1;
-  const int nsplit = kThreads / tp;
-  const int ti = threadIdx.x & (tp - 1);
-  const int si = threadIdx.x / tp;
-  const T seed = phi_seed<T, KIND>(pb);
-  for (int c0 = 0; c0 < nt; c0 += R * tp) {
-    V4<T> tq[R];
-    T ax[R], ay[R], az[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-      const int i = c0 + r * tp + ti;
-      tq[r] = i < nt ? point_as<T>(tpts[ts + i]) : V4<T>{T(0), T(0), T(0), T(0)};
-      ax[r] = ay[r] = az[r] = T(0);
-    }
-    for (int cb = 0; cb < total; cb += CAP) {
-      const int cnt = min(CAP, total - cb);
-      __syncthreads();
-      for (int e = threadIdx.x; e < cnt; e += kThreads) {
-        int g = cb + e;
-        int k = 0;
-        while (k + 1 < nnb && nb_start[k + 1] <= g) k++;
-        V4<T> q = point_as<T>(spts[nb_src[k] + (g - nb_start[k])]);
-        q.x += nb_off[k][0];
-        q.y += nb_off[k][1];
-        q.z += nb_off[k][2];
-        q.w *= ag;  // the gradient's factor folded into the weight
-        sp[e] = q;
-      }
-      __syncthreads();
-      for (int j = si; j < cnt; j += nsplit) {
-        const V4<T> q = sp[j];
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-          const T dx = tq[r].x - q.x, dy = tq[r].y - q.y, dz = tq[r].z - q.z;
-          const T r2 = fma(dz, dz, fma(dy, dy, fma(dx, dx, seed)));
-          const T f = q.w * grad_shape<T, KIND>(r2, pb);
-          ax[r] = fma(f, dx, ax[r]);
-          ay[r] = fma(f, dy, ay[r]);
-          az[r] = fma(f, dz, az[r]);
-        }
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-      red[r][0][threadIdx.x] = ax[r];
-      red[r][1][threadIdx.x] = ay[r];
-      red[r][2][threadIdx.x] = az[r];
-    }
-    __syncthreads();
-    if (si == 0) {
-#pragma unroll
-      for (int r = 0; r < R; r++) {
-        const int i = c0 + r * tp + ti;
-        if (i >= nt) continue;
-        double g[3];
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-          T sum = T(0);
-          for (int m = 0; m < nsplit; m++) sum += red[r][k][ti + m * tp];
-          g[k] = static_cast<double>(sum);
-        }
-        double* o = out + 3 * static_cast<int64_t>(tperm[ts + i]);
-#pragma unroll
-        for (int k = 0; k < 3; k++) o[k] = (A.a[k] * g[0] + A.a[3 + k] * g[1]) + A.a[6 + k] * g[2];
-      }
-    }
-    __syncthreads();
-  }
-}
-
-// ---- one column of the Hessian at the targets (the Hessian kernel,
+// ---- far field of one column of the Hessian at the targets (the Hessian kernel,
 // fmm/hessian_kernel.hpp:46-64, applied to one weight component):
 // out_i = A^T sum_j w_j H(A (t_i - s_j)) a_k, a_k the k-th column of A ----
 
@@ -1227,117 +1142,6 @@ l2p_hess_col_kernel(const int32_t* __restrict__ leaf_start, const V4<double>* __
     double* o = out + 3 * static_cast<int64_t>(perm[i]);
 #pragma unroll
     for (int k = 0; k < 3; k++) o[k] += (A.a[k] * v[0] + A.a[3 + k] * v[1]) + A.a[6 + k] * v[2];
-  }
-}
-
-template <class T, int KIND>
-__global__ void __launch_bounds__(kThreads)
-p2p_hess_col_kernel(const int32_t* __restrict__ tls, const int32_t* __restrict__ sls,
-                    const int32_t* __restrict__ p2p, const V4<double>* __restrict__ tpts,
-                    const V4<double>* __restrict__ spts, const int32_t* __restrict__ tperm, T hc, T pb, Aniso3 A,
-                    int kcol, double* __restrict__ out) {
-  constexpr int CAP = 32768 / static_cast<int>(sizeof(V4<T>));
-  constexpr int R = 2;
-  __shared__ V4<T> sp[CAP];
-  __shared__ int nb_start[28];
-  __shared__ int nb_src[27];
-  __shared__ T nb_off[27][3];
-  __shared__ int nb_count;
-  __shared__ T red[R][3][kThreads];
-  const int leaf = blockIdx.x;
-  const int ts = tls[leaf], te = tls[leaf + 1];
-  const int nt = te - ts;
-  if (threadIdx.x == 0) {
-    int k = 0, total = 0;
-    for (int s = 0; s < 27; s++) {
-      int sl = p2p[static_cast<int64_t>(leaf) * 27 + s];
-      if (sl < 0) continue;
-      int a = sls[sl], b = sls[sl + 1];
-      nb_src[k] = a;
-      nb_start[k] = total;
-      nb_off[k][0] = T(2 * (s / 9 - 1));
-      nb_off[k][1] = T(2 * ((s / 3) % 3 - 1));
-      nb_off[k][2] = T(2 * (s % 3 - 1));
-      total += b - a;
-      k++;
-    }
-    nb_start[k] = total;
-    nb_count = k;
-  }
-  __syncthreads();
-  const int nnb = nb_count;
-  const int total = nb_start[nnb];
-  const int per = (nt + R - 1) / R;
-  int tp = 1;
-  while (tp < per && tp < kThreads) tp <<= 1;
-  const int nsplit = kThreads / tp;
-  const int ti = threadIdx.x & (tp - 1);
-  const int si = threadIdx.x / tp;
-  const T seed = phi_seed<T, KIND>(pb);
-  const T ak0 = static_cast<T>(A.a[kcol]), ak1 = static_cast<T>(A.a[3 + kcol]), ak2 = static_cast<T>(A.a[6 + kcol]);
-  for (int c0 = 0; c0 < nt; c0 += R * tp) {
-    V4<T> tq[R];
-    T ax[R], ay[R], az[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-      const int i = c0 + r * tp + ti;
-      tq[r] = i < nt ? point_as<T>(tpts[ts + i]) : V4<T>{T(0), T(0), T(0), T(0)};
-      ax[r] = ay[r] = az[r] = T(0);
-    }
-    for (int cb = 0; cb < total; cb += CAP) {
-      const int cnt = min(CAP, total - cb);
-      __syncthreads();
-      for (int e = threadIdx.x; e < cnt; e += kThreads) {
-        int g = cb + e;
-        int k = 0;
-        while (k + 1 < nnb && nb_start[k + 1] <= g) k++;
-        V4<T> q = point_as<T>(spts[nb_src[k] + (g - nb_start[k])]);
-        q.x += nb_off[k][0];
-        q.y += nb_off[k][1];
-        q.z += nb_off[k][2];
-        q.w *= hc;
-        sp[e] = q;
-      }
-      __syncthreads();
-      for (int j = si; j < cnt; j += nsplit) {
-        const V4<T> q = sp[j];
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-          const T dx = tq[r].x - q.x, dy = tq[r].y - q.y, dz = tq[r].z - q.z;
-          const T r2 = fma(dz, dz, fma(dy, dy, fma(dx, dx, seed)));
-          const T f = q.w * grad_shape<T, KIND>(r2, pb);
-          const T tu = hess_t<T, KIND>(r2, pb) * fma(dz, ak2, fma(dy, ak1, dx * ak0));
-          ax[r] = fma(f, fma(tu, dx, ak0), ax[r]);
-          ay[r] = fma(f, fma(tu, dy, ak1), ay[r]);
-          az[r] = fma(f, fma(tu, dz, ak2), az[r]);
-        }
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-      red[r][0][threadIdx.x] = ax[r];
-      red[r][1][threadIdx.x] = ay[r];
-      red[r][2][threadIdx.x] = az[r];
-    }
-    __syncthreads();
-    if (si == 0) {
-#pragma unroll
-      for (int r = 0; r < R; r++) {
-        const int i = c0 + r * tp + ti;
-        if (i >= nt) continue;
-        double g[3];
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-          T sum = T(0);
-          for (int m = 0; m < nsplit; m++) sum += red[r][k][ti + m * tp];
-          g[k] = static_cast<double>(sum);
-        }
-        double* o = out + 3 * static_cast<int64_t>(tperm[ts + i]);
-#pragma unroll
-        for (int k = 0; k < 3; k++) o[k] = (A.a[k] * g[0] + A.a[3 + k] * g[1]) + A.a[6 + k] * g[2];
-      }
-    }
-    __syncthreads();
   }
 }
 
@@ -2326,40 +2130,81 @@ L2PJob<T> make_l2p_job(const Tree& t, const T* l_leaf, const V4<T>* pts, T* y_fa
   return j;
 }
 
+// Shares a job's leaves out: parts, sparts, and where the source parts' sums
+// of `outs` numbers per target go.
 template <class T>
-P2PJob<T> make_p2p_job(const RbfDesc& rbf, const Tree& trg, const Tree& src, const Lists& lists,
-                       const V4<double>* tpts, const V4<double>* spts, const double* y_far, double* out,
-                       DevBuf<double>& partial) {
+void p2p_split(P2PJob<T>& j, int64_t n_src, int64_t src_leaves, int part_targets, int most_parts, int most_sparts,
+               int outs, DevBuf<double>& partial) {
+  j.parts = j.sparts = 1;
+  if (j.n_leaves == 0) return;
+  j.parts = std::clamp((kP2PBlocks + j.n_leaves - 1) / j.n_leaves, 1, most_parts);
+  // averages over the leaves
+  const double blocks = j.n_leaves * std::clamp(static_cast<double>(j.n_trg) / j.n_leaves / part_targets, 1.0,
+                                                static_cast<double>(j.parts));
+  const double chunks = 27.0 * static_cast<double>(n_src) / static_cast<double>(std::max<int64_t>(src_leaves, 1)) / kThreads;
+  j.sparts = std::clamp(static_cast<int>(std::min(kP2PFill / blocks, chunks / kP2PPartChunks)), 1, most_sparts);
+  if (j.sparts > 1) {
+    partial.resize(static_cast<size_t>(j.sparts) * j.n_trg * outs);
+    j.partial = partial.get();
+  }
+}
+
+template <class T>
+P2PJob<T> p2p_job_base(const Tree& trg, const Tree& src, const Lists& lists, const V4<double>* tpts,
+                       const V4<double>* spts, double* out) {
   P2PJob<T> j{};
-  const double h = trg.box.width / std::ldexp(1.0, trg.level) / 2.0;
-  // The mixed form's kernel works in units of kMfUnit of the leaf half width.
-  const PhiConsts pc = phi_consts(rbf, sizeof(T) == 4 ? h * kMfUnit : h);
   j.tls = trg.leaf_start.get();
   j.sls = src.leaf_start.get();
   j.p2p = lists.p2p.get();
   j.tpts = tpts;
   j.spts = spts;
-  j.y_far = y_far;
   j.tperm = trg.perm.get();
-  j.pa = static_cast<T>(pc.a);
-  j.pb = static_cast<T>(phi_shape_const<T>(rbf.kind, pc.b));
   j.out = out;
   j.n_leaves = static_cast<int>(trg.n_leaves());
   j.n_trg = trg.n_points;
-  j.parts = j.sparts = 1;
-  if (sizeof(T) == 4 && j.n_leaves > 0) {
-    j.parts = std::clamp((kMfBlocks + j.n_leaves - 1) / j.n_leaves, 1, kMfMaxParts);
-    // averages over the leaves
-    const double tiles = static_cast<double>(j.n_trg) / j.n_leaves / 16;
-    const double blocks = j.n_leaves * std::clamp(tiles / kMfPartTiles, 1.0, static_cast<double>(j.parts));
-    const double chunks = 27.0 * static_cast<double>(src.n_points) / static_cast<double>(std::max<int64_t>(src.n_leaves(), 1)) / kMfSrc;
-    j.sparts = std::clamp(static_cast<int>(std::min(kMfFill / blocks, chunks / kMfPartChunks)), 1, kMfMaxSparts);
-    if (j.sparts > 1) {
-      partial.resize(static_cast<size_t>(j.sparts) * j.n_trg);
-      j.partial = partial.get();
-    }
-  }
   return j;
+}
+
+template <class T>
+P2PJob<T> make_p2p_job(const RbfDesc& rbf, const Tree& trg, const Tree& src, const Lists& lists,
+                       const V4<double>* tpts, const V4<double>* spts, const double* y_far, double* out,
+                       DevBuf<double>& partial) {
+  P2PJob<T> j = p2p_job_base<T>(trg, src, lists, tpts, spts, out);
+  const double h = trg.box.width / std::ldexp(1.0, trg.level) / 2.0;
+  // The mixed form's kernel works in units of kMfUnit of the leaf half width.
+  const PhiConsts pc = phi_consts(rbf, sizeof(T) == 4 ? h * kMfUnit : h);
+  j.y_far = y_far;
+  j.pa = static_cast<T>(pc.a);
+  j.pb = static_cast<T>(phi_shape_const<T>(rbf.kind, pc.b));
+  if constexpr (sizeof(T) == 4) p2p_split(j, src.n_points, src.n_leaves(), 16 * kMfPartTiles, kP2PMaxParts, kMfMaxSparts, 1, partial);
+  else p2p_split(j, src.n_points, src.n_leaves(), 16 * kNearTiles<T, kNearValue>, kP2PMaxParts, kNearMaxSparts, 1, partial);
+  return j;
+}
+
+// Gradients (MODE kNearGradient) or Hessian column kcol at the targets.
+template <class T, int MODE>
+void launch_p2p_vector(const RbfDesc& rbf, const Tree& trg, const Tree& src, const Lists& lists,
+                       const V4<double>* tpts, const V4<double>* spts, int kcol, double* out3,
+                       DevBuf<double>& partial, hipStream_t s) {
+  if (trg.n_leaves() == 0) return;
+  const double h = trg.box.width / std::ldexp(1.0, trg.level) / 2.0;
+  const PhiConsts gc = grad_consts(rbf, h);
+  Aniso3 A;
+  for (int k = 0; k < 9; k++) A.a[k] = rbf.aniso[k];
+  P2PJob<T> j = p2p_job_base<T>(trg, src, lists, tpts, spts, out3);
+  j.pa = static_cast<T>(MODE == kNearHessian ? gc.a / h : gc.a);
+  j.pb = static_cast<T>(gc.b);
+  p2p_split(j, src.n_points, src.n_leaves(), 16 * kNearTiles<T, MODE>, kP2PMaxParts, kNearMaxSparts, 3, partial);
+  const int64_t blocks = static_cast<int64_t>(j.n_leaves) * j.parts * j.sparts;
+  if (blocks > INT32_MAX) throw_runtime("near field: too many leaves");
+  dispatch_kind(rbf.kind, [&](auto K) {
+    p2p_vector_kernel<T, decltype(K)::value, MODE><<<static_cast<unsigned>(blocks), kThreads, 0, s>>>(j, A, kcol);
+  });
+  PAM_LAUNCH_CHECK();
+  if (j.sparts > 1) {
+    p2p_fold3_kernel<T><<<ceil_div(j.n_trg, kThreads), kThreads, 0, s>>>(j, A);
+    PAM_LAUNCH_CHECK();
+  }
 }
 
 template <class T>
@@ -2493,37 +2338,17 @@ void launch_l2p_hess_col(int p, const Tree& t, const double* l_leaf, const V4<do
 
 template <class T>
 void launch_p2p_hess_col(const RbfDesc& rbf, const Tree& trg, const Tree& src, const Lists& lists,
-                         const V4<double>* tpts, const V4<double>* spts, int kcol, double* out3, hipStream_t s) {
-  int64_t nl = trg.n_leaves();
-  if (nl == 0) return;
-  if (kcol < 0 || kcol > 2) throw_invalid("Hessian column out of range");
-  const double h = trg.box.width / std::ldexp(1.0, trg.level) / 2.0;
-  const PhiConsts gc = grad_consts(rbf, h);
-  Aniso3 A;
-  for (int k = 0; k < 9; k++) A.a[k] = rbf.aniso[k];
-  dispatch_kind(rbf.kind, [&](auto K) {
-    p2p_hess_col_kernel<T, decltype(K)::value><<<static_cast<unsigned>(nl), kThreads, 0, s>>>(
-        trg.leaf_start.get(), src.leaf_start.get(), lists.p2p.get(), tpts, spts, trg.perm.get(),
-        static_cast<T>(gc.a / h), static_cast<T>(gc.b), A, kcol, out3);
-  });
-  PAM_LAUNCH_CHECK();
+                         const V4<double>* tpts, const V4<double>* spts, int kcol, double* out3,
+                         DevBuf<double>& partial, hipStream_t s) {
+  if (trg.n_leaves() > 0 && (kcol < 0 || kcol > 2)) throw_invalid("Hessian column out of range");
+  launch_p2p_vector<T, kNearHessian>(rbf, trg, src, lists, tpts, spts, kcol, out3, partial, s);
 }
 
 template <class T>
 void launch_p2p_grad(const RbfDesc& rbf, const Tree& trg, const Tree& src, const Lists& lists,
-                     const V4<double>* tpts, const V4<double>* spts, double* out3, hipStream_t s) {
-  int64_t nl = trg.n_leaves();
-  if (nl == 0) return;
-  const double h = trg.box.width / std::ldexp(1.0, trg.level) / 2.0;
-  const PhiConsts gc = grad_consts(rbf, h);
-  Aniso3 A;
-  for (int k = 0; k < 9; k++) A.a[k] = rbf.aniso[k];
-  dispatch_kind(rbf.kind, [&](auto K) {
-    p2p_grad_kernel<T, decltype(K)::value><<<static_cast<unsigned>(nl), kThreads, 0, s>>>(
-        trg.leaf_start.get(), src.leaf_start.get(), lists.p2p.get(), tpts, spts, trg.perm.get(),
-        static_cast<T>(gc.a), static_cast<T>(gc.b), A, out3);
-  });
-  PAM_LAUNCH_CHECK();
+                     const V4<double>* tpts, const V4<double>* spts, double* out3, DevBuf<double>& partial,
+                     hipStream_t s) {
+  launch_p2p_vector<T, kNearGradient>(rbf, trg, src, lists, tpts, spts, 0, out3, partial, s);
 }
 
 template <class T>
@@ -2587,9 +2412,9 @@ void launch_m2l_batch(const M2LOperator& op, const std::vector<M2LLevelSpec<TM, 
   template void launch_p2p<T>(const RbfDesc&, const Tree&, const Tree&, const Lists&, const V4<double>*, \
                               const V4<double>*, const double*, double*, DevBuf<double>&, hipStream_t, bool);   \
   template void launch_p2p_grad<T>(const RbfDesc&, const Tree&, const Tree&, const Lists&, const V4<double>*, \
-                                   const V4<double>*, double*, hipStream_t);                                  \
+                                   const V4<double>*, double*, DevBuf<double>&, hipStream_t);                 \
   template void launch_p2p_hess_col<T>(const RbfDesc&, const Tree&, const Tree&, const Lists&, const V4<double>*, \
-                                       const V4<double>*, int, double*, hipStream_t);                           \
+                                       const V4<double>*, int, double*, DevBuf<double>&, hipStream_t);          \
   template void build_m2l_dense<T>(int, const RbfDesc&, double, M2LOperator&, DevBuf<T>&,          \
                                    hipStream_t);                                                    \
   template void launch_m2l_batch<T, double>(const M2LOperator&,                                        \

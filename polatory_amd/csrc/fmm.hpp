@@ -67,7 +67,7 @@ struct P2PJob {
   const int32_t* tperm;  // tree order -> input order of the targets
   double* out;           // output, input order
   T pa, pb;              // kernel constants in the leaf unit (phi_shape_const)
-  double* partial;       // [sparts][n_trg] sums of the source parts, tree order (sparts > 1)
+  double* partial;       // [sparts][n_trg][outputs] sums of the source parts, tree order (sparts > 1)
   int64_t n_trg;
   int n_leaves, parts, sparts, first_block;  // parts x sparts workgroups per leaf: target tiles x sources
 };
@@ -127,7 +127,8 @@ void launch_p2p(const RbfDesc& rbf, const Tree& trg, const Tree& src, const List
 // the far field then adds A^T grad of the leaf local expansions.
 template <class T>
 void launch_p2p_grad(const RbfDesc& rbf, const Tree& trg, const Tree& src, const Lists& lists,
-                     const V4<double>* tpts, const V4<double>* spts, double* out3, hipStream_t s);
+                     const V4<double>* tpts, const V4<double>* spts, double* out3, DevBuf<double>& partial,
+                     hipStream_t s);
 void launch_l2p_grad(int p, const Tree& t, const double* l_leaf, const V4<double>* pts, const double* aniso,
                      double* out3, hipStream_t s);
 // Column kcol of the Hessian kernel at the targets (fmm/hessian_kernel.hpp:46-64
@@ -135,7 +136,8 @@ void launch_l2p_grad(int p, const Tree& t, const double* l_leaf, const V4<double
 // near field writes, the far field adds.
 template <class T>
 void launch_p2p_hess_col(const RbfDesc& rbf, const Tree& trg, const Tree& src, const Lists& lists,
-                         const V4<double>* tpts, const V4<double>* spts, int kcol, double* out3, hipStream_t s);
+                         const V4<double>* tpts, const V4<double>* spts, int kcol, double* out3,
+                         DevBuf<double>& partial, hipStream_t s);
 void launch_l2p_hess_col(int p, const Tree& t, const double* l_leaf, const V4<double>* pts, const double* aniso,
                          int kcol, double* out3, hipStream_t s);
 

@@ -674,8 +674,8 @@ void FmmEvaluator::run_fmm(double* d_out) {
     PAM_HIP(hipEventRecord(fork_ev_, stream_));
     PAM_HIP(hipStreamWaitEvent(ps, fork_ev_, 0));
     record(7, ps);
-    if (hess_col_ >= 0) launch_p2p_hess_col<TP>(rbf_, tt, stree, lists_, tpts, spts, hess_col_, d_out, ps);
-    else if (grad_) launch_p2p_grad<TP>(rbf_, tt, stree, lists_, tpts, spts, d_out, ps);
+    if (hess_col_ >= 0) launch_p2p_hess_col<TP>(rbf_, tt, stree, lists_, tpts, spts, hess_col_, d_out, st.p2p_partial, ps);
+    else if (grad_) launch_p2p_grad<TP>(rbf_, tt, stree, lists_, tpts, spts, d_out, st.p2p_partial, ps);
     else launch_p2p<TP>(rbf_, tt, stree, lists_, tpts, spts, nullptr, d_out, st.p2p_partial, ps, cfg_.precision == kMixedComp);
     record(8, ps);
     PAM_HIP(hipEventRecord(join_ev_, ps));

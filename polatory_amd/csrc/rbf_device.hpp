@@ -53,23 +53,6 @@ __device__ __forceinline__ float phi_f32(float r2, float a, float b) {
   }
 }
 
-// Square root for the FP64 near field: the hardware reciprocal square root
-// (v_rsq_f64, accurate to about 2^-23 relative) refined by one Goldschmidt
-// step and a final Newton correction of the remainder (Markstein's method),
-// within a few ulp of the correctly rounded sqrt in 8 instructions instead of
-// the compiler's IEEE-rounded expansion. 0 for x = 0 (coincident points); x is
-// a sum of squares, never negative.
-__device__ __forceinline__ double sqrt_nr(double x) {
-  const double y = __builtin_amdgcn_rsq(x);
-  double s = x * y, h = 0.5 * y;
-  const double r = fma(-s, h, 0.5);
-  s = fma(s, r, s);
-  h = fma(h, r, h);
-  const double d = fma(-s, s, x);
-  s = fma(d, h, s);
-  return x > 0.0 ? s : 0.0;
-}
-
 // The constant b that phi_shape<T> expects: the FP32 exponential is 2^(b r),
 // with log2 e folded in before the rounding to FP32.
 template <class T>
@@ -77,14 +60,25 @@ inline double phi_shape_const(int kind, double b) {
   return sizeof(T) == 4 && kind == kExp ? b * 1.4426950408889634074 : b;
 }
 
-// The same for x > 0 (no test for zero).
+// Square root for the FP64 sums, x > 0 and finite: the hardware reciprocal
+// square root (v_rsq_f64, accurate to about 2^-23 relative), one Goldschmidt
+// step and a Newton correction of the remainder (Markstein's method), within a
+// few ulp of the correctly rounded sqrt in 7 instructions instead of the
+// compiler's IEEE-rounded expansion. The correction's factor h needs no step
+// of its own: its 2^-23 meet a remainder below 2^-44.
 __device__ __forceinline__ double sqrt_pos(double x) {
   const double y = __builtin_amdgcn_rsq(x);
-  double s = x * y, h = 0.5 * y;
-  const double r = fma(-s, h, 0.5);
-  s = fma(s, r, s);
-  h = fma(h, r, h);
+  const double s0 = x * y, h = 0.5 * y;
+  const double s = fma(s0, fma(-s0, h, 0.5), s0);
   return fma(fma(-s, s, x), h, s);
+}
+
+// 1 / sqrt(x), x > 0 and finite: the hardware's reciprocal root and one
+// correction of third order, within an ulp.
+__device__ __forceinline__ double rsqrt_nr(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-(x * y), y, 1.0);
+  return fma(y, e * fma(0.375, e, 0.5), y);
 }
 
 // sum_k c_k m_k(x, y, z) over the monomials of degree 0..2
@@ -104,12 +98,11 @@ template <class T, int KIND>
 __device__ __forceinline__ T phi_shape(T r2c, T b) {
   if constexpr (sizeof(T) == 8) {
     if constexpr (KIND == kBh3) {
-      return sqrt_nr(r2c);
+      return sqrt_pos(r2c);
     } else if constexpr (KIND == kTh3) {
-      double rho = sqrt_nr(r2c);
-      return rho * rho * rho;
+      return r2c * sqrt_pos(r2c);
     } else {
-      return exp(b * sqrt_nr(r2c));
+      return exp(b * sqrt_pos(r2c));
     }
   } else {
     if constexpr (KIND == kBh3) {
@@ -122,24 +115,25 @@ __device__ __forceinline__ T phi_shape(T r2c, T b) {
   }
 }
 
-// Seed of the sum of squares that phi_shape expects.
+// Seed of the sum of squares that phi_shape expects. FP64: at least 1e-290, so
+// that the root of a coincident pair needs no test (r is then 1e-145 h).
 template <class T, int KIND>
 __device__ __forceinline__ T phi_seed(T b) {
-  if constexpr (KIND == kExp) {
-    return T(0);
-  } else {
-    return b;
-  }
+  const T s = KIND == kExp ? T(0) : b;
+  if constexpr (sizeof(T) == 8) return fmax(s, 1e-290);
+  else return s;
 }
 
-// Gradient in physical units from differences d in a local unit h:
-//   grad phi = ag * grad_shape(r2c) * d,  r2c = |d|^2 + phi_seed(b),
-// with (ag, b) from grad_consts(rbf, h) (rbf/polyharmonic_odd.hpp:41-53,
-// rbf/cov_exponential.hpp:42-50):
-//   bh3: ag = -slope,          grad_shape = 1 / sqrt(r2c)  (0 where r2c = 0)
-//   th3: ag = 3 slope h^2,     grad_shape = sqrt(r2c)
-//   exp: ag = -3 psill / range, grad_shape = exp(b r) / r, r = sqrt(r2c)
-// (at r = 0 the exponential's gradient is undefined, as in the reference).
+// Gradient and Hessian in physical units from differences u in a local unit h
+// (rbf/polyharmonic_odd.hpp:41-72, rbf/cov_exponential.hpp:42-62):
+//   grad phi = ag f u,  H a = (ag / h) f (a + t u (u . a)),
+// with (ag, b) from grad_consts(rbf, h) and f, t from grad_terms at
+// r2c = |u|^2 + grad_seed(b):
+//   bh3: ag = -slope,           f = 1 / sqrt(r2c)                      t = -1 / r2c
+//   th3: ag = 3 slope h^2,      f = sqrt(r2c)                          t = 1 / r2c
+//   exp: ag = -3 psill / range, f = exp(b r) / r, r = sqrt(r2c)        t = -(1 - b r) / r2c
+// At r2c = 0 the polyharmonic terms are zero; the exponential's are undefined,
+// as in the reference.
 inline PhiConsts grad_consts(const RbfDesc& rbf, double h) {
   const PhiConsts pc = phi_consts(rbf, h);
   switch (rbf.kind) {
@@ -150,43 +144,46 @@ inline PhiConsts grad_consts(const RbfDesc& rbf, double h) {
   throw_invalid("unknown rbf kind");
 }
 
+// FP64: at least 1e-200 (polyharmonic kernels), so that 1 / sqrt is finite.
 template <class T, int KIND>
-__device__ __forceinline__ T grad_shape(T r2c, T b) {
-  if constexpr (sizeof(T) == 8) {
-    if constexpr (KIND == kBh3) {
-      return r2c > 0.0 ? 1.0 / sqrt(r2c) : 0.0;
-    } else if constexpr (KIND == kTh3) {
-      return sqrt(r2c);
-    } else {
-      const double r = sqrt(r2c);
-      return exp(b * r) / r;
-    }
-  } else {
-    if constexpr (KIND == kBh3) {
-      return r2c > 0.0f ? __builtin_amdgcn_rsqf(r2c) : 0.0f;
-    } else if constexpr (KIND == kTh3) {
-      return __builtin_amdgcn_sqrtf(r2c);
-    } else {
-      const float rs = __builtin_amdgcn_rsqf(r2c);
-      return __expf(b * (r2c * rs)) * rs;
-    }
-  }
+__device__ __forceinline__ T grad_seed(T b) {
+  if constexpr (KIND == kExp) return T(0);
+  else if constexpr (sizeof(T) == 8) return fmax(b, 1e-200);
+  else return b;
 }
 
-// Hessian in physical units from local differences u (unit h):
-//   H a = (ag / h) grad_shape(r2c) (a + hess_t(r2c) u (u . a))
-// (rbf/polyharmonic_odd.hpp:56-72, rbf/cov_exponential.hpp:52-62):
-//   bh3 / th3: hess_t = (K - 2) / r2c   (0 where r2c = 0, where the reference returns 0)
-//   exp:       hess_t = -(1 - b r) / r^2, r = sqrt(r2c)
-template <class T, int KIND>
-__device__ __forceinline__ T hess_t(T r2c, T b) {
-  if constexpr (KIND == kBh3) {
-    return r2c > T(0) ? T(-1) / r2c : T(0);
-  } else if constexpr (KIND == kTh3) {
-    return r2c > T(0) ? T(1) / r2c : T(0);
+template <class T, int KIND, bool kHess>
+__device__ __forceinline__ void grad_terms(T r2c, T b, T* f, T* t) {
+  if constexpr (sizeof(T) == 8) {
+    if constexpr (KIND == kTh3 && !kHess) {
+      *f = sqrt_pos(r2c);
+    } else {
+      const double y = rsqrt_nr(r2c);
+      if constexpr (KIND == kBh3) {
+        // The Hessian's first term does not vanish with u.
+        *f = kHess && !(r2c > 1e-190) ? 0.0 : y;
+        *t = -(y * y);
+      } else if constexpr (KIND == kTh3) {
+        *f = r2c * y;
+        *t = y * y;
+      } else {
+        const double br = b * (r2c * y);
+        *f = exp(br) * y;
+        *t = (br - 1.0) * (y * y);
+      }
+    }
   } else {
-    const T r = sqrt(r2c);
-    return -(T(1) - b * r) / r2c;
+    if constexpr (KIND == kBh3) {
+      *f = r2c > 0.0f ? __builtin_amdgcn_rsqf(r2c) : 0.0f;
+      *t = r2c > 0.0f ? -1.0f / r2c : 0.0f;
+    } else if constexpr (KIND == kTh3) {
+      *f = __builtin_amdgcn_sqrtf(r2c);
+      *t = r2c > 0.0f ? 1.0f / r2c : 0.0f;
+    } else {
+      const float rs = __builtin_amdgcn_rsqf(r2c);
+      *f = __expf(b * (r2c * rs)) * rs;
+      *t = -(1.0f - b * sqrtf(r2c)) / r2c;
+    }
   }
 }
 

@@ -73,3 +73,70 @@ def test_mixed_near_field_does_not_depend_on_shared_launches():
         ev.set_target_points(trg)
         outs.append(ev.evaluate())
     np.testing.assert_array_equal(outs[0], outs[1])
+
+
+def pair_terms(kind, params, u, r2):
+    """phi, f, t with grad phi = f u and H = f (I + t u u^T) of the isotropic kernels."""
+    with np.errstate(divide="ignore", invalid="ignore"):
+        if kind in ("bh3", "bh3c"):
+            rho = np.sqrt(r2 + params[1] ** 2)
+            return -params[0] * rho, np.where(rho > 0, -params[0] / rho, 0.0), np.where(rho > 0, -1.0 / rho ** 2, 0.0)
+        if kind == "th3":
+            rho = np.sqrt(r2)
+            return params[0] * rho ** 3, 3 * params[0] * rho, np.where(rho > 0, 1.0 / r2, 0.0)
+        r, c = np.sqrt(r2), 3.0 / params[1]
+        e = params[0] * np.exp(-c * r)
+        return e, -c * e / r, -(1.0 / r2 + c / r)
+
+
+@pytest.mark.parametrize("mode", ["fp64 value", "fp64 gradient", "mixed gradient", "fp64 hessian", "mixed hessian"])
+@pytest.mark.parametrize("kind", list(KINDS))
+@pytest.mark.parametrize("n_src,n_trg", [(1, 1), (300, 4), (257, 33), (700, 129 * 8), (5000, 3000), (20000, 120)])
+def test_near_field_on_the_vector_units(kind, mode, n_src, n_trg):
+    """FP64 values, gradients and Hessian sums: 4, 8 or 16 target slots, up to
+    8 (5) targets per thread, several passes, shared sources."""
+    print("near field", kind, mode, n_src, n_trg, flush=True)
+    _, cls, params = KINDS[kind]
+    precision, what = mode.split()
+    rng = np.random.default_rng(n_src + n_trg)
+    src = rng.uniform(0.25, 0.75, (n_src, 3))
+    trg = rng.uniform(0.25, 0.75, (n_trg, 3))
+    if not (kind == "exp" and what != "value"):  # undefined at r = 0
+        k = min(n_src, n_trg) // 2
+        trg[:k] = src[:k]
+    w = rng.normal(size=(n_src, 3) if what == "hessian" else n_src)
+    make = {"value": pa.make_fmm_evaluator, "gradient": pa.make_fmm_gradient_transpose_evaluator,
+            "hessian": pa.make_fmm_hessian_evaluator}[what]
+    ev = make(cls(params), ((0, 0, 0), (1, 1, 1)))
+    ev.set_config(pa.FmmConfig(precision, 4, 2, "fmm"))
+    ev.set_source_points(src)
+    ev.set_weights(w.ravel())
+    ev.set_target_points(trg)
+    y = ev.evaluate().reshape(n_trg, -1)
+    assert ev.stats()["direct"] == 0
+    rows = rng.permutation(n_trg)[:200]
+    u = trg[rows][:, None, :] - src[None]
+    r2 = (u * u).sum(-1)
+    phi, f, t = pair_terms(kind, params, u, r2)
+    r = np.sqrt(r2)
+    if what == "value":
+        term, mag = (w * phi)[..., None], np.abs(w * phi)
+    elif what == "gradient":
+        term, mag = (w * f)[..., None] * u, np.abs(w * f) * r
+    else:
+        uw = (u * w).sum(-1)
+        term = -f[..., None] * (w + (t * uw)[..., None] * u)
+        mag = np.abs(f) * np.linalg.norm(w, axis=1) * (1 + np.abs(t) * r2)
+    # Sums: chains of at most n / 16 + 30 additions and products of half an ulp
+    # each. Coordinates in the leaf frame: 2 ulp of the half width on each
+    # side, so relative to r; the terms are of degree at most 3 in it.
+    ulp = 2.0 ** -53 if precision == "fp64" else 2.0 ** -24
+    rel = ulp * (n_src / 16 + 30 + 12 * 3 ** 0.5 * H / np.maximum(r, ulp))
+    bound = (mag * np.where(r > 0, rel, 0.0)).sum(1) + 1e-15 * (np.abs(w).max() * (1 + params[0]))
+    if kind == "bh3c" or what == "value":
+        bound += (mag * ulp * (n_src / 16 + 30)).sum(1)  # coincident pairs count
+    if kind == "exp":
+        bound *= 1 + 3 * np.sqrt(3) / params[1]  # degree of exp in r
+    worst = np.max(np.abs(y[rows] - term.sum(1)) / bound[:, None])
+    print(f"  worst error / bound {worst:.3f}", flush=True)
+    assert worst <= 1.0
