@@ -20,6 +20,8 @@ void launch_bbox(const double* pts, int64_t n, double* d_out, DevBuf<double>& sc
 void exclusive_scan_i32(const int32_t* in, int32_t* out, int64_t n, DevBuf<int32_t>& scratch,
                         hipStream_t s);
 // Stable LSD radix sort of (key, value) pairs on the low `bits` bits of key.
+// With an odd number of passes the input is in tk, tv (n entries each).
+int radix_sort_passes(int64_t n, int bits);
 void radix_sort_pairs(uint64_t* keys, int32_t* vals, int64_t n, int bits, DevBuf<uint64_t>& tk,
                       DevBuf<int32_t>& tv, DevBuf<int32_t>& hist, DevBuf<int32_t>& scratch,
                       hipStream_t s);

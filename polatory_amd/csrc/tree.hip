@@ -506,9 +506,15 @@ void sort_tree_points(Tree& t, const double* d_pts, int64_t n, const Box& box, i
   t.perm.resize(n);
   Lo3 lo{{box.lo[0], box.lo[1], box.lo[2]}};
   const double inv_cell = std::ldexp(1.0, sort_level) / box.width;
-  morton_kernel<<<ceil_div(n, 256), 256, 0, s>>>(d_pts, n, lo, inv_cell,
-                                                 (int64_t{1} << sort_level) - 1, t.point_codes.get(),
-                                                 t.perm.get());
+  // An odd number of passes starts from the workspace and ends in the tree.
+  const bool from_ws = radix_sort_passes(n, 3 * sort_level) % 2;
+  if (from_ws) {
+    ws.tk.resize(n);
+    ws.tv.resize(n);
+  }
+  morton_kernel<<<ceil_div(n, 256), 256, 0, s>>>(d_pts, n, lo, inv_cell, (int64_t{1} << sort_level) - 1,
+                                                 from_ws ? ws.tk.get() : t.point_codes.get(),
+                                                 from_ws ? ws.tv.get() : t.perm.get());
   PAM_LAUNCH_CHECK();
   radix_sort_pairs(t.point_codes.get(), t.perm.get(), n, 3 * sort_level, ws.tk, ws.tv, ws.hist,
                    ws.scan_scratch, s);

@@ -1,5 +1,5 @@
 // Generic device building blocks: point transforms, bbox reduction, prefix
-// sums, a stable LSD radix sort (4-bit digits), gathers and polynomial terms.
+// sums, a stable LSD radix sort, gathers and polynomial terms.
 #include <type_traits>
 #include <vector>
 
@@ -181,65 +181,97 @@ void scan_rec(const int32_t* in, int32_t* out, int64_t n, int32_t* scratch, hipS
   PAM_LAUNCH_CHECK();
 }
 
-// ---- radix sort: 4-bit digits, 256 threads x 8 consecutive items per tile ----
+// ---- radix sort: digits of up to 8 bits, tiles of 2,048 items ----
+//
+// Bound by launches up to some 100,000 items. A Morton code of 9 to 18 bits
+// takes two or three passes this way (three to five with 4-bit digits, whose
+// counters fitted in registers). Each wavefront of a tile ranks eight times 64
+// consecutive items: lanes with the same digit find each other by one ballot
+// per bit, and the digit's counter in LDS carries over to the next 64, so the
+// order stays stable and reads are coalesced.
+// MI355X, two trees of 1M points (18 bits, three passes instead of five and
+// two copies): tree stage 0.69 to 0.65 ms; of 50k points 0.46 to 0.43 ms.
 constexpr int kRsThreads = 256;
 constexpr int kRsItems = 8;
 constexpr int kRsTile = kRsThreads * kRsItems;
+constexpr int kRsMaxBits = 8;
 
-__global__ void radix_hist_kernel(const uint64_t* __restrict__ keys, int64_t n, int shift,
-                                  int32_t* __restrict__ hist, int nblocks) {
-  __shared__ int32_t cnt[16];
-  if (threadIdx.x < 16) cnt[threadIdx.x] = 0;
+__global__ void __launch_bounds__(kRsThreads)
+radix_hist_kernel(const uint64_t* __restrict__ keys, int64_t n, int shift, int bits, int32_t* __restrict__ hist,
+                  int nblocks) {
+  __shared__ int32_t cnt[1 << kRsMaxBits];
+  const unsigned digits = 1u << bits;
+  for (unsigned e = threadIdx.x; e < digits; e += kRsThreads) cnt[e] = 0;
   __syncthreads();
-  int64_t base = static_cast<int64_t>(blockIdx.x) * kRsTile;
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * kRsTile;
+#pragma unroll
   for (int q = 0; q < kRsItems; q++) {
-    int64_t i = base + threadIdx.x + q * kRsThreads;
-    if (i < n) atomicAdd(&cnt[(keys[i] >> shift) & 15u], 1);
+    const int64_t i = base + threadIdx.x + q * kRsThreads;
+    if (i < n) atomicAdd(&cnt[(keys[i] >> shift) & (digits - 1)], 1);
   }
   __syncthreads();
-  if (threadIdx.x < 16) hist[threadIdx.x * nblocks + blockIdx.x] = cnt[threadIdx.x];
+  for (unsigned e = threadIdx.x; e < digits; e += kRsThreads)
+    hist[static_cast<int64_t>(e) * nblocks + blockIdx.x] = cnt[e];
 }
 
-// Counters for 16 digits packed as 4 x uint64 with 16-bit fields (a tile holds
-// at most 2048 items, so no field overflows).
-__global__ void radix_scatter_kernel(const uint64_t* __restrict__ kin, const int32_t* __restrict__ vin,
-                                     uint64_t* __restrict__ kout, int32_t* __restrict__ vout,
-                                     int64_t n, int shift, const int32_t* __restrict__ offs,
-                                     int nblocks) {
-  __shared__ uint64_t pk[4][kRsThreads];
-  __shared__ int32_t boff[16];
-  int64_t base = static_cast<int64_t>(blockIdx.x) * kRsTile + threadIdx.x * kRsItems;
+__global__ void __launch_bounds__(kRsThreads)
+radix_scatter_kernel(const uint64_t* __restrict__ kin, const int32_t* __restrict__ vin, uint64_t* __restrict__ kout,
+                     int32_t* __restrict__ vout, int64_t n, int shift, int bits, const int32_t* __restrict__ offs,
+                     int nblocks) {
+  constexpr int kWaves = kRsThreads / 64;
+  __shared__ int32_t cnt[kWaves][1 << kRsMaxBits];  // per wave: items so far, then where its first one goes
+  const unsigned digits = 1u << bits;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  for (unsigned e = threadIdx.x; e < digits; e += kRsThreads)
+    for (int w = 0; w < kWaves; w++) cnt[w][e] = 0;
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * kRsTile + wave * (kRsTile / kWaves) + lane;
   uint64_t key[kRsItems];
-  int32_t val[kRsItems];
-  uint64_t c[4] = {0, 0, 0, 0};
+  int32_t val[kRsItems], rank[kRsItems];
+#pragma unroll
   for (int q = 0; q < kRsItems; q++) {
-    if (base + q < n) {
-      key[q] = kin[base + q];
-      val[q] = vin[base + q];
-      unsigned d = (key[q] >> shift) & 15u;
-      c[d >> 2] += 1ull << (16 * (d & 3));
-    }
+    const int64_t i = base + 64 * q;
+    key[q] = i < n ? kin[i] : 0;
+    val[q] = i < n ? vin[i] : 0;
   }
-  for (int k = 0; k < 4; k++) pk[k][threadIdx.x] = c[k];
-  if (threadIdx.x < 16) boff[threadIdx.x] = offs[threadIdx.x * nblocks + blockIdx.x];
   __syncthreads();
-  for (int off = 1; off < kRsThreads; off <<= 1) {
-    uint64_t t[4];
-    for (int k = 0; k < 4; k++) t[k] = (static_cast<int>(threadIdx.x) >= off) ? pk[k][threadIdx.x - off] : 0;
-    __syncthreads();
-    for (int k = 0; k < 4; k++) pk[k][threadIdx.x] += t[k];
-    __syncthreads();
-  }
-  uint64_t run[4];
-  for (int k = 0; k < 4; k++) run[k] = pk[k][threadIdx.x] - c[k];
+#pragma unroll
   for (int q = 0; q < kRsItems; q++) {
-    if (base + q < n) {
-      unsigned d = (key[q] >> shift) & 15u;
-      int64_t pos = boff[d] + static_cast<int64_t>((run[d >> 2] >> (16 * (d & 3))) & 0xFFFFull);
-      run[d >> 2] += 1ull << (16 * (d & 3));
-      kout[pos] = key[q];
-      vout[pos] = val[q];
+    const bool valid = base + 64 * q < n;
+    const unsigned d = static_cast<unsigned>(key[q] >> shift) & (digits - 1);
+    uint64_t same = __ballot(valid);
+    for (int b = 0; b < bits; b++) {
+      const uint64_t set = __ballot((d >> b) & 1u);
+      same &= ((d >> b) & 1u) ? set : ~set;
     }
+    const int before = __popcll(same & ((uint64_t{1} << lane) - 1));
+    const int32_t seen = cnt[wave][d];
+    rank[q] = seen + before;
+    // The reads of this step come before its writes, and those before the
+    // next step's reads; the counters belong to this wave.
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (valid && before == 0) cnt[wave][d] = seen + __popcll(same);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+  __syncthreads();
+  for (unsigned e = threadIdx.x; e < digits; e += kRsThreads) {
+    int32_t run = offs[static_cast<int64_t>(e) * nblocks + blockIdx.x];
+#pragma unroll
+    for (int w = 0; w < kWaves; w++) {
+      const int32_t c = cnt[w][e];
+      cnt[w][e] = run;
+      run += c;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < kRsItems; q++) {
+    if (base + 64 * q >= n) continue;
+    const unsigned d = static_cast<unsigned>(key[q] >> shift) & (digits - 1);
+    const int64_t pos = cnt[wave][d] + rank[q];
+    kout[pos] = key[q];
+    vout[pos] = val[q];
   }
 }
 
@@ -315,32 +347,35 @@ void exclusive_scan_i32(const int32_t* in, int32_t* out, int64_t n, DevBuf<int32
   scan_rec(in, out, n, scratch.get(), s);
 }
 
+int radix_sort_passes(int64_t n, int bits) { return n <= 1 || bits <= 0 ? 0 : (bits + kRsMaxBits - 1) / kRsMaxBits; }
+
 void radix_sort_pairs(uint64_t* keys, int32_t* vals, int64_t n, int bits, DevBuf<uint64_t>& tk,
                       DevBuf<int32_t>& tv, DevBuf<int32_t>& hist, DevBuf<int32_t>& scratch,
                       hipStream_t s) {
-  if (n <= 1 || bits <= 0) return;
-  int nb = ceil_div(n, kRsTile);
+  const int passes = radix_sort_passes(n, bits);
+  if (passes == 0) return;
+  const int nb = ceil_div(n, kRsTile);
+  const int width = (bits + passes - 1) / passes;
   tk.resize(static_cast<size_t>(n));
   tv.resize(static_cast<size_t>(n));
-  hist.resize(static_cast<size_t>(16) * nb);
+  hist.resize((static_cast<size_t>(1) << width) * nb);
   uint64_t* ka = keys;
   int32_t* va = vals;
   uint64_t* kb = tk.get();
   int32_t* vb = tv.get();
-  int passes = (bits + 3) / 4;
-  for (int p = 0; p < passes; p++) {
-    int shift = 4 * p;
-    radix_hist_kernel<<<nb, kRsThreads, 0, s>>>(ka, n, shift, hist.get(), nb);
-    PAM_LAUNCH_CHECK();
-    exclusive_scan_i32(hist.get(), hist.get(), static_cast<int64_t>(16) * nb, scratch, s);
-    radix_scatter_kernel<<<nb, kRsThreads, 0, s>>>(ka, va, kb, vb, n, shift, hist.get(), nb);
-    PAM_LAUNCH_CHECK();
+  if (passes % 2) {  // the input is in tk, tv
     std::swap(ka, kb);
     std::swap(va, vb);
   }
-  if (ka != keys) {
-    PAM_HIP(hipMemcpyAsync(keys, ka, sizeof(uint64_t) * n, hipMemcpyDeviceToDevice, s));
-    PAM_HIP(hipMemcpyAsync(vals, va, sizeof(int32_t) * n, hipMemcpyDeviceToDevice, s));
+  for (int p = 0; p < passes; p++) {
+    const int shift = width * p, w = std::min(width, bits - shift);
+    radix_hist_kernel<<<nb, kRsThreads, 0, s>>>(ka, n, shift, w, hist.get(), nb);
+    PAM_LAUNCH_CHECK();
+    exclusive_scan_i32(hist.get(), hist.get(), (static_cast<int64_t>(1) << w) * nb, scratch, s);
+    radix_scatter_kernel<<<nb, kRsThreads, 0, s>>>(ka, va, kb, vb, n, shift, w, hist.get(), nb);
+    PAM_LAUNCH_CHECK();
+    std::swap(ka, kb);
+    std::swap(va, vb);
   }
 }
 
