@@ -2,9 +2,9 @@
 // make_fmm_gradient_evaluator, make_fmm_evaluator.cpp:78-107): sources carry
 // 3-vector weights (gradient data) and the targets receive values,
 //   out_i = sum_j w_j . (-A^T grad phi(A (t_i - s_j))) = -sum_k d/dx_k F_k(t_i),
-// with F_k the scalar-weight sum of the k-th weight components. Evaluated as
-// three gradient-transpose passes over one source tree, keeping the k-th
-// component of pass k.
+// with F_k the scalar-weight sum of the k-th weight components. One direct sum
+// where that is chosen, otherwise three gradient-transpose passes over one
+// source tree, keeping the k-th component of pass k.
 #pragma once
 
 #include "fmm_evaluator.hpp"
@@ -30,7 +30,7 @@ class DipoleSourceEvaluator {
 // make_fmm_evaluator.cpp:160-188): sources carry 3-vector weights and the
 // targets receive 3-vectors,
 //   out_i = -sum_j A^T H(A (t_i - s_j)) A w_j = -sum_k column k of the Hessian of F_k,
-// as three Hessian-column passes over one source tree.
+// as one direct sum or three Hessian-column passes over one source tree.
 class DipoleHessianEvaluator {
  public:
   explicit DipoleHessianEvaluator(FmmEvaluator& ev);
