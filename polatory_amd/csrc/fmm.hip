@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "fmm.hpp"
+#include "share.hpp"
 
 namespace pam {
 
@@ -599,19 +600,18 @@ __device__ __forceinline__ void near_leaf(const P2PJob<T>& j, int unit, const An
   __shared__ double red[kOut][16 * kTiles][4];
   int leaf, part, spart;
   p2p_unit(j, unit, &leaf, &part, &spart);
-  const int ts = j.tls[leaf], te = j.tls[leaf + 1];
-  const int parts = min(j.parts, (te - ts + 16 * kTiles - 1) / (16 * kTiles));
+  const int ts = j.tls[leaf], nt = j.tls[leaf + 1] - ts;
+  const int parts = min(j.parts, share_count(nt, 16 * kTiles));
   if (part >= parts) return;
-  const int p0 = ts + static_cast<int>(static_cast<int64_t>(te - ts) * part / parts);
-  const int p1 = ts + static_cast<int>(static_cast<int64_t>(te - ts) * (part + 1) / parts);
+  const int p0 = ts + share_begin(nt, part, parts), np = ts + share_begin(nt, part + 1, parts) - p0;
   if (threadIdx.x < 64) nb.build(j, leaf, T(2), threadIdx.x);
   T col[3] = {T(0), T(0), T(0)};
   if constexpr (MODE == kNearHessian)
     for (int k = 0; k < 3; k++) col[k] = static_cast<T>(A.a[3 * k + kcol]);
   __syncthreads();
-  const int npass = (p1 - p0 + 16 * kTiles - 1) / (16 * kTiles);
+  const int npass = share_count(np, 16 * kTiles);
   for (int ps = 0; ps < npass; ps++) {
-    const int t0 = p0 + (p1 - p0) * ps / npass, n = p0 + (p1 - p0) * (ps + 1) / npass - t0;
+    const int t0 = p0 + share_begin(np, ps, npass), n = p0 + share_begin(np, ps + 1, npass) - t0;
     int slots = 16;
     while (slots > 4 && 2 * n <= kTiles * slots) slots /= 2;
 #define PAM_NEAR_PASS(RR)                                                                    \
@@ -836,11 +836,11 @@ __global__ void __launch_bounds__(kThreads, 4) p2p_mf_jobs_kernel(P2PJobs<float>
   int leaf, part, spart;
   p2p_unit(j, static_cast<int>(blockIdx.x) - j.first_block, &leaf, &part, &spart);
   const int ts = j.tls[leaf], te = j.tls[leaf + 1];
-  const int tiles = (te - ts + 15) / 16;
+  const int tiles = share_count(te - ts, 16);
   const int parts = min(j.parts, max(1, tiles / kMfPartTiles));
   if (part >= parts) return;
-  const int tile0 = tiles * part / parts, tile1 = tiles * (part + 1) / parts;
-  if (tile0 == tile1) return;
+  const int tile0 = share_begin(tiles, part, parts), ntile = share_begin(tiles, part + 1, parts) - tile0;
+  if (ntile == 0) return;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   if (wave == 0) nb.build(j, leaf, static_cast<float>(2.0 / kMfUnit), lane);
   __syncthreads();
@@ -857,10 +857,9 @@ __global__ void __launch_bounds__(kThreads, 4) p2p_mf_jobs_kernel(P2PJobs<float>
     a[64 + 32] = mf_pack(1.0f, 1.0f, 0.0f, 0.0f);
     a[128 + 48] = mf_pack(0x1p-10f, 0.0f, 0.0f, 0.0f);
   }
-  const int npass = (tile1 - tile0 + 4 * kMfMaxTiles - 1) / (4 * kMfMaxTiles);
+  const int npass = share_count(ntile, 4 * kMfMaxTiles);
   for (int ps = 0; ps < npass; ps++) {
-    const int p0 = tile0 + (tile1 - tile0) * ps / npass, p1 = tile0 + (tile1 - tile0) * (ps + 1) / npass;
-    const int n = p1 - p0;
+    const int p0 = tile0 + share_begin(ntile, ps, npass), n = tile0 + share_begin(ntile, ps + 1, npass) - p0;
     // The pass's tiles over G groups of waves, the sources over 4 / G splits:
     // as few groups as kMfMaxTiles tiles per wave allow.
     const int G = n <= kMfMaxTiles ? 1 : (n <= 2 * kMfMaxTiles ? 2 : 4), S = 4 / G;

@@ -140,3 +140,38 @@ def test_near_field_on_the_vector_units(kind, mode, n_src, n_trg):
     worst = np.max(np.abs(y[rows] - term.sum(1)) / bound[:, None])
     print(f"  worst error / bound {worst:.3f}", flush=True)
     assert worst <= 1.0
+
+
+@pytest.mark.parametrize("what,precision,many", [("value", "fp64", 600_001), ("gradient", "mixed", 600_001),
+                                                 ("gradient", "fp64", 420_001), ("value", "mixed", 3_400_001)])
+def test_very_many_targets_in_one_leaf(what, precision, many):
+    """A zoom into one leaf: so many targets that their number times the
+    number of passes over them does not fit 32 bits. 4,096 occupied leaves, so
+    that no leaf is shared out to several workgroups."""
+    print("many targets", what, precision, many, flush=True)
+    rng = np.random.default_rng(many)
+    width = 1.01 / 16
+    centre = -0.005 + (np.arange(16) + 0.5) * width
+    spots = centre[8] + rng.uniform(-0.49, 0.49, (1000, 3)) * width
+    pick = rng.integers(0, 1000, many)
+    grid = np.stack(np.meshgrid(centre, centre, centre, indexing="ij"), -1).reshape(-1, 3)
+    src = centre[8] + rng.uniform(-1.49, 1.49, (300, 3)) * width  # in its neighbours: no far field
+    w = rng.normal(size=300)
+    make = pa.make_fmm_evaluator if what == "value" else pa.make_fmm_gradient_transpose_evaluator
+    ev = make(pa.Biharmonic3D(), ((0, 0, 0), (1, 1, 1)))
+    ev.set_config(pa.FmmConfig(precision, 3, 4, "fmm"))
+    ev.set_source_points(src)
+    ev.set_weights(w)
+    ev.set_target_points(np.concatenate([grid, spots[pick]]))
+    y = ev.evaluate().reshape(len(grid) + many, -1)[len(grid):]
+    assert ev.stats()["n_trg_leaves"] == 4096
+    u = spots[:, None, :] - src[None]
+    r = np.linalg.norm(u, axis=2)
+    term = -(w * r)[..., None] if what == "value" else -(w / r)[..., None] * u
+    # Half an ulp per operation of a chain of at most 300 + 30, coordinates to
+    # two ulp of the half width on each side.
+    ulp = 2.0 ** -53 if precision == "fp64" else 2.0 ** -24
+    bound = (np.linalg.norm(term, axis=2) * ulp * (330 + 12 * 3 ** 0.5 * (width / 2) / r)).sum(1)
+    worst = np.max(np.abs(y - term.sum(1)[pick]) / bound[pick, None])
+    print(f"  worst error / bound {worst:.3f}", flush=True)
+    assert worst <= 1.0
