@@ -669,22 +669,29 @@ __global__ void __launch_bounds__(kThreads, 3) p2p_vector_kernel(P2PJob<T> j, An
 // with VALU work). The FP16 matrix unit is separate, so |s|^2 - 2 s.t + |t|^2
 // is formed there, from coordinates split so that the cancellation is exact:
 // in units of 2^-9 of the leaf half width, s = S + s1 + s2 with S an integer
-// (|S| <= 1536), s1 a multiple of 2^-11 (|s1| <= 1/2) and s2 the rest in FP16
-// (|s2| <= 2^-12, stored times 2^12). Three v_mfma_f32_16x16x16_f16 give, for
-// 16 sources and 16 targets, each starting from the sum so far,
-//   |S - T|^2                          integers below 2^24: exact;
-//   2 (S - T).(s1 - t1)                multiples of 2^-11 below 2^13: exact
-//                                      beside a small |S - T|^2, else one rounding;
-//   |s1 - t1|^2 + 2 (S - T).(s2 - t2)  one rounding; terms below 2^2.
-// What only the source (target) decides is summed beforehand and enters as
-// one or two FP16 pieces against constants. The neglected 2 (s1 - t1).(s2 -
-// t2) is below 2^-9 units (2^-27 of the half width squared) and zero for
-// coincident points. So r^2 keeps FP32 relative accuracy down to distances
-// where FP32 coordinates end. The VALU is left with root and FMA (12 cycles
-// per 64 pairs; the three matrix instructions show with 7 more).
+// (|S| <= 1536), s1 a multiple of 2^-11 (|s1| <= 1/2) and s2 the rest to a
+// multiple of 2^-22 (|s2| <= 2^-12, stored times 2^12). The unit adds eight
+// products at a time, in order, to the sum so far: terms below 2^-24 of the
+// largest of them are cut off, and the sum is rounded to FP32 (measured). So
+// the terms are laid out by size, in eight steps of eight, which are two
+// v_mfma_f32_16x16x32_f16 for 16 sources and 16 targets:
+//   0     |S - T|^2                          integers below 2^24
+//   1, 2  2 (S - T).(s1 - t1)                multiples of 2^-10 below 2^13
+//   3, 4  |s1 - t1|^2 + 2 (S - T).(s2 - t2)  multiples of 2^-22 below 2^2
+//   5, 6  2 (s1 - t1).(s2 - t2)              multiples of 2^-32 below 2^-9
+//   7     |s2 - t2|^2                        multiples of 2^-44 below 2^-21
+// What only the source (target) decides is summed beforehand and enters as two
+// FP16 pieces against constants. For points so close that the sums of the
+// first steps nearly vanish, every step is exact, and r^2 is rounded where it
+// no longer shrinks: its error is relative to r^2 itself, 2^-23, and
+// coincident points give zero. The coordinates are those in FP64 to 2^-32 of
+// the half width. (With s2 in FP16 and the last three steps left out, r was
+// off by up to 2^-20 half widths: 3.5e-5 of it at 2^-8 half widths, 5e-3 at
+// 2^-12.) The VALU is left with root and FMA.
 // Near field of 1M x 1M uniform points at order 8 (5.9e9 pairs, MI355X, alone):
-// 1.65 ms on the VALU, 1.62 ms with FP64 matrix distances, 0.99 ms this way;
-// 300k surface points (symmetric, uneven leaves): 1.68 to 0.65 ms, of which
+// 1.65 ms on the VALU, 1.62 ms with FP64 matrix distances, 1.10 ms this way
+// (1.12 ms beside it with three v_mfma_f32_16x16x16_f16 that left the last
+// three steps out); 300k surface points (symmetric, uneven leaves): 1.68 to 0.65 ms, of which
 // about half is the finer split of the leaves. Four or six tiles per wave
 // instead of five: 1.09 and 1.00 ms. Two workgroups per leaf at 4,096 leaves:
 // 1.05 ms; at 512 leaves eight per leaf fill the chip.
@@ -695,25 +702,27 @@ constexpr double kMfUnit = 0x1p-9;
 // itself), and source parts at most.
 constexpr int kMfPartTiles = 4, kMfMaxSparts = 3;
 
-using h16x4 = _Float16 __attribute__((ext_vector_type(4)));
+using h16x8 = _Float16 __attribute__((ext_vector_type(8)));
 using f32x4v = float __attribute__((ext_vector_type(4)));
 
 // A leaf-local coordinate split as above; the FP64 rest of the integer part
 // is below 1/2, so FP32 holds it to 2^-26 units.
 struct MfCoord {
-  float i, f1, f2;  // integer part, multiple of 2^-11, 2^12 x the rest (FP16 values)
+  float i, f1, f2;  // integer part, multiple of 2^-11, 2^12 x the rest, a multiple of 2^-10 (FP16 values)
 };
 __device__ __forceinline__ MfCoord mf_split(double x) {
   const double u = x * (1.0 / kMfUnit);
   const double r = rint(u);
   const float rho = static_cast<float>(u - r);
   const float f1 = rintf(rho * 2048.0f) * 0x1p-11f;
-  return {static_cast<float>(r), f1, static_cast<float>(static_cast<_Float16>((rho - f1) * 4096.0f))};
+  return {static_cast<float>(r), f1, rintf((rho - f1) * 0x1p22f) * 0x1p-10f};
 }
 // The parts that only one point decides: |P|^2 = 4096 a + b, 2 P.p1 = c1 + c2,
-// |p1|^2 + 2 P.p2 = d1 + 2^-10 d2, all FP16 values.
+// |p1|^2 + 2 P.p2 = d1 + 2^-10 d2, 2 p1.p2 = 2^-11 (e1 + e2), |p2|^2 = 2^-24
+// (g1 + g2), all FP16 values. Exact (d where |P| is small enough for the
+// point to be close to a target: |d| < 2).
 struct MfSelf {
-  float a, b, c1, c2, d1, d2;
+  float a, b, c1, c2, d1, d2, e1, e2, g1, g2;
 };
 __device__ __forceinline__ float mf_half(float v) { return static_cast<float>(static_cast<_Float16>(v)); }
 __device__ __forceinline__ MfSelf mf_self(const MfCoord& x, const MfCoord& y, const MfCoord& z) {
@@ -728,11 +737,22 @@ __device__ __forceinline__ MfSelf mf_self(const MfCoord& x, const MfCoord& y, co
                   0x1p-11f * fmaf(z.i, z.f2, fmaf(y.i, y.f2, x.i * x.f2));
   s.d1 = mf_half(d);
   s.d2 = (d - s.d1) * 1024.0f;
+  const float e = fmaf(z.f1, z.f2, fmaf(y.f1, y.f2, x.f1 * x.f2));
+  s.e1 = rintf(e * 1024.0f) * 0x1p-10f;
+  s.e2 = e - s.e1;
+  const float g = fmaf(z.f2, z.f2, fmaf(y.f2, y.f2, x.f2 * x.f2));
+  s.g1 = rintf(g * 512.0f) * 0x1p-9f;
+  s.g2 = g - s.g1;
   return s;
 }
-__device__ __forceinline__ h16x4 mf_pack(float a, float b, float c, float d) {
-  return h16x4{static_cast<_Float16>(a), static_cast<_Float16>(b), static_cast<_Float16>(c),
-               static_cast<_Float16>(d)};
+// The values are FP16 values, so the pairwise conversion does not round.
+__device__ __forceinline__ h16x8 mf_pack(float a, float b, float c, float d, float e, float f, float g, float h) {
+  using pair = decltype(__builtin_amdgcn_cvt_pkrtz(a, b));
+  struct {
+    pair v[4];
+  } r{{__builtin_amdgcn_cvt_pkrtz(a, b), __builtin_amdgcn_cvt_pkrtz(c, d), __builtin_amdgcn_cvt_pkrtz(e, f),
+       __builtin_amdgcn_cvt_pkrtz(g, h)}};
+  return __builtin_bit_cast(h16x8, r);
 }
 
 // Running sums of a lane's rows of one target tile: two FP32 chains, or, for
@@ -749,32 +769,49 @@ struct MfSum<true> {
   __device__ double value() const { return sum; }
 };
 
-// A target as a matrix column of the three products: reduction indices 4 grp
-// .. 4 grp + 3 (the sources' rows are written in p2p_mf_jobs_kernel).
+// A source's row of step k, and a target's column: their products add up to
+// the terms above. Lane group g of a wave (lane / 16) holds steps g and g + 4.
+// Subnormal FP16 values (below 2^-14) count in full.
+__device__ __forceinline__ void mf_rows(const MfCoord& x, const MfCoord& y, const MfCoord& z, h16x8* row) {
+  const MfSelf q = mf_self(x, y, z);
+  const float k = 0x1p-12f;
+  row[0] = mf_pack(x.i, y.i, z.i, q.a, q.b, 4096.0f, 1.0f, 0.0f);
+  row[1 * 16] = mf_pack(x.f1, y.f1, z.f1, x.i, y.i, z.i, q.c1, q.c2);
+  row[3 * 16] = mf_pack(x.f1, y.f1, z.f1, x.i, y.i, z.i, q.d1, q.d2);
+  row[4 * 16] = mf_pack(x.f2, y.f2, z.f2, 1.0f, 0x1p-10f, 0.0f, 0.0f, 0.0f);
+  row[5 * 16] = mf_pack(x.f1, y.f1, z.f1, x.f2, y.f2, z.f2, q.e1, q.e2);
+  row[7 * 16] = mf_pack(k * x.f2, k * y.f2, k * z.f2, k * q.g1, q.g2, k, k * k, 0.0f);
+}
+// Steps 2 and 6 are the same for every source.
+__device__ __forceinline__ void mf_const_rows(h16x8* row) {
+  row[2 * 16] = mf_pack(1.0f, 1.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f);
+  row[6 * 16] = mf_pack(0x1p-11f, 0x1p-11f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f);
+}
 struct MfColumn {
-  h16x4 b[3];
+  h16x8 b[2];
 };
 __device__ __forceinline__ MfColumn mf_column(const V4<double>& p, int grp) {
   const MfCoord x = mf_split(p.x), y = mf_split(p.y), z = mf_split(p.z);
   const MfSelf q = mf_self(x, y, z);
-  const float k = 0x1p-12f;
-  const h16x4 zero = mf_pack(0.0f, 0.0f, 0.0f, 0.0f);
+  const float k = 0x1p-12f, m = -0x1p-11f;
   if (grp == 0)
-    return {{mf_pack(x.i, y.i, z.i, 4096.0f), mf_pack(-2.0f * x.i, -2.0f * y.i, -2.0f * z.i, -2.0f * x.f1),
-             mf_pack(-2.0f * x.f1, -2.0f * y.f1, -2.0f * z.f1, -2.0f * k * x.i)}};
+    return {{mf_pack(-2.0f * x.i, -2.0f * y.i, -2.0f * z.i, 4096.0f, 1.0f, q.a, q.b, 0.0f),
+             mf_pack(m * x.i, m * y.i, m * z.i, q.d1, q.d2, 0.0f, 0.0f, 0.0f)}};
   if (grp == 1)
-    return {{mf_pack(1.0f, q.a, q.b, 0.0f), mf_pack(-2.0f * y.f1, -2.0f * z.f1, 1.0f, 1.0f),
-             mf_pack(-2.0f * k * y.i, -2.0f * k * z.i, -2.0f * x.f2, -2.0f * y.f2)}};
+    return {{mf_pack(-2.0f * x.i, -2.0f * y.i, -2.0f * z.i, -2.0f * x.f1, -2.0f * y.f1, -2.0f * z.f1, 1.0f, 1.0f),
+             mf_pack(m * x.f2, m * y.f2, m * z.f2, m * x.f1, m * y.f1, m * z.f1, -m, -m)}};
   if (grp == 2)
-    return {{zero, mf_pack(q.c1, q.c2, 0.0f, 0.0f), mf_pack(-2.0f * z.f2, 1.0f, 0x1p-10f, q.d1)}};
-  return {{zero, zero, mf_pack(q.d2, 0.0f, 0.0f, 0.0f)}};
+    return {{mf_pack(q.c1, q.c2, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f),
+             mf_pack(q.e1, q.e2, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f)}};
+  return {{mf_pack(-2.0f * x.f1, -2.0f * y.f1, -2.0f * z.f1, m * x.f2, m * y.f2, m * z.f2, 1.0f, 0x1p-10f),
+           mf_pack(m * x.f2, m * y.f2, m * z.f2, k, k * k, k * q.g1, q.g2, 0.0f)}};
 }
 
 // Adds to tot[0..M) the sums of M target tiles (their columns t) over the
 // staged source blocks s0, s0 + ds, ...: MFMA row = source, column = target; a
 // lane holds rows 4 (lane / 16) + i of column lane % 16.
 template <int KIND, bool kComp, int M>
-__device__ __forceinline__ void mf_tiles(const h16x4* sa, const f32x4v* sw, int nblk, int s0, int ds,
+__device__ __forceinline__ void mf_tiles(const h16x8* sa, const f32x4v* sw, int nblk, int s0, int ds,
                                          const MfColumn* t, float pb, float seed, MfSum<kComp>* tot) {
   const int lane = threadIdx.x & 63, grp = lane >> 4;
   const f32x4v init{seed, seed, seed, seed};
@@ -789,15 +826,13 @@ __device__ __forceinline__ void mf_tiles(const h16x4* sa, const f32x4v* sw, int 
     }
   }
   for (int blk = s0; blk < nblk; blk += ds) {
-    const h16x4 a0 = sa[blk * 192 + lane], a1 = sa[blk * 192 + 64 + lane], a2 = sa[blk * 192 + 128 + lane];
+    const h16x8 a0 = sa[blk * 128 + lane], a1 = sa[blk * 128 + 64 + lane];
     const f32x4v w = sw[blk * 4 + grp];
     f32x4v d[M];
 #pragma unroll
-    for (int m = 0; m < M; m++) d[m] = __builtin_amdgcn_mfma_f32_16x16x16f16(a0, t[m].b[0], init, 0, 0, 0);
+    for (int m = 0; m < M; m++) d[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, t[m].b[0], init, 0, 0, 0);
 #pragma unroll
-    for (int m = 0; m < M; m++) d[m] = __builtin_amdgcn_mfma_f32_16x16x16f16(a1, t[m].b[1], d[m], 0, 0, 0);
-#pragma unroll
-    for (int m = 0; m < M; m++) d[m] = __builtin_amdgcn_mfma_f32_16x16x16f16(a2, t[m].b[2], d[m], 0, 0, 0);
+    for (int m = 0; m < M; m++) d[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, t[m].b[1], d[m], 0, 0, 0);
 #pragma unroll
     for (int m = 0; m < M; m++)
 #pragma unroll
@@ -828,7 +863,7 @@ __device__ __forceinline__ void mf_tiles(const h16x4* sa, const f32x4v* sw, int 
 
 template <int KIND, bool kComp>
 __global__ void __launch_bounds__(kThreads, 4) p2p_mf_jobs_kernel(P2PJobs<float> jobs) {
-  __shared__ h16x4 sa[kMfSrc / 16 * 192];  // [16-source block][product][reduction index / 4][row]
+  __shared__ h16x8 sa[kMfSrc / 16 * 128];  // [16-source block][step][row]
   __shared__ f32x4v sw[kMfSrc / 4];        // [block][row]: weights
   __shared__ P2PNeighbours<float> nb;  // offsets in units
   __shared__ double red[4][kMfMaxTiles * 16];
@@ -849,14 +884,8 @@ __global__ void __launch_bounds__(kThreads, 4) p2p_mf_jobs_kernel(P2PJobs<float>
   const int first = spart * kMfSrc, step = j.sparts * kMfSrc;
   const float pa = j.pa, pb = j.pb;
   const float seed = phi_seed<float, KIND>(pb);
-  // Entries that no source changes: the constants against the targets' own
-  // parts, and the unused reduction indices.
-  {
-    h16x4* a = sa + (tid >> 4) * 192 + (tid & 15);
-    a[32] = a[48] = a[64 + 48] = mf_pack(0.0f, 0.0f, 0.0f, 0.0f);
-    a[64 + 32] = mf_pack(1.0f, 1.0f, 0.0f, 0.0f);
-    a[128 + 48] = mf_pack(0x1p-10f, 0.0f, 0.0f, 0.0f);
-  }
+  h16x8* const row = sa + (tid >> 4) * 128 + (tid & 15);  // this thread's source of a chunk
+  mf_const_rows(row);
   const int npass = share_count(ntile, 4 * kMfMaxTiles);
   for (int ps = 0; ps < npass; ps++) {
     const int p0 = tile0 + share_begin(ntile, ps, npass), n = tile0 + share_begin(ntile, ps + 1, npass) - p0;
@@ -893,17 +922,8 @@ __global__ void __launch_bounds__(kThreads, 4) p2p_mf_jobs_kernel(P2PJobs<float>
       x.i += nb.off[k][0];  // exact: an integer number of units
       y.i += nb.off[k][1];
       z.i += nb.off[k][2];
-      const MfSelf s = mf_self(x, y, z);
-      const float c = 0x1p-12f;
       __syncthreads();
-      h16x4* a = sa + (tid >> 4) * 192 + (tid & 15);
-      a[0] = mf_pack(-2.0f * x.i, -2.0f * y.i, -2.0f * z.i, s.a);
-      a[16] = mf_pack(s.b, 4096.0f, 1.0f, 0.0f);
-      a[64] = mf_pack(x.f1, y.f1, z.f1, x.i);
-      a[64 + 16] = mf_pack(y.i, z.i, s.c1, s.c2);
-      a[128] = mf_pack(x.f1, y.f1, z.f1, x.f2);
-      a[128 + 16] = mf_pack(y.f2, z.f2, c * x.i, c * y.i);
-      a[128 + 32] = mf_pack(c * z.i, s.d1, s.d2, 1.0f);
+      mf_rows(x, y, z, row);
       reinterpret_cast<float*>(sw)[tid] = static_cast<float>(q.w) * pa;  // the kernel's factor a folded in
       fetch(cb + step + tid);
       __syncthreads();

@@ -37,11 +37,11 @@ def test_mixed_near_field_matches_direct_sum(orc, kind, precision, n_src, n_trg)
     ev.set_target_points(trg)
     y = ev.evaluate()
     ref = orc.direct_rbf_sum(orc.make_rbf(getattr(orc, name), params), src, w, trg)
-    # Per pair: r^2 in FP32 from exact splits (three roundings of the matrix
-    # unit of up to 2^-21 together, observed 4.8e-7 of the largest term), root,
-    # product and sums 2^-24 each along chains of n / 8; the exponential turns
-    # a relative error of r into 3 r / range times as much. Absolute floor:
-    # r^2 is off by up to 2^-37 H^2 for coincident points, r by 2^-18 H.
+    # Per pair: r^2 in FP32 from exact splits (eight steps of the matrix unit
+    # with roundings of up to 2^-21 together, observed 4.8e-7 of the largest
+    # term), root, product and sums 2^-24 each along chains of n / 8; the
+    # exponential turns a relative error of r into 3 r / range times as much.
+    # Coordinates to 2^-32 H on each side: r to 2^-30 H.
     d = np.linalg.norm(trg[:, None, :] - src[None, :, :], axis=2)
     if kind in ("bh3", "bh3c"):
         phi, slope, grow = params[0] * np.sqrt(d * d + params[1] ** 2), params[0], 1.0
@@ -50,10 +50,50 @@ def test_mixed_near_field_matches_direct_sum(orc, kind, precision, n_src, n_trg)
     else:
         phi, slope, grow = params[0] * np.exp(-3 * d / params[1]), 3 * params[0] / params[1], 1.0 + 3 * d / params[1]
     rel = 2.0 ** -21 * grow + 2.0 ** -24 * (2 + n_src / 8 ** 0.5 / 8)
-    bound = (np.abs(w) * (phi * rel + slope * H * 2.0 ** -18 * (d < 1e-3))).sum(axis=1) + 1e-12
+    bound = (np.abs(w) * (phi * rel + slope * H * 2.0 ** -30 * (d > 0))).sum(axis=1) + 1e-12
     worst = np.max(np.abs(y - ref) / bound)
     print(f"  worst error / bound {worst:.3f}, rel {np.abs(y - ref).max() / np.abs(ref).max():.2e}", flush=True)
     assert worst <= 1.0
+
+
+def single_pairs(rng, cls, params, precision, dist):
+    """Values, exact values and distances of targets around single sources of
+    weight 1, dist leaf half widths away; half of the sources sit so that
+    leaves' common face lies between them and some of their targets."""
+    out = []
+    for k in range(8):
+        s = rng.uniform(0.26, 0.74, 3)
+        if k % 2:
+            s[k // 2 % 3] = 0.5 - 0.3 * dist * H
+        u = rng.normal(size=(300, 3))
+        t = s + dist * H * u / np.linalg.norm(u, axis=1)[:, None]
+        t = t[np.all((t > 0.25) & (t < 0.75), axis=1)]
+        ev = pa.make_fmm_evaluator(cls(params), ((0, 0, 0), (1, 1, 1)))
+        ev.set_config(pa.FmmConfig(precision, 4, 2, "fmm"))
+        ev.set_source_points(s[None])
+        ev.set_weights(np.ones(1))
+        ev.set_target_points(t)
+        y = ev.evaluate()
+        assert ev.stats()["direct"] == 0
+        out.append((y, np.linalg.norm(t - s, axis=1)))
+    return [np.concatenate(a) for a in zip(*out)]
+
+
+@pytest.mark.parametrize("precision", ["mixed", "mixed_comp"])
+@pytest.mark.parametrize("k", range(0, 21, 2))
+def test_mixed_near_field_of_one_close_pair(k, precision):
+    print("close pair", k, precision, flush=True)
+    y, r = single_pairs(np.random.default_rng(k), pa.Biharmonic3D, [1.0, 0.0], precision, 2.0 ** -k)
+    # As above: 2^-21 of r, and each coordinate to 2^-32 H on each side.
+    worst = np.max(np.abs(y + r) / (2.0 ** -21 * r + 2 * 3 ** 0.5 * 2.0 ** -32 * H))
+    print(f"  worst error / bound {worst:.3f}, rms of r {np.sqrt(np.mean((y + r) ** 2 / r ** 2)):.1e}", flush=True)
+    assert worst <= 1.0
+
+
+@pytest.mark.parametrize("precision", ["mixed", "mixed_comp"])
+def test_mixed_near_field_of_coincident_points_is_zero(precision):
+    y, r = single_pairs(np.random.default_rng(1), pa.Biharmonic3D, [1.0, 0.0], precision, 0.0)
+    assert not r.any() and not y.any()
 
 
 def test_mixed_near_field_does_not_depend_on_shared_launches():
