@@ -687,7 +687,10 @@ __global__ void __launch_bounds__(kThreads, 3) p2p_vector_kernel(P2PJob<T> j, An
 // coincident points give zero. The coordinates are those in FP64 to 2^-32 of
 // the half width. (With s2 in FP16 and the last three steps left out, r was
 // off by up to 2^-20 half widths: 3.5e-5 of it at 2^-8 half widths, 5e-3 at
-// 2^-12.) The VALU is left with root and FMA.
+// 2^-12.) A kernel's offset is added to the finished r^2: as the sum's start it
+// would be rounded to what is left beside the large terms (one of 0.03 units^2
+// came out 18 % off at coincident points). The VALU is left with root and FMA,
+// and that addition where there is an offset.
 // Near field of 1M x 1M uniform points at order 8 (5.9e9 pairs, MI355X, alone):
 // 1.65 ms on the VALU, 1.62 ms with FP64 matrix distances, 1.10 ms this way
 // (1.12 ms beside it with three v_mfma_f32_16x16x16_f16 that left the last
@@ -814,7 +817,7 @@ template <int KIND, bool kComp, int M>
 __device__ __forceinline__ void mf_tiles(const h16x8* sa, const f32x4v* sw, int nblk, int s0, int ds,
                                          const MfColumn* t, float pb, float seed, MfSum<kComp>* tot) {
   const int lane = threadIdx.x & 63, grp = lane >> 4;
-  const f32x4v init{seed, seed, seed, seed};
+  const f32x4v zero{0.0f, 0.0f, 0.0f, 0.0f};
   float acc[M], cmp[M];  // kComp: sum and compensation; else the even and odd chains
 #pragma unroll
   for (int m = 0; m < M; m++) {
@@ -830,9 +833,15 @@ __device__ __forceinline__ void mf_tiles(const h16x8* sa, const f32x4v* sw, int 
     const f32x4v w = sw[blk * 4 + grp];
     f32x4v d[M];
 #pragma unroll
-    for (int m = 0; m < M; m++) d[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, t[m].b[0], init, 0, 0, 0);
+    for (int m = 0; m < M; m++) d[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, t[m].b[0], zero, 0, 0, 0);
 #pragma unroll
     for (int m = 0; m < M; m++) d[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, t[m].b[1], d[m], 0, 0, 0);
+    if (KIND != kExp && seed != 0.0f) {
+#pragma unroll
+      for (int m = 0; m < M; m++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) d[m][i] = fabsf(d[m][i]) + seed;
+    }
 #pragma unroll
     for (int m = 0; m < M; m++)
 #pragma unroll

@@ -96,6 +96,26 @@ def test_mixed_near_field_of_coincident_points_is_zero(precision):
     assert not r.any() and not y.any()
 
 
+@pytest.mark.parametrize("precision", ["mixed", "mixed_comp"])
+@pytest.mark.parametrize("kind", ["bh3", "th3"])
+@pytest.mark.parametrize("units2", [1e-9, 1e-3, 0.03, 0.3, 7.3, 1.3e4, 1.6e7, 1.7e7, 3e12])
+def test_mixed_near_field_keeps_small_and_large_offsets(units2, kind, precision):
+    """The kernels' offset, from far below the 2^-9 half widths that the
+    coordinates are split at to far above the leaf, at close pairs."""
+    print("offset", units2, kind, precision, flush=True)
+    c = units2 ** 0.5 * H / 512
+    _, cls, _ = KINDS[kind]
+    for dist in (0.0, 2.0 ** -12, 2.0 ** -9, 0.3):
+        y, r = single_pairs(np.random.default_rng(3), cls, [1.0, c], precision, dist)
+        rho = np.sqrt(r * r + c * c)
+        ref, grow = (-rho, 1.0) if kind == "bh3" else (rho ** 3, 3.0)
+        # As for pairs without an offset; it is rounded to FP32 itself.
+        off = 2.0 ** -21 + 2 * 3 ** 0.5 * 2.0 ** -32 * H * r / rho ** 2
+        worst = np.max(np.abs(y - ref) / (np.abs(ref) * grow * off))
+        print(f"  at {dist:.1e}: worst error / bound {worst:.3f}", flush=True)
+        assert worst <= 1.0
+
+
 def test_mixed_near_field_does_not_depend_on_shared_launches():
     """One leaf of many targets next to leaves of few: every pass and split of
     the wave groups gives the bits of the same evaluation repeated."""
