@@ -448,7 +448,7 @@ struct P2PNeighbours {
 template <class T>
 __device__ __forceinline__ void p2p_store(const P2PJob<T>& j, int spart, int i, double sum) {
   if (j.sparts > 1) j.partial[static_cast<int64_t>(spart) * j.n_trg + i] = sum;
-  else j.out[j.tperm[i]] = (j.y_far ? j.y_far[i] : 0.0) + sum;
+  else j.out[j.tperm[i]] = (j.y_far ? j.y_far[i] : 0.0) + j.scale * sum;
 }
 
 // The source parts of every target, in order.
@@ -461,7 +461,7 @@ __global__ void p2p_fold_kernel(P2PJobs<T> jobs) {
          i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
       double sum = 0.0;
       for (int s = 0; s < j.sparts; s++) sum += j.partial[static_cast<int64_t>(s) * j.n_trg + i];
-      j.out[j.tperm[i]] = (j.y_far ? j.y_far[i] : 0.0) + sum;
+      j.out[j.tperm[i]] = (j.y_far ? j.y_far[i] : 0.0) + j.scale * sum;
     }
   }
 }
@@ -546,7 +546,7 @@ __device__ __forceinline__ void near_pass(const P2PJob<T>& j, const P2PNeighbour
     s.x += nb.off[k][0];
     s.y += nb.off[k][1];
     s.z += nb.off[k][2];
-    s.w *= j.pa;
+    s.w = static_cast<T>(q.w * j.pa);
     __syncthreads();
     sp[tid] = s;
     fetch(cb + step + tid);
@@ -891,7 +891,7 @@ __global__ void __launch_bounds__(kThreads, 4) p2p_mf_jobs_kernel(P2PJobs<float>
   const int nnb = nb.count, total = nb.start[nnb];
   // This source part's chunks: every sparts-th one.
   const int first = spart * kMfSrc, step = j.sparts * kMfSrc;
-  const float pa = j.pa, pb = j.pb;
+  const float pb = j.pb;
   const float seed = phi_seed<float, KIND>(pb);
   h16x8* const row = sa + (tid >> 4) * 128 + (tid & 15);  // this thread's source of a chunk
   mf_const_rows(row);
@@ -933,7 +933,7 @@ __global__ void __launch_bounds__(kThreads, 4) p2p_mf_jobs_kernel(P2PJobs<float>
       z.i += nb.off[k][2];
       __syncthreads();
       mf_rows(x, y, z, row);
-      reinterpret_cast<float*>(sw)[tid] = static_cast<float>(q.w) * pa;  // the kernel's factor a folded in
+      reinterpret_cast<float*>(sw)[tid] = static_cast<float>(q.w * j.pa);  // the kernel's factor folded in
       fetch(cb + step + tid);
       __syncthreads();
       switch (mine) {
@@ -2202,7 +2202,23 @@ P2PJob<T> make_p2p_job(const RbfDesc& rbf, const Tree& trg, const Tree& src, con
   // The mixed form's kernel works in units of kMfUnit of the leaf half width.
   const PhiConsts pc = phi_consts(rbf, sizeof(T) == 4 ? h * kMfUnit : h);
   j.y_far = y_far;
-  j.pa = static_cast<T>(pc.a);
+  j.pa = pc.a;
+  j.scale = 1.0;
+  if (sizeof(T) == 4 && rbf.kind == kTh3) {
+    // Cubes of distances in units span 2^31, and the factor a = m 2^(e - 27)
+    // the cube of whatever length unit the points are in. The FP32 weights get
+    // about the root of it, m 2^(e / 2 - 14), so that weights of any size that
+    // belongs to the lengths (about 1, or about 2^-e for values about 1) stay
+    // within FP32 at half widths of 1e-20 to 1e20; the rest goes to the FP64 sums.
+    // All of it in FP32 lost bits below half widths of 2e-10.
+    int e = 0;
+    (void)std::frexp(rbf.p0 * h * h * h, &e);
+    const int rest = e - 27 - (e / 2 - 14);
+    if (std::isnormal(pc.a)) {
+      j.pa = std::ldexp(pc.a, -rest);
+      j.scale = std::ldexp(1.0, rest);
+    }
+  }
   j.pb = static_cast<T>(phi_shape_const<T>(rbf.kind, pc.b));
   if constexpr (sizeof(T) == 4) p2p_split(j, src.n_points, src.n_leaves(), 16 * kMfPartTiles, kP2PMaxParts, kMfMaxSparts, 1, partial);
   else p2p_split(j, src.n_points, src.n_leaves(), 16 * kNearTiles<T, kNearValue>, kP2PMaxParts, kNearMaxSparts, 1, partial);
@@ -2220,7 +2236,7 @@ void launch_p2p_vector(const RbfDesc& rbf, const Tree& trg, const Tree& src, con
   Aniso3 A;
   for (int k = 0; k < 9; k++) A.a[k] = rbf.aniso[k];
   P2PJob<T> j = p2p_job_base<T>(trg, src, lists, tpts, spts, out3);
-  j.pa = static_cast<T>(MODE == kNearHessian ? gc.a / h : gc.a);
+  j.pa = MODE == kNearHessian ? gc.a / h : gc.a;
   j.pb = static_cast<T>(gc.b);
   p2p_split(j, src.n_points, src.n_leaves(), 16 * kNearTiles<T, MODE>, kP2PMaxParts, kNearMaxSparts, 3, partial);
   const int64_t blocks = static_cast<int64_t>(j.n_leaves) * j.parts * j.sparts;

@@ -66,7 +66,8 @@ struct P2PJob {
   const double* y_far;   // far field in tree order, or null
   const int32_t* tperm;  // tree order -> input order of the targets
   double* out;           // output, input order
-  T pa, pb;              // kernel constants in the leaf unit (phi_shape_const)
+  double pa, scale;      // the kernel's factor: in the weights, before they become T, and in the sums
+  T pb;                  // kernel constant in the leaf unit (phi_shape_const)
   double* partial;       // [sparts][n_trg][outputs] sums of the source parts, tree order (sparts > 1)
   int64_t n_trg;
   int n_leaves, parts, sparts, first_block;  // parts x sparts workgroups per leaf: target tiles x sources

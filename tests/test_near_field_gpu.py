@@ -116,6 +116,30 @@ def test_mixed_near_field_keeps_small_and_large_offsets(units2, kind, precision)
         assert worst <= 1.0
 
 
+@pytest.mark.parametrize("precision", ["mixed", "mixed_comp"])
+@pytest.mark.parametrize("unit_weights", [True, False])
+@pytest.mark.parametrize("width", [1e-12, 1e-10, 1e-9, 1.0, 1e9, 1e12])
+def test_mixed_triharmonic_near_field_in_any_length_unit(width, unit_weights, precision):
+    """Weights of about 1, and weights that give values of about 1."""
+    print("width", width, unit_weights, precision, flush=True)
+    rng = np.random.default_rng(17)
+    src, trg = rng.uniform(0.25, 0.75, (2, 500, 3))
+    w = rng.normal(size=500)
+    ev = pa.make_fmm_evaluator(pa.Triharmonic3D([1.0, 0.0]), (np.zeros(3), np.full(3, width)))
+    ev.set_config(pa.FmmConfig(precision, 4, 2, "fmm"))
+    ev.set_source_points(width * src)
+    ev.set_weights(w if unit_weights else w / width ** 3)
+    ev.set_target_points(width * trg)
+    y = ev.evaluate() / (width ** 3 if unit_weights else 1.0)
+    assert ev.stats()["direct"] == 0
+    term = w * np.linalg.norm(trg[:, None] - src[None], axis=2) ** 3
+    # Three times the error of r, products, and sums along chains of 500 / 8.
+    bound = np.abs(term).sum(1) * (3 * 2.0 ** -21 + 2.0 ** -24 * (2 + 500 / 8))
+    worst = np.max(np.abs(y - term.sum(1)) / bound)
+    print(f"  worst error / bound {worst:.3f}", flush=True)
+    assert worst <= 1.0
+
+
 def test_mixed_near_field_does_not_depend_on_shared_launches():
     """One leaf of many targets next to leaves of few: every pass and split of
     the wave groups gives the bits of the same evaluation repeated."""
