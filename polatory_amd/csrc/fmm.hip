@@ -511,7 +511,6 @@ __device__ __forceinline__ V4<T> point_as(const V4<double>& q) {
 // gradients in FP32, 200k x 200k, 1.12 to 0.69 ms. Eight source parts at most
 // instead of four: within 2 %.
 enum NearMode : int { kNearValue = 0, kNearGradient = 1, kNearHessian = 2 };
-constexpr int kNearMaxSparts = 4;
 template <class T, int MODE>
 constexpr int kNearTiles = MODE == kNearValue || sizeof(T) == 4 ? 8 : 5;
 
@@ -702,8 +701,8 @@ constexpr int kMfSrc = kThreads;  // sources staged per chunk: one per thread
 constexpr int kMfMaxTiles = 5;  // 16-target tiles per wave and pass
 constexpr double kMfUnit = 0x1p-9;
 // Target tiles per part at least (every part stages the leaf's sources for
-// itself), and source parts at most.
-constexpr int kMfPartTiles = 4, kMfMaxSparts = 3;
+// itself).
+constexpr int kMfPartTiles = 4;
 
 using h16x8 = _Float16 __attribute__((ext_vector_type(8)));
 using f32x4v = float __attribute__((ext_vector_type(4)));

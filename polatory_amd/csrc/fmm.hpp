@@ -56,6 +56,9 @@ void launch_l2l(int p, const Tree& t, int l, const T* l_parent, T* l_child, hipS
 // of each (serving). A lone evaluation runs the same kernels with one job.
 // T: arithmetic of the kernel values and sums; the points are FP64 either way.
 constexpr int kMaxFmmJobs = 8;
+// Most shares that a target's sources are dealt out in, mixed and FP64 form: a
+// near field keeps that many sums of 8 bytes per target at most.
+constexpr int kMfMaxSparts = 3, kNearMaxSparts = 4;
 template <class T>
 struct P2PJob {
   const int32_t* tls;    // target leaf starts

@@ -215,16 +215,20 @@ int64_t Server::model_bytes(int id) const {
 
 int64_t Server::estimate_bytes(const ModelEntry& m, int64_t n) const {
   // Working set of one request: the query points and outputs, and per rbf the
-  // transformed targets, their octree and sort buffers, the FP64/FP32
-  // tree-order copies, the far-field values, the local expansions and lists.
+  // transformed targets, their octree and sort buffers, the tree-order copy,
+  // the near field's sums of source parts, the local expansions and lists; for
+  // a direct sum its partial sums. (The M2L's per-pair transfers, whose number
+  // the lists decide, are not in it.)
   const int kp = kpad_of(m.cfg.order);
   const int64_t nr = static_cast<int64_t>(m.model.rbfs.size());
   int64_t cells = 0;
   for (int l = 2; l <= m.level; l++) cells += std::min<int64_t>(n, int64_t{1} << (3 * l));
   int64_t leaves = std::min<int64_t>(n, int64_t{1} << (3 * m.level));
-  int64_t per_pt = 24 + 8 + (nr > 1 ? 8 : 0) + nr * (24 + 40 + 32 + 16 + 8);
+  const int64_t sparts = m.cfg.precision == kFp64 ? kNearMaxSparts : kMfMaxSparts;
+  int64_t per_pt = 24 + 8 + (nr > 1 ? 8 : 0) + nr * (24 + 40 + 32 + 8 * sparts);
   int64_t per_cell = nr * (static_cast<int64_t>(kp) * 8 + kM2LSlots * 4 + 64);
-  return n * per_pt + cells * per_cell + leaves * nr * 27 * 4 + (int64_t{1} << 20);
+  const int64_t direct = direct_answer(m, n) ? nr * 8 * static_cast<int64_t>(direct_partial_size(n, m.n)) : 0;
+  return n * per_pt + cells * per_cell + leaves * nr * 27 * 4 + direct + (int64_t{1} << 20);
 }
 
 int64_t Server::submit(int model, const double* pts, int64_t n, double* out) {
@@ -255,11 +259,14 @@ int64_t Server::submit(int model, const double* pts, int64_t n, double* out) {
 bool Server::batchable(const Request& r) {
   // Requests that the evaluator would answer with the FP64 direct sum (below
   // 2^26 source-target pairs, or a model fixed to direct mode).
-  if (r.n <= 0) return false;
-  const ModelEntry& m = *r.model;
+  return direct_answer(*r.model, r.n);
+}
+
+bool Server::direct_answer(const ModelEntry& m, int64_t n) {
+  if (n <= 0) return false;
   if (m.cfg.mode == kModeDirect) return true;
   if (m.cfg.mode != kModeAuto) return false;
-  return static_cast<double>(r.n) * static_cast<double>(m.n) < 67108864.0;
+  return static_cast<double>(n) * static_cast<double>(m.n) < 67108864.0;
 }
 
 void Server::worker(int slot) {

@@ -90,6 +90,7 @@ class Server {
   void run_fmm_batch(Slot& slot, const std::vector<Request*>& batch);
   void run_batch(Slot& slot, const std::vector<Request*>& batch);
   static bool batchable(const Request& r);
+  static bool direct_answer(const ModelEntry& m, int64_t n);
 
   // Limits of one shared direct-sum launch.
   static constexpr size_t kMaxBatch = 64;

@@ -191,3 +191,25 @@ def test_fmm_requests_share_near_and_far_field_launches(orc, served):
         ref = reference(orc, models[m], q[sub])
         err = np.abs(mixed[i][sub] - ref).max() / np.abs(ref).max()
         assert err <= REL_TOL, f"request {i}: rel err {err:.2e}"
+
+
+@pytest.mark.parametrize("precision,per_point", [("mixed", 24 + 8 + 24 + 40 + 32 + 3 * 8),
+                                                 ("fp64", 24 + 8 + 24 + 40 + 32 + 4 * 8)])
+def test_admission_counts_what_a_query_point_takes(precision, per_point):
+    """Per query point: coordinates in and a value out, the transformed copy,
+    octree and sort buffers, the copy in tree order, and the near field's sums
+    of up to 3 (FP64: 4) source parts."""
+    rng = np.random.default_rng(7)
+    ip = pa.Interpolant(pa.Model(pa.Biharmonic3D(), poly_degree=1))
+    ip.set_fitted(rng.uniform(0, 1, (20_000, 3)), rng.normal(size=20_004))
+    srv = pa.Server(n_slots=1)
+    try:
+        mid = srv.add_model(ip, config=pa.FmmConfig(precision, 6, 3, "fmm"))
+        admitted = []
+        for n in (50_000, 150_000):  # more points than the 512 leaves: what the cells take is the same
+            srv.reset_stats()
+            srv.wait(srv.submit(mid, rng.uniform(0, 1, (n, 3))))
+            admitted.append(srv.stats()["peak_admitted_bytes"])
+        assert admitted[1] - admitted[0] == 100_000 * per_point
+    finally:
+        srv.close()
