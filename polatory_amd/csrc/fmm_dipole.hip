@@ -27,6 +27,21 @@ __global__ void minus_all_kernel(const double* __restrict__ g3, int64_t n3, int 
   out3[i] = k == 0 ? -g3[i] : out3[i] - g3[i];
 }
 
+// An accuracy is searched with the first components of the weights, before the
+// direct sum or the passes are chosen, so that the first evaluation goes the
+// way of all others.
+void choose_config(FmmEvaluator& ev, const double* w3, DevBuf<double>& wk) {
+  if (ev.config_chosen()) return;
+  const int64_t n = ev.n_src();
+  wk.resize(static_cast<size_t>(n));
+  if (n > 0) {
+    extract_component_kernel<<<ceil_div(n, 256), 256, 0, ev.stream()>>>(w3, n, 0, wk.get());
+    PAM_LAUNCH_CHECK();
+  }
+  ev.set_weights(wk.get(), n, true);
+  ev.ensure_config();
+}
+
 }  // namespace
 
 DipoleSourceEvaluator::DipoleSourceEvaluator(FmmEvaluator& ev) : ev_(ev) {
@@ -53,6 +68,7 @@ void DipoleSourceEvaluator::evaluate(double* out, int64_t n, bool on_device) {
     tmp_.resize(static_cast<size_t>(nt));
     d_out = tmp_.get();
   }
+  choose_config(ev_, w3_.get(), wk_);
   if (!ev_.evaluate_vector_direct(w3_.get(), false, d_out, nt)) {
     wk_.resize(static_cast<size_t>(n_src_));
     g3_.resize(static_cast<size_t>(nt) * 3);
@@ -99,6 +115,7 @@ void DipoleHessianEvaluator::evaluate(double* out, int64_t n, bool on_device) {
     tmp_.resize(static_cast<size_t>(nt) * 3);
     d_out = tmp_.get();
   }
+  choose_config(ev_, w3_.get(), wk_);
   if (!ev_.evaluate_vector_direct(w3_.get(), true, d_out, nt)) {
     wk_.resize(static_cast<size_t>(n_src_));
     g3_.resize(static_cast<size_t>(nt) * 3);

@@ -1017,7 +1017,8 @@ bool FmmEvaluator::evaluate_vector_direct(const double* d_w3, bool hessian, doub
   if (so_ || symmetric_) return false;
   const int64_t nt = n_trg();
   if (n != nt) throw_invalid("output size must equal the number of target points");
-  if (nt == 0 || n_src_ == 0 || !config_valid_) return false;
+  if (nt == 0 || n_src_ == 0) return false;
+  if (!config_valid_) throw_runtime("the configuration is not chosen");
   timing_valid_ = true;
   record(0);
   if (!use_direct()) return false;

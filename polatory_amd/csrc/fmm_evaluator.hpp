@@ -111,8 +111,9 @@ class FmmEvaluator {
   // Sums over sources with 3-vector weights (d_w3: x y z per source) in one
   // pass, when this evaluator would take the direct sum: values
   // (fmm/gradient_kernel.hpp) or, with hessian, 3-vectors
-  // (fmm/hessian_kernel.hpp) at the targets. Returns false, with nothing done,
-  // when it would not.
+  // (fmm/hessian_kernel.hpp) at the targets. Returns false, with no output
+  // written, when it would not (the trees may have been built to tell). The
+  // configuration must have been chosen (ensure_config).
   bool evaluate_vector_direct(const double* d_w3, bool hessian, double* d_out, int64_t n);
   // Makes this a gradient-transpose evaluator (make_fmm_evaluator.cpp:119-148):
   // evaluate() returns the gradients and the accuracy search measures them.
@@ -142,6 +143,10 @@ class FmmEvaluator {
   // alive while attached. Targets must lie in the owner's box. nullptr detaches.
   void attach_source(const FmmEvaluator* owner);
   const FmmConfig& active_config() const { return cfg_; }
+  bool config_chosen() const { return config_valid_; }
+  void ensure_config() {
+    if (!config_valid_) choose_config();
+  }
   int64_t n_src() const { return n_src_; }
   int64_t n_trg() const { return symmetric_ ? n_src_ : n_trg_; }
   const double* d_source_points() const { return src_pts_.get(); }

@@ -127,3 +127,29 @@ def test_overflowing_distances_keep_their_infinities():
     np.testing.assert_allclose(y, [np.exp(-3.0), 1.0, np.exp(-15.0)], rtol=1e-14)
     y = pa.direct_evaluate(pa.Biharmonic3D(), src[:1], np.array([np.nan]), trg[:1])
     assert np.isnan(y[0])
+
+
+@pytest.mark.parametrize("accuracy", [None, 1e-4])
+@pytest.mark.parametrize("make_evaluator,per", [(pa.make_fmm_gradient_evaluator, 1), (pa.make_fmm_hessian_evaluator, 3)])
+def test_first_sum_over_vector_weights_goes_the_way_of_the_next(make_evaluator, per, accuracy):
+    """Without a fixed configuration the first evaluation chooses one; its
+    values are the bits of the second's, and so are those after new points."""
+    rng = np.random.default_rng(31)
+    ev = make_evaluator(make("th3"))
+    if accuracy is not None:
+        ev.set_accuracy(accuracy)
+    for n_src, n_trg in ((700, 900), (2500, 40)):
+        src, trg = rng.uniform(0, 1, (n_src, 3)), rng.uniform(0, 1, (n_trg, 3))
+        w = rng.normal(size=(n_src, 3))
+        ev.set_source_points(src)
+        ev.set_target_points(trg)
+        ev.set_weights(w.ravel())
+        first = ev.evaluate()
+        assert ev.stats()["direct"] == 1
+        np.testing.assert_array_equal(first, ev.evaluate())
+        fixed = make_evaluator(make("th3"))
+        fixed.set_config(pa.FmmConfig("fp64", 10, -1, "direct"))
+        fixed.set_source_points(src)
+        fixed.set_target_points(trg)
+        fixed.set_weights(w.ravel())
+        np.testing.assert_array_equal(first, fixed.evaluate())
