@@ -140,9 +140,9 @@ def test_mixed_triharmonic_near_field_in_any_length_unit(width, unit_weights, pr
     assert worst <= 1.0
 
 
-def test_mixed_near_field_does_not_depend_on_shared_launches():
-    """One leaf of many targets next to leaves of few: every pass and split of
-    the wave groups gives the bits of the same evaluation repeated."""
+def test_mixed_near_field_is_the_same_on_either_stream():
+    """One leaf of many targets next to leaves of few, with the near field
+    beside the far field and after it."""
     rng = np.random.default_rng(3)
     src = rng.uniform(0.25, 0.75, (4000, 3))
     trg = np.concatenate([rng.uniform(0.26, 0.49, (2000, 3)), rng.uniform(0.51, 0.75, (37, 3))])

@@ -193,6 +193,37 @@ def test_fmm_requests_share_near_and_far_field_launches(orc, served):
         assert err <= REL_TOL, f"request {i}: rel err {err:.2e}"
 
 
+@pytest.mark.parametrize("precision", ["mixed", "fp64"])
+def test_near_fields_of_all_shapes_share_launches(orc, precision):
+    """Near fields of one launch that differ in everything that a workgroup
+    looks up: a model whose few leaves' sources are dealt out to several
+    workgroups and one whose are not, and requests of 3 to 40,000 points. Each
+    answer is the bits of the same request alone, and within 1.6e-5 (four times
+    the error of order 8) of the oracle's sum."""
+    rng = np.random.default_rng(95)
+    srv = pa.Server(n_slots=1)
+    try:
+        models, ids = [], []
+        for n, level in ((60_000, 2), (5000, 3)):
+            ip = pa.Interpolant(pa.Model(pa.Biharmonic3D(), poly_degree=1))
+            ip.set_fitted(rng.uniform(0, 1, (n, 3)), rng.normal(size=n + 4))
+            models.append((ip, pa.Biharmonic3D(), 1))
+            ids.append(srv.add_model(ip, config=pa.FmmConfig(precision, 8, level, "fmm")))
+        first = [(0, rng.uniform(0, 1, (300_000, 3)))]  # the others queue behind it
+        reqs = [(m, rng.uniform(0, 1, (n, 3))) for m, n in ((0, 300), (1, 20_000), (0, 3), (0, 40_000), (1, 3),
+                                                            (0, 2000), (1, 300), (1, 700))]
+        srv.reset_stats()
+        rids = [srv.submit(ids[m], q) for m, q in first + reqs]
+        mixed = [srv.wait(r) for r in rids][1:]
+        assert srv.stats()["max_fmm_batch"] >= 3
+        for (m, q), v in zip(reqs, mixed):
+            assert np.array_equal(srv.wait(srv.submit(ids[m], q)), v), f"{len(q)} points: other bits alone"
+            ref = reference(orc, models[m], q[:300])
+            assert np.abs(v[:300] - ref).max() <= 1.6e-5 * np.abs(ref).max()
+    finally:
+        srv.close()
+
+
 @pytest.mark.parametrize("precision,per_point", [("mixed", 24 + 8 + 24 + 40 + 32 + 3 * 8),
                                                  ("fp64", 24 + 8 + 24 + 40 + 32 + 4 * 8)])
 def test_admission_counts_what_a_query_point_takes(precision, per_point):

@@ -27,7 +27,8 @@ def test_points_are_stably_sorted_by_cell(n, level):
         step = np.diff(c)
         assert np.all(step >= 0)
         assert np.all(np.diff(perm)[step == 0] > 0)  # stable
-        cell = np.minimum(np.floor((p[perm] - info["lo"]) * info["inv_cell"]), 2 ** 20).astype(np.int64)
-        same = np.all(np.diff(cell, axis=0) == 0, axis=1)
-        if info["inv_cell"] * info["width"] == 2.0 ** level:
-            assert np.all(same[step == 0])
+        # The codes are those of the cells that the points lie in: bit k of x, y
+        # and z in bits 3 k + 2, 3 k + 1 and 3 k.
+        cell = np.clip(np.floor((p[perm] - info["lo"]) * info["inv_cell"]), 0, 2 ** level - 1).astype(np.int64)
+        want = sum(((cell[:, a] >> k) & 1) << (3 * k + 2 - a) for a in range(3) for k in range(level))
+        np.testing.assert_array_equal(c, want)
