@@ -381,8 +381,8 @@ __device__ __forceinline__ const P2PJob<T>& p2p_job_of(const P2PJobs<T>& jobs, i
 // kP2PBlocks leaves; where that leaves fewer than kP2PFill workgroups (four
 // rounds of the chip's 1,024), the source chunks are dealt out as well, at
 // least kP2PPartChunks to each part, and the parts' sums added by a second
-// launch. Mixed form, 220,731 sources in 512 leaves: 43,881 targets 0.349 to
-// 0.148 ms, 8,000 targets 0.170 to 0.083 ms.
+// launch (kP2PMaxSparts). Mixed form, 220,731 sources in 512 leaves: 43,881
+// targets 0.350 to 0.134 ms, 8,000 targets 0.185 to 0.082 ms.
 constexpr int kP2PBlocks = 4096, kP2PMaxParts = 8, kP2PFill = 4096, kP2PPartChunks = 4;
 
 // The leaf, target part and source part of a job's workgroup. Groups of 64
@@ -508,8 +508,7 @@ __device__ __forceinline__ V4<T> point_as(const V4<double>& q) {
 // workgroup and a test for zero in the root before (2.0 ms when the chip
 // starts cool); 50k surface points 2.45 to 0.38 ms (0.66 with one source part);
 // 30k sources against 60k targets in clusters, exponential, 3.97 to 0.48 ms;
-// gradients in FP32, 200k x 200k, 1.12 to 0.69 ms. Eight source parts at most
-// instead of four: within 2 %.
+// gradients in FP32, 200k x 200k, 1.12 to 0.69 ms.
 enum NearMode : int { kNearValue = 0, kNearGradient = 1, kNearHessian = 2 };
 template <class T, int MODE>
 constexpr int kNearTiles = MODE == kNearValue || sizeof(T) == 4 ? 8 : 5;
@@ -2160,7 +2159,7 @@ L2PJob<T> make_l2p_job(const Tree& t, const T* l_leaf, const V4<T>* pts, T* y_fa
 // Shares a job's leaves out: parts, sparts, and where the source parts' sums
 // of `outs` numbers per target go.
 template <class T>
-void p2p_split(P2PJob<T>& j, int64_t n_src, int64_t src_leaves, int part_targets, int most_parts, int most_sparts,
+void p2p_split(P2PJob<T>& j, int64_t n_src, int64_t src_leaves, int part_targets, int most_parts,
                int outs, DevBuf<double>& partial) {
   j.parts = j.sparts = 1;
   if (j.n_leaves == 0) return;
@@ -2169,7 +2168,7 @@ void p2p_split(P2PJob<T>& j, int64_t n_src, int64_t src_leaves, int part_targets
   const double blocks = j.n_leaves * std::clamp(static_cast<double>(j.n_trg) / j.n_leaves / part_targets, 1.0,
                                                 static_cast<double>(j.parts));
   const double chunks = 27.0 * static_cast<double>(n_src) / static_cast<double>(std::max<int64_t>(src_leaves, 1)) / kThreads;
-  j.sparts = std::clamp(static_cast<int>(std::min(kP2PFill / blocks, chunks / kP2PPartChunks)), 1, most_sparts);
+  j.sparts = std::clamp(static_cast<int>(std::min(kP2PFill / blocks, chunks / kP2PPartChunks)), 1, kP2PMaxSparts);
   if (j.sparts > 1) {
     partial.resize(static_cast<size_t>(j.sparts) * j.n_trg * outs);
     j.partial = partial.get();
@@ -2219,8 +2218,8 @@ P2PJob<T> make_p2p_job(const RbfDesc& rbf, const Tree& trg, const Tree& src, con
     }
   }
   j.pb = static_cast<T>(phi_shape_const<T>(rbf.kind, pc.b));
-  if constexpr (sizeof(T) == 4) p2p_split(j, src.n_points, src.n_leaves(), 16 * kMfPartTiles, kP2PMaxParts, kMfMaxSparts, 1, partial);
-  else p2p_split(j, src.n_points, src.n_leaves(), 16 * kNearTiles<T, kNearValue>, kP2PMaxParts, kNearMaxSparts, 1, partial);
+  if constexpr (sizeof(T) == 4) p2p_split(j, src.n_points, src.n_leaves(), 16 * kMfPartTiles, kP2PMaxParts, 1, partial);
+  else p2p_split(j, src.n_points, src.n_leaves(), 16 * kNearTiles<T, kNearValue>, kP2PMaxParts, 1, partial);
   return j;
 }
 
@@ -2237,7 +2236,7 @@ void launch_p2p_vector(const RbfDesc& rbf, const Tree& trg, const Tree& src, con
   P2PJob<T> j = p2p_job_base<T>(trg, src, lists, tpts, spts, out3);
   j.pa = MODE == kNearHessian ? gc.a / h : gc.a;
   j.pb = static_cast<T>(gc.b);
-  p2p_split(j, src.n_points, src.n_leaves(), 16 * kNearTiles<T, MODE>, kP2PMaxParts, kNearMaxSparts, 3, partial);
+  p2p_split(j, src.n_points, src.n_leaves(), 16 * kNearTiles<T, MODE>, kP2PMaxParts, 3, partial);
   const int64_t blocks = static_cast<int64_t>(j.n_leaves) * j.parts * j.sparts;
   if (blocks > INT32_MAX) throw_runtime("near field: too many leaves");
   dispatch_kind(rbf.kind, [&](auto K) {

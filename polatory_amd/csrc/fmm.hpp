@@ -56,9 +56,17 @@ void launch_l2l(int p, const Tree& t, int l, const T* l_parent, T* l_child, hipS
 // of each (serving). A lone evaluation runs the same kernels with one job.
 // T: arithmetic of the kernel values and sums; the points are FP64 either way.
 constexpr int kMaxFmmJobs = 8;
-// Most shares that a target's sources are dealt out in, mixed and FP64 form: a
-// near field keeps that many sums of 8 bytes per target at most.
-constexpr int kMfMaxSparts = 3, kNearMaxSparts = 4;
+// Most shares that a target's sources are dealt out in: a near field keeps that
+// many sums of 8 bytes per target and output at most. Where the rule in
+// p2p_split deals sources out at all, with 1, 2, 3, 4 and 8 shares (MI355X):
+//   mixed, 220,731 sources, 43,881 targets  0.350 0.201 0.155 0.134 0.173 ms
+//   mixed, 220,731 sources,  8,000 targets  0.185 0.112 0.091 0.082 0.101 ms
+//   FP64,  100,000 sources,  8,000 targets  0.118 0.079  -    0.064 0.079 ms
+//   FP64,  300,007 sources, 250,013 targets 2.30  2.05   -    2.04  2.05 ms
+// (more shares stage, and add, more than they fill). The sums of shorter
+// chains are the more accurate ones: rms error of cancelling weights in the
+// mixed form 2.6e-7, 1.8e-7, 1.4e-7, 1.2e-7, 0.9e-7.
+constexpr int kP2PMaxSparts = 4;
 template <class T>
 struct P2PJob {
   const int32_t* tls;    // target leaf starts

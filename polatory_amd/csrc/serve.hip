@@ -224,8 +224,7 @@ int64_t Server::estimate_bytes(const ModelEntry& m, int64_t n) const {
   int64_t cells = 0;
   for (int l = 2; l <= m.level; l++) cells += std::min<int64_t>(n, int64_t{1} << (3 * l));
   int64_t leaves = std::min<int64_t>(n, int64_t{1} << (3 * m.level));
-  const int64_t sparts = m.cfg.precision == kFp64 ? kNearMaxSparts : kMfMaxSparts;
-  int64_t per_pt = 24 + 8 + (nr > 1 ? 8 : 0) + nr * (24 + 40 + 32 + 8 * sparts);
+  int64_t per_pt = 24 + 8 + (nr > 1 ? 8 : 0) + nr * (24 + 40 + 32 + 8 * kP2PMaxSparts);
   int64_t per_cell = nr * (static_cast<int64_t>(kp) * 8 + kM2LSlots * 4 + 64);
   const int64_t direct = direct_answer(m, n) ? nr * 8 * static_cast<int64_t>(direct_partial_size(n, m.n)) : 0;
   return n * per_pt + cells * per_cell + leaves * nr * 27 * 4 + direct + (int64_t{1} << 20);
