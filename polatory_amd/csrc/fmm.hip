@@ -772,21 +772,24 @@ struct MfSum<true> {
 
 // A source's row of step k, and a target's column: their products add up to
 // the terms above. Lane group g of a wave (lane / 16) holds steps g and g + 4.
-// Subnormal FP16 values (below 2^-14) count in full.
+// Subnormal FP16 values (below 2^-14) count in full. Steps 2 and 6 have the
+// same row for every source, so only six rows of 16 sources are staged, 0, 1,
+// 3 and, kMfHalf further, 4, 5, 7 (with all eight in 32 KB of LDS, the far
+// field's transfers found less room beside the near field).
+constexpr int kMfHalf = 3 * 16, kMfBlock = 2 * kMfHalf;
 __device__ __forceinline__ void mf_rows(const MfCoord& x, const MfCoord& y, const MfCoord& z, h16x8* row) {
   const MfSelf q = mf_self(x, y, z);
   const float k = 0x1p-12f;
   row[0] = mf_pack(x.i, y.i, z.i, q.a, q.b, 4096.0f, 1.0f, 0.0f);
   row[1 * 16] = mf_pack(x.f1, y.f1, z.f1, x.i, y.i, z.i, q.c1, q.c2);
-  row[3 * 16] = mf_pack(x.f1, y.f1, z.f1, x.i, y.i, z.i, q.d1, q.d2);
-  row[4 * 16] = mf_pack(x.f2, y.f2, z.f2, 1.0f, 0x1p-10f, 0.0f, 0.0f, 0.0f);
-  row[5 * 16] = mf_pack(x.f1, y.f1, z.f1, x.f2, y.f2, z.f2, q.e1, q.e2);
-  row[7 * 16] = mf_pack(k * x.f2, k * y.f2, k * z.f2, k * q.g1, q.g2, k, k * k, 0.0f);
+  row[2 * 16] = mf_pack(x.f1, y.f1, z.f1, x.i, y.i, z.i, q.d1, q.d2);
+  row[kMfHalf] = mf_pack(x.f2, y.f2, z.f2, 1.0f, 0x1p-10f, 0.0f, 0.0f, 0.0f);
+  row[kMfHalf + 1 * 16] = mf_pack(x.f1, y.f1, z.f1, x.f2, y.f2, z.f2, q.e1, q.e2);
+  row[kMfHalf + 2 * 16] = mf_pack(k * x.f2, k * y.f2, k * z.f2, k * q.g1, q.g2, k, k * k, 0.0f);
 }
-// Steps 2 and 6 are the same for every source.
 __device__ __forceinline__ void mf_const_rows(h16x8* row) {
-  row[2 * 16] = mf_pack(1.0f, 1.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f);
-  row[6 * 16] = mf_pack(0x1p-11f, 0x1p-11f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f);
+  row[0] = mf_pack(1.0f, 1.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f);
+  row[kMfHalf] = mf_pack(0x1p-11f, 0x1p-11f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f);
 }
 struct MfColumn {
   h16x8 b[2];
@@ -826,8 +829,11 @@ __device__ __forceinline__ void mf_tiles(const h16x8* sa, const f32x4v* sw, int 
       cmp[m] = tot[m].odd;
     }
   }
-  for (int blk = s0; blk < nblk; blk += ds) {
-    const h16x8 a0 = sa[blk * 128 + lane], a1 = sa[blk * 128 + 64 + lane];
+  // Lane group 2's rows do not move with the sources.
+  const int stride = grp == 2 ? 0 : kMfBlock;
+  const h16x8* a = grp == 2 ? sa + kMfSrc / 16 * kMfBlock : sa + s0 * kMfBlock + (grp == 3 ? 2 : grp) * 16 + (lane & 15);
+  for (int blk = s0; blk < nblk; blk += ds, a += ds * stride) {
+    const h16x8 a0 = a[0], a1 = a[kMfHalf];
     const f32x4v w = sw[blk * 4 + grp];
     f32x4v d[M];
 #pragma unroll
@@ -870,7 +876,7 @@ __device__ __forceinline__ void mf_tiles(const h16x8* sa, const f32x4v* sw, int 
 
 template <int KIND, bool kComp>
 __global__ void __launch_bounds__(kThreads, 4) p2p_mf_jobs_kernel(P2PJobs<float> jobs) {
-  __shared__ h16x8 sa[kMfSrc / 16 * 128];  // [16-source block][step][row]
+  __shared__ h16x8 sa[kMfSrc / 16 * kMfBlock + kMfHalf + 1];  // [16-source block][step][row], rows of steps 2 and 6
   __shared__ f32x4v sw[kMfSrc / 4];        // [block][row]: weights
   __shared__ P2PNeighbours<float> nb;  // offsets in units
   __shared__ double red[4][kMfMaxTiles * 16];
@@ -891,8 +897,8 @@ __global__ void __launch_bounds__(kThreads, 4) p2p_mf_jobs_kernel(P2PJobs<float>
   const int first = spart * kMfSrc, step = j.sparts * kMfSrc;
   const float pb = j.pb;
   const float seed = phi_seed<float, KIND>(pb);
-  h16x8* const row = sa + (tid >> 4) * 128 + (tid & 15);  // this thread's source of a chunk
-  mf_const_rows(row);
+  h16x8* const row = sa + (tid >> 4) * kMfBlock + (tid & 15);  // this thread's source of a chunk
+  if (tid == 0) mf_const_rows(sa + kMfSrc / 16 * kMfBlock);
   const int npass = share_count(ntile, 4 * kMfMaxTiles);
   for (int ps = 0; ps < npass; ps++) {
     const int p0 = tile0 + share_begin(ntile, ps, npass), n = tile0 + share_begin(ntile, ps + 1, npass) - p0;
