@@ -166,8 +166,14 @@ double leaf_occupancy_target(int order, int precision) {
   // Per leaf of n points the near field costs ~27 n^2 pair evaluations (rate
   // R_pair) and the far field ~1.14 x 189 dense transfers of 2 P^6 flops
   // (rate R_m2l); the cost per point is least at n = P^3 sqrt(16 R_pair/R_m2l):
-  // 0.8 P^3 in the mixed form (1.9e12 pairs/s, 4.8e13 flop/s measured on
-  // MI355X), 0.66 P^3 in FP64 (6.6e11 pairs/s, 2.4e13 flop/s).
+  // 0.8 P^3 in the mixed form (1.9e12 pairs/s, 4.8e13 flop/s), 0.66 P^3 in FP64
+  // (6.6e11 pairs/s, 2.4e13 flop/s). These are the rates of the kernels that
+  // the targets were set with. The near fields give 5.4e12 and 1.5e12 pairs/s
+  // now and transfers at orders 7 and 8 are compressed, which moves the best
+  // level both ways; the targets are kept, as levels decide results. MI355X,
+  // order 8, levels 3 and 4: 100,000 uniform points 0.30 and 0.65 ms (mixed),
+  // 0.50 and 1.06 (FP64), level 3 chosen; a million 6.5 and 1.5, 23.9 and 4.8,
+  // level 4 chosen; but 300,000 0.90 and 0.74, 3.3 and 1.4, level 3 chosen.
   const double c = precision == kFp64 ? 0.66 : 0.8;
   return std::max(64.0, c * static_cast<double>(order) * order * order);
 }
@@ -303,7 +309,15 @@ bool FmmEvaluator::use_direct() {
   // dense transfer set (189 x 2 P^6 flops) per occupied target cell and level
   // whatever the number of targets in it, the FP64 direct sum n_src pair
   // evaluations per target. The trees are built to count the occupied cells
-  // (they are needed for the FMM anyway). Rates measured on MI355X.
+  // (they are needed for the FMM anyway). The rates, too, are those of the
+  // kernels that the rule was set with; now the direct sum gives 1.45e12
+  // pairs/s, the near fields 5.4e12 (mixed) and 1.5e12, and transfers at orders
+  // 7 and 8 are compressed. Kept, as the choice decides results. MI355X, direct
+  // sum against FMM: 30,000 x 7,000 0.18 and 0.14 ms (mixed, order 8, FMM
+  // chosen), 0.17 and 0.24 (FP64, direct chosen); 1M x 700 at order 6 0.55 and
+  // 0.38 (FMM chosen); but 1M x 2,000 at order 8 1.33 and 0.44 (mixed), 1.34
+  // and 0.63 (FP64), direct chosen. Vector weights take one direct pass against
+  // three by FMM: 15,000 x 100,000 1.02 and 1.48 ms, direct chosen.
   ensure_trees();
   const FmmEvaluator& src = S();
   const Tree& tt = target_tree();
