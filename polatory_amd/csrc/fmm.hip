@@ -681,7 +681,7 @@ __global__ void __launch_bounds__(kThreads, 3) p2p_vector_kernel(P2PJob<T> j, An
 // What only the source (target) decides is summed beforehand and enters as two
 // FP16 pieces against constants. For points so close that the sums of the
 // first steps nearly vanish, every step is exact, and r^2 is rounded where it
-// no longer shrinks: its error is relative to r^2 itself, 2^-23, and
+// no longer shrinks: its error is relative to r^2 itself, about 2^-23, and
 // coincident points give zero. The coordinates are those in FP64 to 2^-32 of
 // the half width. (With s2 in FP16 and the last three steps left out, r was
 // off by up to 2^-20 half widths: 3.5e-5 of it at 2^-8 half widths, 5e-3 at
@@ -692,10 +692,10 @@ __global__ void __launch_bounds__(kThreads, 3) p2p_vector_kernel(P2PJob<T> j, An
 // Near field of 1M x 1M uniform points at order 8 (5.9e9 pairs, MI355X, alone):
 // 1.65 ms on the VALU, 1.62 ms with FP64 matrix distances, 1.10 ms this way
 // (1.12 ms beside it with three v_mfma_f32_16x16x16_f16 that left the last
-// three steps out); 300k surface points (symmetric, uneven leaves): 1.68 to 0.65 ms, of which
-// about half is the finer split of the leaves. Four or six tiles per wave
-// instead of five: 1.09 and 1.00 ms. Two workgroups per leaf at 4,096 leaves:
-// 1.05 ms; at 512 leaves eight per leaf fill the chip.
+// three steps out), 1.25 ms with an offset; 300k surface points (symmetric,
+// uneven leaves): 1.68 to 0.57 ms, of which about half is the finer split of
+// the leaves. Four tiles per wave instead of five: 1.17 ms. Two workgroups per
+// leaf at 4,096 leaves: 1.15 ms; at 512 leaves eight per leaf fill the chip.
 constexpr int kMfSrc = kThreads;  // sources staged per chunk: one per thread
 constexpr int kMfMaxTiles = 5;  // 16-target tiles per wave and pass
 constexpr double kMfUnit = 0x1p-9;
